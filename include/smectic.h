@@ -236,8 +236,9 @@ int smx_batch_create(int nbox, const smx_config *cfgs, smx_batch **out);
 void smx_batch_destroy(smx_batch *b);
 /* Per-box handle for set/get/diagnostics; owned by the batch. */
 int smx_batch_handle(smx_batch *b, int box, smx_handle **h);
-/* Advance every box by nsteps: graph launches of `graph_steps` steps each
- * (captured once per batch) plus a direct remainder. */
+/* Advance every box by nsteps: launches of a graph of `graph_steps` steps, or of up to four times as
+ * many where that divides nsteps / graph_steps (captured once and kept while it fits the calls), plus a
+ * direct remainder. */
 int smx_batch_run(smx_batch *b, int64_t nsteps, int64_t graph_steps);
 /* Number of kernel nodes in the captured graph (0 before the first run). */
 int smx_batch_graph_nodes(smx_batch *b, int64_t *nodes);
@@ -272,7 +273,10 @@ int smx_batch_adjoint_nodes(smx_batch *b, int64_t *nodes);
  * nc = 16, variant = 0 in every slot.  The advected step uses the schedules of slots 0 and 2 for
  * its eleven y passes.  Neumann handles: the tile width only (variant 0): 32 (default) or 16
  * columns in FP32, 16 (default) or 8 in FP64; the advected Neumann step keeps the defaults.
- * The step's result depends on the schedule only through rounding.
+ * The step's result depends on the schedule only through rounding.  While the default schedule is
+ * in place a periodic handle without advection steps in two launches instead of four where its grid
+ * allows it (the y transform divided between the z and the x kernel: every grid with ny <= 384 whose
+ * tiles fit a workgroup's LDS); any other schedule selects the four kernels it names.
  */
 typedef struct smx_schedule {
   int nc[4];
@@ -291,7 +295,9 @@ int smx_set_schedule(smx_handle *h, const smx_schedule *s);
  * printed to stderr.  Results are cached per (device,
  * precision, grid) for the life of the process.  Replaces the FFTW_MEASURE planning of
  * pf3d.cpp:226-291 (which times candidate FFT algorithms at set-up).  An advected Neumann
- * handle keeps its fixed tiles (the call returns them); not callable during stream capture. */
+ * handle keeps its fixed tiles (the call returns them); not callable during stream capture.  On a
+ * grid that steps in two launches the tuned tiles serve the adjoint's four-pass chains and *chosen is
+ * the default schedule. */
 int smx_autotune(smx_handle *h, int reps, smx_schedule *chosen);
 /* smx_autotune on every box (boxes of one shape are tuned once; advected Neumann boxes keep
  * their fixed tiles); the next smx_batch_run captures its graph again with the new schedules. */
@@ -308,7 +314,7 @@ int smx_sync(smx_handle *h);
  * Replaces the reference's restart from a 6-digit text dump of psi, which re-bootstraps
  * N_hat_past from N(psi) without advection (pf3dMorph.cpp:416-472) and is therefore not
  * continuation-exact.  Binary file: header (magic "SMXCKPT1", ABI version, smx_config, step
- * count, array sizes), the arrays, the mean mode and an FNV-1a 64-bit checksum.  Loading
+ * count, array sizes; "SMXCKPT2" and a layout word for the state of the two-launch step), the arrays, the mean mode and an FNV-1a 64-bit checksum.  Loading
  * fails with SMX_ERR_INVALID for a file of another grid, precision or operator (the configs
  * must agree in every field but device) or with a bad checksum.
  */

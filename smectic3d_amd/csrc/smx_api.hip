@@ -15,6 +15,7 @@
 #include "../../include/smectic.h"
 #include "smx_diag.h"
 #include "smx_launch.h"
+#include "smx_split_ops.h"
 #include "smx_surf.h"
 
 using namespace smx;
@@ -104,7 +105,11 @@ struct smx_handle {
   bool l1_track = true;         // snapshot the stage buffer before the last step of each smx_step call
   int64_t finite_every = 100;   // steps between the non-finite checks of smx_step (0: off)
   int64_t steps = 0;
-  PassSched sched[NSLOTS];  // tile schedules of the step kernels (Neumann: tile widths, variant 0)
+  PassSched sched[NSLOTS];  // tile schedules of the four-pass kernels (Neumann: tile widths, variant 0)
+  bool auto_path = true;    // no schedule was installed: the two-launch step where the grid has it
+  bool split_ok = false;    // the grid has the two-launch step (smx_split.h)
+  bool split = false;       // A and R hold the split form
+  bool prev_split = false;  // Aprev does
   // device bytes the adjoint may spend on resident record sets: -1 (default) = a share of
   // the free memory for the duration of one call; >= 0 = this many, kept between calls
   int64_t adj_budget = -1;
@@ -363,6 +368,7 @@ static int bootstrap(smx_handle* h) {
 
 // Kernel slots of one step, in launch order.
 static const char* kSlotNamesP[] = {"k_ypass_inv", "k_zpass_nl", "k_ypass_fwd", "k_xpass_step"};
+static const char* kSlotNamesS[] = {"k_zsplit", "k_xsplit"};
 static const char* kSlotNamesN[] = {"k_dct_ypass_inv", "k_dct_zpass_nl", "k_dct_ypass_fwd", "k_dct_xpass_step"};
 static const char* kSlotNamesA[] = {"k_ypass_inv_dy", "k_ypass_inv_psi", "k_ypass_inv_dx", "k_ypass_inv_sh",
                                     "k_zpass_force", "k_ypass_fwd_s0", "k_ypass_fwd_s1", "k_ypass_fwd_s2",
@@ -373,10 +379,10 @@ static const char* kSlotNamesNA[] = {"k_dct_ypass_inv_dy", "k_dct_ypass_inv_psi"
                                      "k_dct_ypass_fwd_s1", "k_dct_ypass_fwd_s2", "k_dctx_stokes",
                                      "k_dct_ypass_inv_u0", "k_dct_ypass_inv_u1", "k_dct_ypass_inv_u2",
                                      "k_dctz_advnl", "k_dct_ypass_fwd_n", "k_dctx_adv"};
-static int num_slots(const smx_handle* h) { return h->cfg.advect ? 15 : 4; }
+static int num_slots(const smx_handle* h) { return h->cfg.advect ? 15 : (h->split ? 2 : 4); }
 static const char* slot_name(const smx_handle* h, int s) {
   if (h->cfg.advect) return h->neumann ? kSlotNamesNA[s] : kSlotNamesA[s];
-  return h->neumann ? kSlotNamesN[s] : kSlotNamesP[s];
+  return h->neumann ? kSlotNamesN[s] : (h->split ? kSlotNamesS[s] : kSlotNamesP[s]);
 }
 
 // Per-kernel timing of a step chain: slot k's kernel is launched with the event pair
@@ -523,9 +529,19 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
     CHK(xpass<T>(h, q, X_STEP, h->A, h->A, h->R, nullptr, h->sched[SLOT_X], true));
     return SMX_OK;
   }
+  PParams<T> q = p;
+  if (h->split) {  // the two-launch step; the x kernel sums the z kernel's FP64 partials
+    q.npartial = split_z_blocks<T>(p);
+    const SplitArgs<T> sa{(cplx<T>*)h->A, (cplx<T>*)h->R, tables<T>(h).twy, q};
+    tm.arm(0);
+    hipError_t e = split_z<T>(sa, Z_OP_NL, h->st);
+    tm.arm(1);
+    if (e == hipSuccess) e = split_x<T>(sa, h->st);
+    if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("two-launch step: ") + hipGetErrorString(e));
+    return SMX_OK;
+  }
   // periodic chain with the handle's tile schedules; the x pass sums the z pass's
   // FP64 partials, one per z tile
-  PParams<T> q = p;
   q.npartial = PeriodicOps<T>::zpass_blocks(p, h->sched[SLOT_Z].nc);
   tm.arm(0);
   CHK(ypass<T>(h, h->A, h->A, +1, h->sched[SLOT_YINV]));
@@ -538,40 +554,75 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
   return SMX_OK;  // the x pass projects the self-conjugate planes of R itself
 }
 
+// ---- the two forms of a periodic state (smx_split.h) ----
+// Rows of a stage array or carry from one form to the other on the handle's stream, in place
+// allowed.  wide: an FP64 copy of an FP32 array.
+template <typename T>
+static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, bool wide = false) {
+  const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, wide, h->st);
+  if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
+  return SMX_OK;
+}
+static bool use_split(const smx_handle* h) { return h->auto_path && h->split_ok; }
+// The state in the form that the handle's step path takes: nothing to do from step to step; once
+// after a state was set, loaded or left in the other form.
+template <typename T>
+static int ensure_form_T(smx_handle* h, bool split) {
+  cplx<T>*A = (cplx<T>*)h->A, *R = (cplx<T>*)h->R;
+  CHK(form_rows<T>(h, A, A, split ? FORM_FROM_STD : FORM_TO_STD));
+  CHK(form_rows<T>(h, R, R, split ? FORM_PERM_FROM_STD : FORM_PERM_TO_STD));
+  h->split = split;
+  return SMX_OK;
+}
+static int ensure_form(smx_handle* h, bool split) {
+  if (h->split == split) return SMX_OK;
+  return h->fp32 ? ensure_form_T<float>(h, split) : ensure_form_T<double>(h, split);
+}
+
 // ---- FP64 diagnostics on a copy of the state ----
 // FP64 copy of a stage buffer of the working precision into dst.
 // A periodic FP32 stage is also projected onto the stage of the real field it stands for
 // (k_herm_stage), so that FP64 derivatives of the copy are those of the field smx_get_psi returns.
-static int stage_to_f64(smx_handle* h, const void* stage, void* dst) {
+// split: the stage buffer holds the split form; the copy is in the standard one.
+static int stage_to_f64(smx_handle* h, const void* stage, void* dst, bool split) {
   const int64_t ncomp = h->neumann ? h->nspec : 2 * h->nspec;  // real components
   if (h->fp32) {
     hipLaunchKernelGGL(k_f32_to_f64, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, (const float*)stage,
                        (double*)dst, ncomp);
     HIPCHK(hipGetLastError());
+    if (split)
+      CHK(form_rows<double>(h, (const cplx<double>*)dst, (cplx<double>*)dst, FORM_TO_STD, true));
     if (!h->neumann) {
       const int64_t pairs = 2 * (int64_t)h->cfg.nx * (h->cfg.ny / 2 + 1);
       hipLaunchKernelGGL(k_herm_stage, dim3((unsigned)std::min<int64_t>((pairs + 255) / 256, 4096)), dim3(256), 0,
                          h->st, (cplx<double>*)dst, h->cfg.nx, h->cfg.ny, h->cfg.nz);
       HIPCHK(hipGetLastError());
     }
+  } else if (split) {
+    return form_rows<double>(h, (const cplx<double>*)stage, (cplx<double>*)dst, FORM_TO_STD);
   } else {
     HIPCHK(hipMemcpyAsync(dst, stage, sizeof(double) * ncomp, hipMemcpyDeviceToDevice, h->st));
   }
   return SMX_OK;
 }
-static int stage_to_d1(smx_handle* h, const void* stage) { return stage_to_f64(h, stage, h->D1); }
-static int state_to_d1(smx_handle* h) { return stage_to_d1(h, h->A); }
+static int state_to_d1(smx_handle* h) { return stage_to_f64(h, h->A, h->D1, h->split); }
 
 // Real psi of a stage buffer (the x-inverse of psi_hat) into `out` (dense [x][y][z], FP64).
-static int c2r_stage(smx_handle* h, const void* stage, double* out) {
+static int c2r_stage(smx_handle* h, const void* stage, bool split, double* out) {
   PParams<double> p = params<double>(h, false);
-  CHK(stage_to_d1(h, stage));
+  if (split) {  // one kernel: y and z inverse of the split form, FP32 widened as it is read
+    const hipError_t e = h->fp32 ? split_real<float>((const cplx<float>*)stage, out, p, h->st)
+                                 : split_real<double>((const cplx<double>*)stage, out, p, h->st);
+    if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("real field: ") + hipGetErrorString(e));
+    return SMX_OK;
+  }
+  CHK(stage_to_f64(h, stage, h->D1, false));
   CHK(ypass<double>(h, h->D1, h->D1, +1));
   CHK(zpass<double>(h, p, Z_IN_SPEC, Z_OUT_REAL, Z_OP_ID, h->D1, nullptr, nullptr, out));
   return SMX_OK;
 }
 // Real psi of the current state into `out`.
-static int c2r_state(smx_handle* h, double* out) { return c2r_stage(h, h->A, out); }
+static int c2r_state(smx_handle* h, double* out) { return c2r_stage(h, h->A, h->split, out); }
 
 // Inverse chain of a normalised full spectrum in D1 (destroyed) into a real field.
 static int c2r_spectrum_d1(smx_handle* h, double* out) {
@@ -754,10 +805,13 @@ static int run_steps(smx_handle* h, int64_t nsteps, double* partial = nullptr, b
   if (partial && p.partial) p.partial = partial;
   const size_t sbytes = h->wbytes * (size_t)h->nspec;
   snapshot = snapshot && h->l1_track;  // Aprev is allocated with the handle: nothing is allocated here
+  CHK(ensure_form(h, use_split(h)));
   for (int64_t n = 0; n < nsteps; ++n) {
     // stage buffer of psi^n for the L1 criterion of the last step (smx_l1 transforms it)
-    if (n == nsteps - 1 && snapshot)
+    if (n == nsteps - 1 && snapshot) {
       HIPCHK(hipMemcpyAsync(h->Aprev, h->A, sbytes, hipMemcpyDeviceToDevice, h->st));
+      h->prev_split = h->split;
+    }
     CHK(step_once<T>(h, p, nullptr));
     if (h->finite_every > 0 && (h->steps + n + 1) % h->finite_every == 0) CHK(enqueue_finite_check(h));
   }
@@ -1196,6 +1250,7 @@ struct smx_batch {
   std::vector<std::vector<int>> groups;
   std::vector<void*> grp_args;
   std::vector<std::array<PassSched, NSLOTS>> cap_sched;  // every box's schedules at capture
+  std::vector<bool> cap_split;                           // and its path
   // captured adjoint sweeps of every box, kept while every box keeps its workspace
   hipGraph_t adj_graph = nullptr;
   hipGraphExec_t adj_exec = nullptr;
@@ -1251,11 +1306,11 @@ static void batch_make_groups(smx_batch* b, std::vector<int>& single) {
     const smx_handle* h = b->boxes[i];
     std::vector<int> g{i};
     used[i] = true;
-    if (!h->neumann && !h->cfg.advect)
+    if (!h->neumann && !h->cfg.advect)  // (equal schedules and paths: equal forms)
       for (int j = i + 1; j < n; ++j) {
         const smx_handle* o = b->boxes[j];
         if (used[j] || o->neumann || o->cfg.advect || o->fp32 != h->fp32 || o->cfg.nx != h->cfg.nx ||
-            o->cfg.ny != h->cfg.ny || o->cfg.nz != h->cfg.nz || !same_sched(o, h))
+            o->cfg.ny != h->cfg.ny || o->cfg.nz != h->cfg.nz || o->split != h->split || !same_sched(o, h))
           continue;
         g.push_back(j);
         used[j] = true;
@@ -1268,6 +1323,19 @@ static void batch_make_groups(smx_batch* b, std::vector<int>& single) {
 // The GrpArgs array of a group in device memory (the parameters step_once gives each box).
 template <typename T>
 static int group_args(smx_batch* b, const std::vector<int>& members, void** out) {
+  if (b->boxes[members[0]]->split) {
+    std::vector<SplitArgs<T>> host;
+    for (int i : members) {
+      smx_handle* h = b->boxes[i];
+      PParams<T> p = params<T>(h, h->fp32);
+      p.npartial = split_z_blocks<T>(p);
+      host.push_back(SplitArgs<T>{(cplx<T>*)h->A, (cplx<T>*)h->R, tables<T>(h).twy, p});
+    }
+    const size_t bytes = sizeof(SplitArgs<T>) * host.size();
+    HIPCHK(hipMalloc(out, bytes));
+    HIPCHK(hipMemcpy(*out, host.data(), bytes, hipMemcpyHostToDevice));
+    return SMX_OK;
+  }
   std::vector<GrpArgs<T>> host(members.size());
   for (size_t i = 0; i < members.size(); ++i) {
     smx_handle* h = b->boxes[members[i]];
@@ -1289,9 +1357,15 @@ static int group_steps(smx_batch* b, const std::vector<int>& members, const void
                        hipStream_t st) {
   smx_handle* h = b->boxes[members[0]];
   const PParams<T> p = params<T>(h, h->fp32);
+  const int nb = (int)members.size();
   for (int64_t i = 0; i < n; ++i) {
-    hipError_t e = PeriodicOps<T>::step_grp((const GrpArgs<T>*)args, (int)members.size(), p, h->npencils,
-                                            h->sched, st);
+    hipError_t e;
+    if (h->split) {
+      e = split_z_grp<T>((const SplitArgs<T>*)args, nb, p, Z_OP_NL, st);
+      if (e == hipSuccess) e = split_x_grp<T>((const SplitArgs<T>*)args, nb, p, st);
+    } else {
+      e = PeriodicOps<T>::step_grp((const GrpArgs<T>*)args, nb, p, h->npencils, h->sched, st);
+    }
     if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("grouped step: ") + hipGetErrorString(e));
   }
   return SMX_OK;
@@ -1308,10 +1382,12 @@ static int batch_capture(smx_batch* b, int64_t gsteps) {
   }
   batch_free_groups(b);
   b->cap_sched.clear();
+  b->cap_split.clear();
   for (const smx_handle* h : b->boxes) {
     std::array<PassSched, NSLOTS> s;
     for (int k = 0; k < NSLOTS; ++k) s[k] = h->sched[k];
     b->cap_sched.push_back(s);
+    b->cap_split.push_back(h->split);
   }
   std::vector<int> single;
   batch_make_groups(b, single);
@@ -1441,8 +1517,13 @@ static int autotune_T(smx_handle* h, int reps_in, PassSched* best) {
   T* wr = (T*)h->D2;
   auto reset = [&]() -> int {
     if (h->has_state) {
-      HIPCHK(hipMemcpyAsync(wa, h->A, sizeof(T) * ncomp, hipMemcpyDeviceToDevice, h->st));
-      HIPCHK(hipMemcpyAsync(wr, h->R, sizeof(T) * ncomp, hipMemcpyDeviceToDevice, h->st));
+      if (h->split) {
+        CHK(form_rows<T>(h, (const cplx<T>*)h->A, (cplx<T>*)wa, FORM_TO_STD));
+        CHK(form_rows<T>(h, (const cplx<T>*)h->R, (cplx<T>*)wr, FORM_PERM_TO_STD));
+      } else {
+        HIPCHK(hipMemcpyAsync(wa, h->A, sizeof(T) * ncomp, hipMemcpyDeviceToDevice, h->st));
+        HIPCHK(hipMemcpyAsync(wr, h->R, sizeof(T) * ncomp, hipMemcpyDeviceToDevice, h->st));
+      }
       HIPCHK(hipMemcpyAsync(h->mean_state + 4, h->mean_state, 2 * sizeof(double), hipMemcpyDeviceToDevice, h->st));
     } else {
       // stage entries of size a give psi ~ a sqrt(ny nz); the carry is x-normalised
@@ -1552,6 +1633,7 @@ static int field_to_host(smx_handle* h, const double* dev, double* out, int64_t 
 // Bootstrap the state from the real field in real_io (the tail of smx_set_psi).
 static int state_from_real_io(smx_handle* h) {
   HIPCHK(hipMemsetAsync(h->mean_state, 0, sizeof(double) * 8, h->st));
+  h->split = false;
   CHK(h->fp32 ? bootstrap<float>(h) : bootstrap<double>(h));
   CHK(reset_checks(h));
   h->has_state = true;
@@ -1562,9 +1644,10 @@ static int state_from_real_io(smx_handle* h) {
 // ---- exact checkpoints ----
 // File: CkptHeader, then the carried arrays (A, R; with advection also Ax, As), each
 // wbytes * nspec bytes, the FP64 mean state (2 doubles), and an FNV-1a 64-bit checksum of
-// everything before it.
+// everything before it.  A state in the split form is written as it is, so that the resumed run
+// continues bit for bit: magic "SMXCKPT2", with a word for the form's layout behind the header.
 struct CkptHeader {
-  char magic[8];  // "SMXCKPT1"
+  char magic[8];  // "SMXCKPT1" or "SMXCKPT2"
   int32_t abi_version;
   int32_t narrays;
   int64_t wbytes, nspec, steps;
@@ -1586,6 +1669,11 @@ static bool same_operator(const smx_config& a, const smx_config& b) {
          a.q0 == b.q0 && a.alpha == b.alpha && a.beta == b.beta && a.gamma == b.gamma && a.dt == b.dt &&
          a.nl_model == b.nl_model && a.advect == b.advect && a.eta == b.eta && a.rho == b.rho &&
          a.force_form == b.force_form && a.w_mid == b.w_mid && a.mid_plane == b.mid_plane;
+}
+
+static int64_t split_layout(const smx_handle* h) {
+  const int ra = split_ra(h->cfg.ny), rb = ra ? h->cfg.ny / ra : 0;
+  return ra ? ra * 65536 + (h->fp32 ? split_yc<float>(rb) : split_yc<double>(rb)) : 0;
 }
 
 static std::vector<void*> carried_arrays(smx_handle* h) {
@@ -1660,6 +1748,10 @@ int smx_create(const smx_config* cfg, smx_handle** out) {
   h->dx = c.lx / c.nx;
   h->dy = c.ly / c.ny;
   h->dz = c.lz / c.nz;
+  if (!h->neumann && !c.advect)
+    h->split_ok = h->fp32 ? split_z_fits<float>(c.ny, c.nz) && split_x_fits<float>(c.nx, c.ny)
+                          : split_z_fits<double>(c.ny, c.nz) && split_x_fits<double>(c.nx, c.ny);
+  if (h->split_ok) h->split_ok = split_real_fits(c.ny, c.nz);
   if (h->neumann) {  // the default widths; the x pass's tile must divide ny (else 16 columns)
     const int ncd = h->fp32 ? neumann_nc<float>() : neumann_nc<double>();
     for (PassSched& ps : h->sched) ps = PassSched{ncd, 0};
@@ -1803,7 +1895,7 @@ int smx_save_checkpoint(smx_handle* h, const char* path) {
   const size_t abytes = h->wbytes * (size_t)h->nspec;
   CkptHeader hd;
   std::memset(&hd, 0, sizeof(hd));
-  std::memcpy(hd.magic, "SMXCKPT1", 8);
+  std::memcpy(hd.magic, h->split ? "SMXCKPT2" : "SMXCKPT1", 8);
   hd.abi_version = SMX_ABI_VERSION;
   hd.narrays = (int32_t)arrs.size();
   hd.wbytes = (int64_t)h->wbytes;
@@ -1819,6 +1911,11 @@ int smx_save_checkpoint(smx_handle* h, const char* path) {
   uint64_t hsh = 1469598103934665603ull;
   bool ok = std::fwrite(&hd, sizeof(hd), 1, f) == 1;
   hsh = fnv1a(hsh, &hd, sizeof(hd));
+  if (h->split) {
+    const int64_t lay = split_layout(h);
+    ok = ok && std::fwrite(&lay, sizeof(lay), 1, f) == 1;
+    hsh = fnv1a(hsh, &lay, sizeof(lay));
+  }
   for (size_t i = 0; i < arrs.size() && ok; ++i) {
     if (hipMemcpy(buf.data(), arrs[i], abytes, hipMemcpyDeviceToHost) != hipSuccess) {
       std::fclose(f);
@@ -1847,12 +1944,20 @@ int smx_load_checkpoint(smx_handle* h, const char* path) {
     std::fclose(f);
     return fail(SMX_ERR_INVALID, std::string(path) + ": " + why);
   };
-  if (std::fread(&hd, sizeof(hd), 1, f) != 1 || std::memcmp(hd.magic, "SMXCKPT1", 8) != 0)
+  if (std::fread(&hd, sizeof(hd), 1, f) != 1 ||
+      (std::memcmp(hd.magic, "SMXCKPT1", 8) != 0 && std::memcmp(hd.magic, "SMXCKPT2", 8) != 0))
     return bad("not a checkpoint");
+  const bool in_split = hd.magic[7] == '2';
   if (hd.abi_version != SMX_ABI_VERSION || hd.narrays != (int32_t)arrs.size() || hd.wbytes != (int64_t)h->wbytes ||
       hd.nspec != h->nspec || !same_operator(hd.cfg, h->cfg))
     return bad("checkpoint of a different grid, precision or operator");
   uint64_t hsh = fnv1a(1469598103934665603ull, &hd, sizeof(hd));
+  if (in_split) {
+    int64_t lay = 0;
+    if (std::fread(&lay, sizeof(lay), 1, f) != 1) return bad("truncated");
+    if (!h->split_ok || lay != split_layout(h)) return bad("checkpoint of another state layout");
+    hsh = fnv1a(hsh, &lay, sizeof(lay));
+  }
   std::vector<std::vector<char>> data(arrs.size(), std::vector<char>(abytes));
   for (auto& d : data) {
     if (std::fread(d.data(), 1, abytes, f) != abytes) return bad("truncated");
@@ -1871,6 +1976,7 @@ int smx_load_checkpoint(smx_handle* h, const char* path) {
     HIPCHK(hipMemcpyAsync(arrs[i], data[i].data(), abytes, hipMemcpyHostToDevice, h->st));
   HIPCHK(hipMemcpyAsync(h->mean_state, mean, sizeof(mean), hipMemcpyHostToDevice, h->st));
   HIPCHK(hipStreamSynchronize(h->st));  // the host buffers are freed on return
+  h->split = in_split;
   CHK(reset_checks(h));
   h->steps = hd.steps;
   h->has_state = true;
@@ -1889,7 +1995,7 @@ int smx_l1(smx_handle* h, double* l1) {
     return fail(SMX_ERR_STATE, "no L1 snapshot: no smx_step since the state was set, or L1 tracking is off");
   HIPCHK(hipSetDevice(h->cfg.device));
   CHK(check_finite(h));
-  CHK(c2r_stage(h, h->Aprev, h->real_prev));
+  CHK(c2r_stage(h, h->Aprev, h->prev_split, h->real_prev));
   CHK(c2r_state(h, h->real_io));
   hipLaunchKernelGGL(k_reduce_l1, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, h->real_io, h->real_prev, h->N,
                      h->red);
@@ -2002,11 +2108,13 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   const int ns = surf_nsplit(h->neumann, h->cfg.nx, h->cfg.nz);
   // An FP64 state is its own x stage, and an FP32 Neumann stage is read as it is (widened on
   // load); a periodic FP32 stage is copied to FP64 and projected (stage_to_f64) first.
-  const bool f32in = h->fp32 && h->neumann, w0copy = h->fp32 && !h->neumann;
+  // An FP64 split-form state is brought to the standard form there.
+  const bool f32in = h->fp32 && h->neumann, w0copy = !h->neumann && (h->fp32 || h->split);
+  const bool w0room = !h->neumann && (h->fp32 || h->split_ok);
   // real psi, the FP64 x stage copy, the field values at each column's evaluation index (ns
   // parts per field), the z evaluation's trigonometric table, and the crossing and evaluation
   // indices of each column
-  const size_t nw0 = w0copy ? sdoubles : 0, nval = 7 * (size_t)ns * nxy, ntrig = 4 * (size_t)h->cfg.nz;
+  const size_t nw0 = w0room ? sdoubles : 0, nval = 7 * (size_t)ns * nxy, ntrig = 4 * (size_t)h->cfg.nz;
   double* f = h->sfield;  // psi, dense [x][y][z]
   if (!f) {
     CHK(dalloc(h, (void**)&h->sfield,
@@ -2028,7 +2136,7 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   // (X_MUL2, below)
   const void* x_stage = h->A;
   if (w0copy) {
-    CHK(stage_to_f64(h, h->A, W0));
+    CHK(stage_to_f64(h, h->A, W0, h->split));
     x_stage = W0;
   }
   // without advection the x multipliers come from the x stage in pairs (X_MUL2) and psi_hat
@@ -2242,8 +2350,9 @@ int smx_adjoint_info(const smx_handle* h, int64_t* resident_steps, int64_t* reco
 int smx_get_schedule(const smx_handle* h, smx_schedule* s) {
   if (!h || !s) return fail(SMX_ERR_INVALID, "null argument");
   for (int k = 0; k < NSLOTS; ++k) {
-    s->nc[k] = h->sched[k].nc;
-    s->variant[k] = h->sched[k].v;
+    const PassSched ps = use_split(h) ? PassSched{} : h->sched[k];
+    s->nc[k] = ps.nc;
+    s->variant[k] = ps.v;
   }
   return SMX_OK;
 }
@@ -2259,7 +2368,11 @@ int smx_set_schedule(smx_handle* h, const smx_schedule* s) {
   }
   HIPCHK(hipSetDevice(h->cfg.device));
   CHK(h->fp32 ? sched_check<float>(h, c) : sched_check<double>(h, c));
-  for (int k = 0; k < NSLOTS; ++k) h->sched[k] = c[k];
+  h->auto_path = true;  // the default schedule leaves the choice of the path to the library
+  for (int k = 0; k < NSLOTS; ++k) {
+    h->sched[k] = c[k];
+    if (c[k].nc != kNC || c[k].v != 0) h->auto_path = false;
+  }
   return SMX_OK;
 }
 
@@ -2288,6 +2401,7 @@ int smx_autotune(smx_handle* h, int reps, smx_schedule* chosen) {
     g_tune_cache[key] = best;
   }
   for (int k = 0; k < NSLOTS; ++k) h->sched[k] = best[k];
+  h->auto_path = true;
   if (chosen) CHK(smx_get_schedule(h, chosen));
   return SMX_OK;
 }
@@ -2344,14 +2458,29 @@ int smx_batch_run(smx_batch* b, int64_t nsteps, int64_t graph_steps) {
     HIPCHK(hipStreamSynchronize(h->st));
   }
   HIPCHK(hipSetDevice(b->boxes[0]->cfg.device));
+  for (smx_handle* h : b->boxes) {
+    CHK(ensure_form(h, use_split(h)));
+    HIPCHK(hipStreamSynchronize(h->st));
+  }
+  // One graph carries up to four stretches of graph_steps where their number divides evenly (the
+  // kernels of a small box last a few microseconds, as long as the gap between two graphs); a
+  // captured graph that fits is kept.
   const int64_t ng = nsteps / graph_steps, rem = nsteps - ng * graph_steps;
-  bool stale = !b->exec || b->graph_steps != graph_steps || b->cap_sched.size() != b->boxes.size();
-  for (size_t i = 0; !stale && i < b->boxes.size(); ++i)  // a box's schedule set since the capture
+  int64_t m = b->graph_steps / graph_steps;
+  bool stale = !b->exec || m < 1 || b->graph_steps != m * graph_steps || ng % m != 0 ||
+               b->cap_sched.size() != b->boxes.size();
+  for (size_t i = 0; !stale && i < b->boxes.size(); ++i) {  // a box's schedule or path set since the capture
+    if (b->cap_split[i] != b->boxes[i]->split) stale = true;
     for (int k = 0; k < NSLOTS; ++k)
       if (b->cap_sched[i][k].nc != b->boxes[i]->sched[k].nc || b->cap_sched[i][k].v != b->boxes[i]->sched[k].v)
         stale = true;
-  if (ng > 0 && stale) CHK(batch_capture(b, graph_steps));
-  for (int64_t g = 0; g < ng; ++g) HIPCHK(hipGraphLaunch(b->exec, b->st));
+  }
+  if (ng > 0 && stale) {
+    for (m = 4; ng % m != 0;) --m;
+    CHK(batch_capture(b, m * graph_steps));
+  }
+  if (ng > 0)
+    for (int64_t g = 0; g < ng / m; ++g) HIPCHK(hipGraphLaunch(b->exec, b->st));
   HIPCHK(hipStreamSynchronize(b->st));
   for (smx_handle* h : b->boxes) {
     if (rem > 0) CHK(box_steps(h, rem));
@@ -2558,9 +2687,10 @@ int smx_profile_step(smx_handle* h, int64_t nsteps, int max_slots, int* nslots, 
                      char* names, int names_cap) {
   if (!h || !nslots || !avg_ms || !alg_bytes) return fail(SMX_ERR_INVALID, "null argument");
   if (!h->has_state) return fail(SMX_ERR_STATE, "no state: call smx_set_psi first");
+  HIPCHK(hipSetDevice(h->cfg.device));
+  CHK(ensure_form(h, use_split(h)));
   const int ns = num_slots(h);
   if (max_slots < ns) return fail(SMX_ERR_INVALID, "max_slots too small");
-  HIPCHK(hipSetDevice(h->cfg.device));
   std::vector<double> acc;
   CHK(h->fp32 ? profile_T<float>(h, nsteps, acc) : profile_T<double>(h, nsteps, acc));
   const double sc = (double)h->wbytes * (double)h->nspec;  // bytes of one spectral-stage array
@@ -2568,6 +2698,8 @@ int smx_profile_step(smx_handle* h, int64_t nsteps, int max_slots, int* nslots, 
   if (h->cfg.advect)  // reads + writes of spectral-stage arrays per launch
     bytes = {2 * sc, 2 * sc, 2 * sc, 2 * sc, 7 * sc, 2 * sc, 2 * sc, 2 * sc,
              6 * sc, 2 * sc, 2 * sc, 2 * sc, 7 * sc, 2 * sc, 6 * sc};
+  else if (h->split)
+    bytes = {2 * sc, 4 * sc};
   else
     bytes = {2 * sc, 2 * sc, 2 * sc, 4 * sc};
   *nslots = ns;

@@ -1,0 +1,539 @@
+// smx_split.h -- the periodic step in two launches: the y transform divided between the z and
+// the x kernel.
+//
+// A length-ny transform with ny = RA * RB, y = y1 RB + y2, ky = k1 + RA k2, is
+//   X[k1 + RA k2] = sum_y2 w_RB^{y2 k2} w_ny^{y2 k1} ( sum_y1 w_RA^{y1 k1} x[y1 RB + y2] )
+// (Cooley and Tukey 1965): radix RA over y1 at fixed y2, then radix RB over y2 at fixed k1.  The z
+// kernel holds all y1 of a few y2 (and all z), the x kernel all y2 of a few k1 (and all x), so each
+// does its part of the y transform on a tile it has in LDS anyway, and the two y passes, with 4 of
+// the step's 10 moves of a stage array through HBM, are gone:
+//   k_zsplit  (x, k1 y2, kz) -> (x, k1 y2, kz)   radix RA over k1, z C2R, N(psi), z R2C, radix RA over y1
+//   k_xsplit  (x, k1 y2, kz) -> (x, k1 y2, kz)   forward x with radix RB over y2, CNAB2 update, inverse
+// Between the two a stage row (kz, x) holds the y2-space, k1-space values in the order of split_pos,
+// and the carry R(kx, ky = k1 + RA k2, kz) is at [kz][kx][k1 RB + k2] (the split form; the four-pass
+// kernels of smx_periodic.h and the diagnostics use the standard one, ky at its index).
+//
+// Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 67 + 98 us and
+// 41 + 47 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
+// from two launches in place of four as well: 64^3 FP32 3.71 -> 2.97 ms for 200 steps and their checks.
+#pragma once
+#include "smx_periodic.h"
+
+namespace smx {
+
+// RA of a length (RB = ny / RA); 0: no split.  Both tiles hold NZ RA (2 or 4) / 2 and NX RB values, so
+// the two factors are near each other and RB <= 16 (an x tile of 256 x 16 FP64 values is 64 KB).
+constexpr int split_ra(int ny) {
+  return ny == 16 || ny == 32 || ny == 48 ? 4
+         : ny == 64 || ny == 96 || ny == 128 ? 8
+         : ny == 192 ? 12
+         : ny == 256 ? 16
+         : ny == 384 ? 24
+                     : 0;
+}
+
+// Position of (k1, y2) in a split-form stage row: pieces of YC adjacent y2 of two adjacent k1.  The z
+// kernel's tile has every k1 and few y2, the x kernel's few k1 and every y2, so with either index
+// alone fastest one of the two would touch a quarter of each 128-byte line; in this order both use
+// at least half of the lines that they touch.
+template <typename T>
+__host__ __device__ constexpr int split_yc(int rb) {
+  return sizeof(T) == 4 && rb % 8 == 0 ? 8 : 4;
+}
+__host__ __device__ __forceinline__ int split_pos(int k1, int y2, int rb, int yc) {
+  return (k1 >> 1) * 2 * rb + (y2 / yc) * 2 * yc + (k1 & 1) * yc + y2 % yc;
+}
+
+// y2 values per z tile (they are contiguous in the stage rows, and adjacent ones share a complex
+// transform).
+template <typename T, int L, int RA>
+constexpr int split_ny2() {
+  return RA <= 8 ? 4 : (sizeof(T) == 4 && L >= 256 && RA <= 16 ? 4 : 2);
+}
+// Plan variants: E = 8 where the length has it; E = 16 for the FP32 z kernel at 256 and 512.
+template <int L>
+constexpr int split_v() {
+  return HasPlanV<L, 1>::value && L >= 64 ? 1 : 0;
+}
+template <typename T, int L>
+constexpr int split_zv() {
+  return sizeof(T) == 4 && L >= 256 ? 0 : split_v<L>();
+}
+// Columns per x tile: whole k1 groups of RB.
+constexpr int split_nc(int rb) { return rb <= 8 ? 16 : rb; }
+
+template <typename T>
+struct SplitArgs {
+  cplx<T>* a;               // stage array, split form, in place
+  cplx<T>* r;               // carry, split form
+  const cplx<T>* twy;       // e^{-2 pi i m/ny}
+  PParams<T> p;
+};
+
+// ---------------------------------------------------------------------------
+// z kernel.  Tile: one x, NY2 adjacent y2, every k1 (y1) and kz.
+template <typename T_, int L_, int RA_, int NY2_ = split_ny2<T_, L_, RA_>(), int V_ = split_zv<T_, L_>()>
+struct ZS {
+  using T = T_;
+  static constexpr int L = L_, RA = RA_, NY2 = NY2_, V = V_;
+  static constexpr int E = PlanV<L, V>::E, TPC = L / E;
+  static constexpr int NPR = RA * NY2 / 2, NT = NPR * TPC, NZH = L / 2 + 1;
+  // Half-spectrum tile [kz][y1][y2]: rows padded by 32 bytes, so that the NY2-wide pieces which
+  // lanes write down consecutive kz fall in different banks.
+  static constexpr int HP = RA * NY2 + 32 / (int)sizeof(cplx<T>);
+  static constexpr int FP = NPR, SP = NPR + 1;  // transform tile pitch; pitch of the split's copy
+  static constexpr int LDS = (NZH * HP > L * SP ? NZH * HP : L * SP);
+  static constexpr int RED = (NT % 64 == 0) ? NT / 64 : NT;
+  static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
+};
+
+// Sum of x + y of the E values of every thread, FP64, into red[] (one entry per wave, or per thread
+// where the last wave is not full); zs_partial_store adds them after a later barrier.
+template <typename T, int E, int NT>
+__device__ __forceinline__ void zs_partial(const cplx<T>* v, double* red, int tid) {
+  double t[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) t[e] = (double)v[e].x + (double)v[e].y;
+#pragma unroll
+  for (int w = 1; w < E; w *= 2)
+#pragma unroll
+    for (int e = 0; e + w < E; e += 2 * w) t[e] += t[e + w];
+  if constexpr (NT % 64 == 0) {
+    const double ws = wave_sum(t[0]);
+    if ((tid & 63) == 0) red[tid >> 6] = ws;
+  } else {
+    red[tid] = t[0];
+  }
+}
+
+// R(k) <- (R(k) + conj R(-k))/2 on the self-conjugate planes kz = 0 and nz/2 of a split-form carry
+// (why: see xpass_tile).  The blocks of one launch share the pairs; each pair is one thread's.
+template <typename T>
+__device__ __forceinline__ void split_project(cplx<T>* r, const PParams<T>& p, int ra, int blk, int nblk, int tid,
+                                              int nt) {
+  const int rb = p.ny / ra, nxy = (int)p.nxy;
+  for (int i = blk * nt + tid; i < 2 * nxy; i += nblk * nt) {
+    const int pl = i >= nxy, j = i - pl * nxy;
+    const int kx = j / p.ny, c = j - kx * p.ny, k1 = c / rb, k2 = c - k1 * rb;
+    const int mx = kx == 0 ? 0 : p.nx - kx;
+    const int m1 = k1 == 0 ? 0 : ra - k1;
+    const int m2 = k1 == 0 ? (k2 == 0 ? 0 : rb - k2) : rb - 1 - k2;
+    const int m = mx * p.ny + m1 * rb + m2;
+    if (m < j) continue;
+    cplx<T>* q = r + (pl ? (int64_t)(p.nz / 2) * p.nxy : 0);
+    const cplx<T> a = q[j], b = q[m];
+    const cplx<T> h = mk((T)0.5 * (a.x + b.x), (T)0.5 * (a.y - b.y));
+    q[j] = h;
+    q[m] = conjg(h);
+  }
+}
+
+// Inverse half: radix RA over k1 of the tile's rows and the C2R along z; v receives (psi_a, psi_b) of
+// the column pair q at z = pos_in<inv_last>.  TI: type of the stage array (float: widened).
+template <typename Z, typename TI, typename T = typename Z::T>
+__device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, int rb, int yc, cplx<T>* F,
+                                           const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v) {
+  constexpr int L = Z::L, RA = Z::RA;
+  constexpr uint32_t CB = sizeof(cplx<TI>);
+  for (int i = tid; i < Z::NZH * Z::NY2; i += Z::NT) {
+    const int m = i / Z::NY2, c = i - m * Z::NY2;
+    cplx<T> w[RA];
+    const uint32_t o = (uint32_t)m * rowb + (uint32_t)c * CB, step = (uint32_t)(2 * rb) * CB, odd = (uint32_t)yc * CB;
+#pragma unroll
+    for (int k = 0; k < RA; ++k) {
+      const cplx<TI> g = ld_off(src, o + (uint32_t)(k / 2) * step + (k & 1) * odd);
+      w[k] = mk((T)g.x, (T)g.y);
+    }
+    dft<RA, +1>(w);
+    // only the real parts of kz = 0 and nz/2 enter (the half-complex stage of an FFTW c2r)
+    const T im = (m == 0 || m == L / 2) ? (T)0 : (T)1;
+#pragma unroll
+    for (int k = 0; k < RA; ++k) F[m * Z::HP + k * Z::NY2 + c] = mk(w[k].x, im * w[k].y);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < Z::E; ++e) {
+    const int n = Tile<T, L, Z::E, Z::FP>::template pos_in<inv_first<L, Z::V>()>(tc, e);
+    const bool lo = n <= L / 2;
+    const int m = lo ? n : L - n;
+    const cplx<T> A = F[m * Z::HP + 2 * q], B = F[m * Z::HP + 2 * q + 1];
+    v[e] = lo ? mk(A.x - B.y, A.y + B.x) : mk(A.x + B.y, B.x - A.y);
+  }
+  InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
+}
+
+// Forward half: the R2C along z of the pairs in v and radix RA over y1 of the half spectra.
+template <typename Z, typename T = typename Z::T>
+__device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t rowb, int rb, int yc, cplx<T>* F,
+                                           const cplx<T>* twl, int tid, int q, int tc) {
+  constexpr int L = Z::L, RA = Z::RA;
+  constexpr uint32_t CB = sizeof(cplx<T>);
+  FwdFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
+  __syncthreads();
+  Tile<T, L, Z::E, Z::SP>::template store<fwd_last<L, Z::V>()>(v, F, q, tc);
+  __syncthreads();
+  for (int i = tid; i < Z::NZH * Z::NY2; i += Z::NT) {
+    const int m = i / Z::NY2, c = i - m * Z::NY2;
+    const int mm = m == 0 ? 0 : L - m;
+    cplx<T> w[RA];
+#pragma unroll
+    for (int k = 0; k < RA; ++k) {
+      const int col = k * (Z::NY2 / 2) + c / 2;
+      const cplx<T> W = F[m * Z::SP + col], Wm = F[mm * Z::SP + col];
+      // W = X + iY:  X = (W_k + conj W_{-k})/2,  Y = (W_k - conj W_{-k})/(2i)
+      w[k] = (c & 1) == 0 ? mk((T)0.5 * (W.x + Wm.x), (T)0.5 * (W.y - Wm.y))
+                          : mk((T)0.5 * (W.y + Wm.y), (T)0.5 * (Wm.x - W.x));
+    }
+    dft<RA, -1>(w);
+    const uint32_t o = (uint32_t)m * rowb + (uint32_t)c * CB, step = (uint32_t)(2 * rb) * CB, odd = (uint32_t)yc * CB;
+#pragma unroll
+    for (int k = 0; k < RA; ++k) st_off(dst, o + (uint32_t)(k / 2) * step + (k & 1) * odd, w[k]);
+  }
+}
+
+// Tile of block bz: x and the first y2.  Blocks of one x on consecutive slots of one XCD (workgroups
+// go round the 8 XCDs): they share the 128-byte lines of its rows, whose pieces then meet in one L2.
+__device__ __forceinline__ void zs_tile(int bz, int g, int& x, int& yg) {
+  const int xcd = bz & 7, i = bz >> 3;
+  const int xi = i / g;
+  x = xi * 8 + xcd;
+  yg = i - xi * g;
+}
+
+// nproj leading blocks project R (split_project): the x kernel before left it unprojected, and the
+// one behind needs it.
+template <typename Z, typename T = typename Z::T>
+__device__ __forceinline__ void zsplit_tile(cplx<T>* a, cplx<T>* r, int op, const PParams<T> p, int bx, int nproj) {
+  constexpr int E = Z::E, L = Z::L, RA = Z::RA;
+  __shared__ cplx<T> F[Z::LDS];
+  __shared__ cplx<T> TW[L];
+  __shared__ double red[Z::RED];
+  const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
+  if (bx < nproj) {
+    split_project(r, p, RA, bx, nproj, tid, Z::NT);
+    return;
+  }
+  const int bz = bx - nproj;
+  const cplx<T>* twl = tw_lds<L, Z::NT>(TW, p.twz, tid);
+  const int rb = p.ny / RA;
+  int x, yg;
+  zs_tile(bz, rb / Z::NY2, x, yg);
+  const uint32_t rowb = (uint32_t)p.nxy * (uint32_t)sizeof(cplx<T>);
+  const int yc = split_yc<T>(rb);
+  cplx<T>* base = a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb, yc);
+  cplx<T> v[E];
+  zs_inverse<Z>((const cplx<T>*)base, rowb, rb, yc, F, twl, tid, q, tc, v);
+  constexpr int RP = fwd_first<L, Z::V>();
+  static_assert(fwd_first<L, Z::V>() == inv_last<L, Z::V>(), "plan symmetry");
+  // column pair q: y = (q / (NY2/2)) rb + yg NY2 + 2 (q % (NY2/2)) and the next
+  const bool pen = (op == Z_OP_NL) && p.mid > 0 && p.mid < L - 1;
+  if (pen) {
+    __syncthreads();
+    Tile<T, L, E, Z::FP>::template store<RP>(v, F, q, tc);
+    __syncthreads();
+  }
+  if (op == Z_OP_NL && !pen) {
+    if (p.nl_model == 1) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = mk(nonlin3(p, v[e].x), nonlin3(p, v[e].y));
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = mk(nonlin5(p, v[e].x), nonlin5(p, v[e].y));
+    }
+  } else if (op == Z_OP_NL) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int n = Tile<T, L, E, Z::FP>::template pos_in<RP>(tc, e);
+      T s = nonlin(p, v[e].x), t = nonlin(p, v[e].y);
+      if (n == p.mid) {  // pf3dMorph.cpp:572-581
+        const cplx<T> lo = F[(n - 1) * Z::FP + q], hi = F[(n + 1) * Z::FP + q];
+        s += p.pen * (lo.x - (T)2 * v[e].x + hi.x);
+        t += p.pen * (lo.y - (T)2 * v[e].y + hi.y);
+      }
+      v[e] = mk(s, t);
+    }
+  }
+  if (p.partial != nullptr) zs_partial<T, E, Z::NT>(v, red, tid);
+  zs_forward<Z>(v, base, rowb, rb, yc, F, twl, tid, q, tc);  // its barriers order red[]
+  if (p.partial != nullptr && tid == 0) {
+    double s = 0.0;
+    for (int w = 0; w < Z::RED; ++w) s += red[w];
+    p.partial[bz] = s;
+  }
+}
+template <typename Z>
+__global__ __launch_bounds__(Z::NT) void k_zsplit(SplitArgs<typename Z::T> s, int op, int nproj) {
+  zsplit_tile<Z>(s.a, s.r, op, s.p, blockIdx.x, nproj);
+}
+template <typename Z>
+__global__ __launch_bounds__(Z::NT) void k_zsplit_grp(const SplitArgs<typename Z::T>* __restrict__ g, int op,
+                                                      int nproj) {
+  const SplitArgs<typename Z::T>& b = g[blockIdx.y];
+  zsplit_tile<Z>(b.a, b.r, op, b.p, blockIdx.x, nproj);
+}
+
+// Real field (FP64, dense [x][y][z]) of a split-form stage array of type TI: the inverse half alone.
+template <typename Z, typename TI>
+__global__ __launch_bounds__(Z::NT) void k_zsplit_real(const cplx<TI>* a, double* __restrict__ out, PParams<double> p) {
+  constexpr int L = Z::L, RA = Z::RA;
+  __shared__ cplx<double> F[Z::LDS];
+  __shared__ cplx<double> TW[L];
+  const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
+  const cplx<double>* twl = tw_lds<L, Z::NT>(TW, p.twz, tid);
+  const int rb = p.ny / RA;
+  int x, yg;
+  zs_tile(blockIdx.x, rb / Z::NY2, x, yg);
+  cplx<double> v[Z::E];
+  const int yc = split_yc<TI>(rb);
+  zs_inverse<Z, TI>(a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb, yc),
+                    (uint32_t)p.nxy * (uint32_t)sizeof(cplx<TI>), rb, yc, F, twl, tid, q, tc, v);
+  __syncthreads();
+  Tile<double, L, Z::E, Z::SP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
+  __syncthreads();
+  // lanes run along z of one column pair: two coalesced rows
+  for (int i = tid; i < Z::NPR * L; i += Z::NT) {
+    const int qq = i / L, n = i - qq * L;
+    const int y = (qq / (Z::NY2 / 2)) * rb + yg * Z::NY2 + 2 * (qq % (Z::NY2 / 2));
+    const cplx<double> w = F[n * Z::SP + qq];
+    double* row = out + ((int64_t)x * p.ny + y) * L;
+    row[n] = w.x;
+    row[L + n] = w.y;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// x kernel.  Tile: one kz, NC = whole k1 groups of RB columns, every x.
+// The transform's first exchange passes through the rows: between its store and its load each thread
+// takes the RB columns of one group of a row from the tile, does its part of the y transform and puts
+// them back (rowop), which costs one read and one write of the tile and a barrier.
+template <bool LB, typename T, int L, int E, typename AD, int SIGN, typename Rad> struct RowFFT;
+template <bool LB, typename T, int L, int E, typename AD, int SIGN, int R, int... Rest>
+struct RowFFT<LB, T, L, E, AD, SIGN, Radices<R, Rest...>> {
+  template <typename F>
+  __device__ static __forceinline__ void run(cplx<T>* v, cplx<T>* lds, int col, int tc, const cplx<T>* __restrict__ tw,
+                                             F&& rowop) {
+    constexpr int TPC = L / E;
+#pragma unroll
+    for (int u = 0; u < E / R; ++u) dft<R, SIGN>(&v[u * R]);
+    tile_barrier<LB>();
+#pragma unroll
+    for (int u = 0; u < E / R; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) lds[AD::at((tc + TPC * u) * R + r, col)] = v[u * R + r];
+    tile_barrier<LB>();
+    rowop();
+    tile_barrier<LB>();
+    if constexpr (sizeof...(Rest) > 0) {
+      TileA<T, L, E, AD>::template load<First<Rest...>::value>(v, lds, col, tc);
+      fft_passes<LB, T, L, E, AD, SIGN, R, Rest...>(v, lds, col, tc, tw);
+    } else {
+      TileA<T, L, E, AD>::template load<R>(v, lds, col, tc);
+    }
+  }
+};
+
+template <typename T_, int L_, int RB_, int NC_ = split_nc(RB_), int V_ = split_v<L_>(), int ORD_ = 0>
+struct XS {
+  using T = T_;
+  static constexpr int L = L_, RB = RB_, NC = NC_, V = V_, ORD = ORD_;
+  static constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NC * TPC, NCP = NC + 1, NK = NC / RB;
+  static constexpr bool fits =
+      NT <= 1024 && (size_t)(L * (NC + 2) + NC) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
+};
+
+template <typename X, typename T = typename X::T>
+__device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rbuf, const cplx<T>* __restrict__ twy,
+                                            const PParams<T> p, int bx, int kz) {
+  constexpr int L = X::L, RB = X::RB, NC = X::NC, V = X::V, ORD = X::ORD;
+  constexpr int E = X::E, TPC = X::TPC, NT = X::NT, NCP = X::NCP, NK = X::NK;
+  constexpr uint32_t CB = sizeof(cplx<T>);
+  using AD = RowAddr<NCP>;
+  __shared__ cplx<T> S[L * NCP];
+  __shared__ cplx<T> TW[L];
+  __shared__ T KX[L];
+  __shared__ cplx<T> TWY[NC];  // w_ny^{y2 k1} of the tile's columns
+  const int tid = threadIdx.x, col = tid % NC, tc = tid / NC;
+  const cplx<T>* twl = tw_lds<L, NT>(TW, p.twx, tid);
+  for (int i = tid; i < L; i += NT) KX[i] = p.kx[i];
+  const int ra = p.ny / RB;
+  for (int i = tid; i < NC; i += NT) TWY[i] = twy[(bx * NK + i / RB) * (i % RB)];
+  const int ky = bx * NK + col / RB + ra * (col % RB);
+  const int64_t plane = (int64_t)kz * p.nxy;
+  const uint32_t rowb = (uint32_t)p.ny * CB;
+  const uint32_t cofs = (uint32_t)(bx * NC + col) * CB;  // in the carry's rows
+  const uint32_t aofs = (uint32_t)split_pos(bx * NK + col / RB, col % RB, RB, split_yc<T>(RB)) * CB;
+  cplx<T>* src = a + plane;
+  cplx<T>* rb = rbuf + plane;
+  cplx<T> v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    v[e] = ld_off<cplx<T>>(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<fwd_first<L, V>()>(tc, e) * rowb + aofs);
+  // FP64 mean mode (mixed path): the block owning k = 0 sums the z kernel's partials.
+  double nsum = 0.0;
+  const bool owner0 = (p.partial != nullptr) && kz == 0 && bx == 0;
+  if (owner0) {
+    double* red = reinterpret_cast<double*>(S);  // NT doubles fit: NT <= L NC
+    double s = 0.0;
+    for (int i = tid; i < p.npartial; i += NT) s += p.partial[i];
+    red[tid] = s;
+    __syncthreads();
+    for (int w = 512; w > 0; w >>= 1) {
+      if (tid < w && tid + w < NT) red[tid] += red[tid + w];
+      __syncthreads();
+    }
+    nsum = red[0];
+  }
+  auto fwd_row = [&]() {
+    for (int i = tid; i < L * NK; i += NT) {
+      const int g = i / L, row = i - g * L;
+      cplx<T> w[RB];
+      cplx<T>* s = &S[row * NCP + g * RB];
+      w[0] = s[0];
+#pragma unroll
+      for (int c = 1; c < RB; ++c) w[c] = cmul(s[c], TWY[g * RB + c]);
+      dft<RB, -1>(w);
+#pragma unroll
+      for (int c = 0; c < RB; ++c) s[c] = w[c];
+    }
+  };
+  auto inv_row = [&]() {
+    for (int i = tid; i < L * NK; i += NT) {
+      const int g = i / L, row = i - g * L;
+      cplx<T> w[RB];
+      cplx<T>* s = &S[row * NCP + g * RB];
+#pragma unroll
+      for (int c = 0; c < RB; ++c) w[c] = s[c];
+      dft<RB, +1>(w);
+      s[0] = w[0];
+#pragma unroll
+      for (int c = 1; c < RB; ++c) s[c] = cmul(w[c], conjg(TWY[g * RB + c]));
+    }
+  };
+  cplx<T> cr[(ORD == 2) ? E : 1];
+  RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(v, S, col, tc, twl, fwd_row);
+  const T kyv = p.ky[ky], kzv = p.kz[kz];
+  if constexpr (ORD == 2) {
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      cr[e] = ld_off<cplx<T>>(rb, (uint32_t)Tile<T, L, E, NCP>::template pos_in<fwd_last<L, V>()>(tc, e) * rowb + cofs);
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int kxi = Tile<T, L, E, NCP>::template pos_in<fwd_last<L, V>()>(tc, e);
+    const uint32_t o = (uint32_t)kxi * rowb + cofs;
+    const T kxv = KX[kxi];
+    const T k2 = kxv * kxv + kyv * kyv + kzv * kzv;
+    const T d = k2 - p.q02;
+    const T aLin = p.eps - p.alpha * d * d;                        // pf3d.cpp:205-206
+    const T C1 = (T)1 + p.dtd2 * aLin, C2 = (T)1 - p.dtd2 * aLin;  // :214-215
+    const cplx<T> nn = p.scale * v[e];
+    // psi_new = (R + 3 dt/2 N)/C2, R' = C1 psi_new - dt/2 N (pf3d.cpp:476-478, as xpass_tile)
+    const cplx<T> r = (ORD == 2) ? cr[e] : ld_off<cplx<T>>(rb, o);
+    const T ic2 = recip(C2);
+    cplx<T> ps = mk(ic2 * (r.x + (T)3 * p.dtd2 * nn.x), ic2 * (r.y + (T)3 * p.dtd2 * nn.y));
+    cplx<T> rn = mk(C1 * ps.x - p.dtd2 * nn.x, C1 * ps.y - p.dtd2 * nn.y);
+    if (owner0 && tid == 0 && kxi == 0) {  // k = 0 in FP64
+      const double dd = p.m_dtd2, n0 = p.m_scale * nsum;
+      const double ps0 = (p.mean_state[0] + 3.0 * dd * n0) / p.m_c2;
+      p.mean_state[0] = p.m_c1 * ps0 - dd * n0;
+      p.mean_state[1] = ps0;
+      ps = mk((T)ps0, (T)0);
+      rn = mk((T)p.mean_state[0], (T)0);
+    }
+    st_off(rb, o, rn);
+    v[e] = ps;
+  }
+  RowFFT<true, T, L, E, AD, +1, typename PlanV<L, V>::Inv>::run(v, S, col, tc, twl, inv_row);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    st_off(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<inv_last<L, V>()>(tc, e) * rowb + aofs, v[e]);
+}
+// Tile of linear block b of g column groups a plane: with one k1 per tile, the two tiles that share
+// the stage rows' lines are neighbours on one XCD (whole groups of 16 blocks; the rest in order).
+template <typename X>
+__device__ __forceinline__ void xs_tile(int b, int g, int nzh, int& bx, int& kz) {
+  if (X::NK == 1 && b < g * nzh / 16 * 16) b = (b >> 4) * 16 + (b & 7) * 2 + ((b >> 3) & 1);
+  kz = b / g;
+  bx = b - kz * g;
+}
+template <typename X>
+__global__ __launch_bounds__(X::NT) void k_xsplit(SplitArgs<typename X::T> s) {
+  int bx, kz;
+  xs_tile<X>(blockIdx.x, s.p.ny / X::NC, s.p.nzh, bx, kz);
+  xsplit_tile<X>(s.a, s.r, s.twy, s.p, bx, kz);
+}
+template <typename X>
+__global__ __launch_bounds__(X::NT) void k_xsplit_grp(const SplitArgs<typename X::T>* __restrict__ g) {
+  const SplitArgs<typename X::T>& b = g[blockIdx.y];
+  int bx, kz;
+  xs_tile<X>(blockIdx.x, b.p.ny / X::NC, b.p.nzh, bx, kz);
+  xsplit_tile<X>(b.a, b.r, b.twy, b.p, bx, kz);
+}
+
+// ---------------------------------------------------------------------------
+// Between the two forms.  Rows of ny entries, one per (kz, x); ROWS rows per block of 256 threads.
+//   to standard: ky = k1 + RA k2 from radix RB over y2 with the twiddles, divided by RB (the split
+//   form's y2-space values are an unnormalised inverse); from standard: the inverse of it.
+//   perm: the carry's rows, an order of entries only.
+enum FormDir { FORM_TO_STD = 0, FORM_FROM_STD = 1, FORM_PERM_TO_STD = 2, FORM_PERM_FROM_STD = 3 };
+// YT: the type whose split_yc orders the stage rows (an FP32 array widened to FP64 keeps its order).
+template <typename T, int RB, typename YT = T>
+__global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny,
+                                              const cplx<T>* __restrict__ twy, int dir) {
+  constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
+  constexpr int YC = split_yc<YT>(RB);
+  __shared__ cplx<T> S[CAP + CAP / 16];
+  auto at = [](int i) { return i + (i >> 4); };
+  const int ra = ny / RB, rows = CAP / ny, tid = threadIdx.x;
+  const int64_t r0 = (int64_t)blockIdx.x * rows;
+  const int nr = (int)(nrows - r0 < rows ? nrows - r0 : rows);
+  const int n = nr * ny;
+  const cplx<T>* src = in + r0 * ny;
+  cplx<T>* dst = out + r0 * ny;
+  for (int i = tid; i < n; i += 256) S[at(i)] = src[i];
+  __syncthreads();
+  if (dir == FORM_PERM_TO_STD || dir == FORM_PERM_FROM_STD) {
+    for (int i = tid; i < n; i += 256) {
+      const int row = i / ny, c = i - row * ny;
+      dst[i] = S[at(row * ny + (dir == FORM_PERM_TO_STD ? (c % ra) * RB + c / ra : c / RB + ra * (c % RB)))];
+    }
+    return;
+  }
+  // item: one row and k1; its y2 values at split_pos on one side, its k2 values at k1 + ra k2 on the other
+  constexpr int IPT = (CAP / RB + 255) / 256;
+  cplx<T> w[IPT][RB];
+#pragma unroll
+  for (int it = 0; it < IPT; ++it) {
+    const int i = tid + it * 256, row = i / ra, k1 = i - row * ra;
+    if (i < nr * ra) {
+#pragma unroll
+      for (int c = 0; c < RB; ++c)
+        w[it][c] = dir == FORM_TO_STD ? cmul(S[at(row * ny + split_pos(k1, c, RB, YC))], twy[k1 * c])
+                                      : S[at(row * ny + k1 + ra * c)];
+      if (dir == FORM_TO_STD) {
+        dft<RB, -1>(w[it]);
+#pragma unroll
+        for (int c = 0; c < RB; ++c) w[it][c] = (T)(1.0 / RB) * w[it][c];
+      } else {
+        dft<RB, +1>(w[it]);
+#pragma unroll
+        for (int c = 0; c < RB; ++c) w[it][c] = cmul(w[it][c], conjg(twy[k1 * c]));
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < IPT; ++it) {
+    const int i = tid + it * 256, row = i / ra, k1 = i - row * ra;
+    if (i < nr * ra) {
+#pragma unroll
+      for (int c = 0; c < RB; ++c)
+        S[at(row * ny + (dir == FORM_TO_STD ? k1 + ra * c : split_pos(k1, c, RB, YC)))] = w[it][c];
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) dst[i] = S[at(i)];
+}
+
+}  // namespace smx
+

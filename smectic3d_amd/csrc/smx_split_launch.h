@@ -1,0 +1,183 @@
+// smx_split_launch.h -- runtime-length dispatch of the two-launch step's kernels.
+#pragma once
+#include "smx_launch.h"
+#include "smx_split_ops.h"
+
+namespace smx {
+
+// f(IC<L>, IC<RA>) for a z length and a y split, f(IC<L>, IC<RB>) for an x length and a y split.
+template <typename F>
+hipError_t split_z_dispatch(int nz, int ra, F&& f) {
+#define SMX_CASE(L)                          \
+  if (nz == L) {                             \
+    switch (ra) {                            \
+      case 4: return f(IC<L>{}, IC<4>{});    \
+      case 8: return f(IC<L>{}, IC<8>{});    \
+      case 12: return f(IC<L>{}, IC<12>{});  \
+      case 16: return f(IC<L>{}, IC<16>{});  \
+      case 24: return f(IC<L>{}, IC<24>{});  \
+      default: return hipErrorInvalidValue;  \
+    }                                        \
+  }
+  SMX_FOR_EACH_LENGTH(SMX_CASE)
+#undef SMX_CASE
+  return hipErrorInvalidValue;
+}
+template <typename F>
+hipError_t split_x_dispatch(int nx, int rb, F&& f) {
+#define SMX_CASE(L)                          \
+  if (nx == L) {                             \
+    switch (rb) {                            \
+      case 4: return f(IC<L>{}, IC<4>{});    \
+      case 8: return f(IC<L>{}, IC<8>{});    \
+      case 12: return f(IC<L>{}, IC<12>{});  \
+      case 16: return f(IC<L>{}, IC<16>{});  \
+      default: return hipErrorInvalidValue;  \
+    }                                        \
+  }
+  SMX_FOR_EACH_LENGTH(SMX_CASE)
+#undef SMX_CASE
+  return hipErrorInvalidValue;
+}
+
+#ifdef SMX_SPLIT_Z
+template <typename T>
+bool split_z_fits(int ny, int nz) {
+  const int ra = split_ra(ny);
+  return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
+           using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
+           return Z::fits && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+int split_z_blocks(const PParams<T>& p) {
+  int n = 0;
+  const int ra = split_ra(p.ny);
+  (void)split_z_dispatch(p.nz, ra, [&](auto l, auto r) -> hipError_t {
+    n = p.nx * (p.ny / ra / ZS<T, decltype(l)::value, decltype(r)::value>::NY2);
+    return hipSuccess;
+  });
+  return n;
+}
+// Blocks that project the carry: 8 pairs' entries per thread.
+template <typename Z, typename T>
+static int split_nproj(const PParams<T>& p) {
+  return (int)((2 * p.nxy + 8 * Z::NT - 1) / (8 * Z::NT));
+}
+template <typename T>
+hipError_t split_z(const SplitArgs<T>& s, int op, hipStream_t st) {
+  return split_z_dispatch(s.p.nz, split_ra(s.p.ny), [&](auto l, auto r) -> hipError_t {
+    constexpr int L = decltype(l)::value, RA = decltype(r)::value;
+    using Z = ZS<T, L, RA>;
+    if constexpr (!Z::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      const int np = split_nproj<Z>(s.p);
+      SMX_LAUNCH((k_zsplit<Z>), dim3((unsigned)(np + split_z_blocks(s.p))), dim3(Z::NT), 0, st, s, op, np);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename T>
+hipError_t split_z_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, int op, hipStream_t st) {
+  if (nbox < 1 || nbox > 65535) return hipErrorInvalidValue;
+  return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    constexpr int L = decltype(l)::value, RA = decltype(r)::value;
+    using Z = ZS<T, L, RA>;
+    if constexpr (!Z::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      const int np = split_nproj<Z>(p);
+      SMX_LAUNCH((k_zsplit_grp<Z>), dim3((unsigned)(np + split_z_blocks(p)), (unsigned)nbox), dim3(Z::NT), 0, st,
+                 g, op, np);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_REAL
+bool split_real_fits(int ny, int nz) {
+  const int ra = split_ra(ny);
+  return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
+           using Z = ZS<double, decltype(l)::value, decltype(r)::value>;
+           return Z::fits && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename TI>
+hipError_t split_real(const cplx<TI>* a, double* out, const PParams<double>& p, hipStream_t st) {
+  return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    constexpr int L = decltype(l)::value, RA = decltype(r)::value;
+    using Z = ZS<double, L, RA>;
+    if constexpr (!Z::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_zsplit_real<Z, TI>), dim3((unsigned)(p.nx * (p.ny / RA / Z::NY2))), dim3(Z::NT), 0, st, a, out,
+                 p);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_X
+template <typename T>
+bool split_x_fits(int nx, int ny) {
+  const int ra = split_ra(ny);
+  return ra != 0 && split_x_dispatch(nx, ny / ra, [&](auto l, auto r) -> hipError_t {
+           using X = XS<T, decltype(l)::value, decltype(r)::value>;
+           return X::fits && ny % X::NC == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+hipError_t split_x(const SplitArgs<T>& s, hipStream_t st) {
+  return split_x_dispatch(s.p.nx, s.p.ny / split_ra(s.p.ny), [&](auto l, auto r) -> hipError_t {
+    constexpr int L = decltype(l)::value, RB = decltype(r)::value;
+    using X = XS<T, L, RB>;
+    if constexpr (!X::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_xsplit<X>), dim3((unsigned)(s.p.ny / X::NC * s.p.nzh)), dim3(X::NT), 0, st, s);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename T>
+hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, hipStream_t st) {
+  if (nbox < 1 || nbox > 65535) return hipErrorInvalidValue;
+  return split_x_dispatch(p.nx, p.ny / split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    constexpr int L = decltype(l)::value, RB = decltype(r)::value;
+    using X = XS<T, L, RB>;
+    if constexpr (!X::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_xsplit_grp<X>), dim3((unsigned)(p.ny / X::NC * p.nzh), (unsigned)nbox), dim3(X::NT), 0, st, g);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename T, int RB>
+static void split_form_launch(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+                              bool wide, hipStream_t st) {
+  const int rows = 1024 / ny;
+  const dim3 grid((unsigned)((nrows + rows - 1) / rows));
+  if (wide) SMX_LAUNCH((k_form<T, RB, float>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir);
+  else SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir);
+}
+template <typename T>
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir, bool wide,
+                      hipStream_t st) {
+  const int ra = split_ra(ny);
+  if (ra == 0) return hipErrorInvalidValue;
+  switch (ny / ra) {
+    case 4: split_form_launch<T, 4>(in, out, nrows, ny, twy, dir, wide, st); break;
+    case 8: split_form_launch<T, 8>(in, out, nrows, ny, twy, dir, wide, st); break;
+    case 12: split_form_launch<T, 12>(in, out, nrows, ny, twy, dir, wide, st); break;
+    case 16: split_form_launch<T, 16>(in, out, nrows, ny, twy, dir, wide, st); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+#endif
+
+}  // namespace smx

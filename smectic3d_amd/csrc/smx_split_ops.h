@@ -1,0 +1,30 @@
+// smx_split_ops.h -- host launchers of the two-launch step (smx_split.h).  The definitions are in
+// smx_split_launch.h, instantiated per precision in smx_split_z_*.hip and smx_split_x_*.hip.
+#pragma once
+#include "smx_split.h"
+
+namespace smx {
+
+// Whether the two kernels exist for this grid: ny has a split and both tiles fit a workgroup.
+template <typename T> bool split_z_fits(int ny, int nz);
+template <typename T> bool split_x_fits(int nx, int ny);
+
+// Blocks of the z kernel that take a tile each (one FP64 partial per block).
+template <typename T> int split_z_blocks(const PParams<T>& p);
+template <typename T> hipError_t split_z(const SplitArgs<T>& s, int op, hipStream_t st);
+template <typename T> hipError_t split_x(const SplitArgs<T>& s, hipStream_t st);
+// One launch for nbox boxes of one grid (arguments in device memory).
+template <typename T>
+hipError_t split_z_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, int op, hipStream_t st);
+template <typename T> hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, hipStream_t st);
+// FP64 real field of a split-form stage array of type TI.
+template <typename TI>
+hipError_t split_real(const cplx<TI>* a, double* out, const PParams<double>& p, hipStream_t st);
+bool split_real_fits(int ny, int nz);
+// Rows of a stage array (or, with the perm directions, of the carry) between the two forms, in place
+// allowed.  wide: FP64 rows that were widened from FP32 ones (which have another order).
+template <typename T>
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir, bool wide,
+                      hipStream_t st);
+
+}  // namespace smx
