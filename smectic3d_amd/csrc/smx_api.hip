@@ -555,11 +555,10 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
 }
 
 // ---- the two forms of a periodic state (smx_split.h) ----
-// Rows of a stage array or carry from one form to the other on the handle's stream, in place
-// allowed.  wide: an FP64 copy of an FP32 array.
+// Rows of a stage array or carry from one form to the other on the handle's stream, in place allowed.
 template <typename T>
-static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, bool wide = false) {
-  const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, wide, h->st);
+static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
+  const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
   if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
   return SMX_OK;
 }
@@ -591,7 +590,7 @@ static int stage_to_f64(smx_handle* h, const void* stage, void* dst, bool split)
                        (double*)dst, ncomp);
     HIPCHK(hipGetLastError());
     if (split)
-      CHK(form_rows<double>(h, (const cplx<double>*)dst, (cplx<double>*)dst, FORM_TO_STD, true));
+      CHK(form_rows<double>(h, (const cplx<double>*)dst, (cplx<double>*)dst, FORM_TO_STD));
     if (!h->neumann) {
       const int64_t pairs = 2 * (int64_t)h->cfg.nx * (h->cfg.ny / 2 + 1);
       hipLaunchKernelGGL(k_herm_stage, dim3((unsigned)std::min<int64_t>((pairs + 255) / 256, 4096)), dim3(256), 0,
@@ -1672,8 +1671,8 @@ static bool same_operator(const smx_config& a, const smx_config& b) {
 }
 
 static int64_t split_layout(const smx_handle* h) {
-  const int ra = split_ra(h->cfg.ny), rb = ra ? h->cfg.ny / ra : 0;
-  return ra ? ra * 65536 + (h->fp32 ? split_yc<float>(rb) : split_yc<double>(rb)) : 0;
+  const int ra = split_ra(h->cfg.ny);
+  return ra ? ra * 65536 + kSplitYC : 0;
 }
 
 static std::vector<void*> carried_arrays(smx_handle* h) {

@@ -13,8 +13,8 @@
 // and the carry R(kx, ky = k1 + RA k2, kz) is at [kz][kx][k1 RB + k2] (the split form; the four-pass
 // kernels of smx_periodic.h and the diagnostics use the standard one, ky at its index).
 //
-// Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 67 + 98 us and
-// 41 + 47 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
+// Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 64 + 98 us and
+// 33 + 47 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
 // from two launches in place of four as well: 64^3 FP32 3.71 -> 2.97 ms for 200 steps and their checks.
 #pragma once
 #include "smx_periodic.h"
@@ -24,8 +24,8 @@ namespace smx {
 // RA of a length (RB = ny / RA); 0: no split.  Both tiles hold NZ RA (2 or 4) / 2 and NX RB values, so
 // the two factors are near each other and RB <= 16 (an x tile of 256 x 16 FP64 values is 64 KB).
 constexpr int split_ra(int ny) {
-  return ny == 16 || ny == 32 || ny == 48 ? 4
-         : ny == 64 || ny == 96 || ny == 128 ? 8
+  return ny == 16 || ny == 48 ? 4
+         : ny == 32 || ny == 64 || ny == 96 || ny == 128 ? 8
          : ny == 192 ? 12
          : ny == 256 ? 16
          : ny == 384 ? 24
@@ -33,23 +33,26 @@ constexpr int split_ra(int ny) {
 }
 
 // Position of (k1, y2) in a split-form stage row: pieces of YC adjacent y2 of two adjacent k1.  The z
-// kernel's tile has every k1 and few y2, the x kernel's few k1 and every y2, so with either index
-// alone fastest one of the two would touch a quarter of each 128-byte line; in this order both use
-// at least half of the lines that they touch.
+// kernel's tile has every k1 and YC y2, the x kernel's few k1 and every y2, so with either index alone
+// fastest one of the two would touch a quarter of each 128-byte line; in this order both use half of
+// the lines that they touch.
+constexpr int kSplitYC = 4;
+__host__ __device__ __forceinline__ int split_pos(int k1, int y2, int rb) {
+  constexpr int YC = kSplitYC;
+  return (k1 >> 1) * 2 * rb + (y2 / YC) * 2 * YC + (k1 & 1) * YC + y2 % YC;
+}
+// y2 of a z tile: a whole piece or half of one (the tile's two parities of k1 share a line).  Whole pieces
+// where two blocks of the tile still fit a CU (192 x 96 x 384 FP64: 37.6 us with halves, 48.6 with one
+// block of whole pieces; 256^3 FP32: 34 with whole, 42 with halves), except in the shortest boxes, which
+// want more blocks (96^3 FP64 10.9 against 12.1 us, 128^3 FP32 11.7 against 10.2).
 template <typename T>
-__host__ __device__ constexpr int split_yc(int rb) {
-  return sizeof(T) == 4 && rb % 8 == 0 ? 8 : 4;
+constexpr int split_ny2(int l, int ra) {
+  return (l > 96 || ra == 4) && l * (2 * ra + 2) * 2 * (int)sizeof(T) <= 80 * 1024 && (ra <= 8 || sizeof(T) == 4) ? 4 : 2;
 }
-__host__ __device__ __forceinline__ int split_pos(int k1, int y2, int rb, int yc) {
-  return (k1 >> 1) * 2 * rb + (y2 / yc) * 2 * yc + (k1 & 1) * yc + y2 % yc;
-}
+// Lanes that share one y line in the z kernel (pair_dft): two from radix 16 on, where one lane's 16
+// values make its loads the longest part (256^3 FP32: 40.6 -> 34.0 us; 192^3 FP32: 22.3 with one, 27.7).
+constexpr int split_lanes(int ra) { return ra >= 16 ? 2 : 1; }
 
-// y2 values per z tile (they are contiguous in the stage rows, and adjacent ones share a complex
-// transform).
-template <typename T, int L, int RA>
-constexpr int split_ny2() {
-  return RA <= 8 ? 4 : (sizeof(T) == 4 && L >= 256 && RA <= 16 ? 4 : 2);
-}
 // Plan variants: E = 8 where the length has it; E = 16 for the FP32 z kernel at 256 and 512.
 template <int L>
 constexpr int split_v() {
@@ -59,8 +62,19 @@ template <typename T, int L>
 constexpr int split_zv() {
   return sizeof(T) == 4 && L >= 256 ? 0 : split_v<L>();
 }
-// Columns per x tile: whole k1 groups of RB.
-constexpr int split_nc(int rb) { return rb <= 8 ? 16 : rb; }
+// Whether the x kernel reads the carry together with the stage rows.  In short boxes, which are bound by
+// latency (64^3 FP32 5.4 -> 4.8 us, 96^3 11.6 -> 10.2); in others the registers cost a block per CU
+// (256^3 FP64 102 -> 116 us).
+template <typename T, int L>
+constexpr bool split_pre() {
+  return L <= 96 || (sizeof(T) == 4 && L <= 128);
+}
+// Columns per x tile: whole k1 groups of RB, rows of 128 bytes or more (96^3 FP32 with 12 columns 10.2
+// us, with 24 9.3; FP64 keeps 12, twice the blocks).
+template <typename T>
+constexpr int split_nc(int rb) {
+  return rb <= 8 ? 16 : (rb == 12 && sizeof(T) == 4 ? 24 : rb);
+}
 
 template <typename T>
 struct SplitArgs {
@@ -72,16 +86,26 @@ struct SplitArgs {
 
 // ---------------------------------------------------------------------------
 // z kernel.  Tile: one x, NY2 adjacent y2, every k1 (y1) and kz.
-template <typename T_, int L_, int RA_, int NY2_ = split_ny2<T_, L_, RA_>(), int V_ = split_zv<T_, L_>()>
+template <typename T_, int L_, int RA_, int NY2_ = split_ny2<T_>(L_, RA_), int V_ = split_zv<T_, L_>(),
+          int P_ = split_lanes(RA_)>
 struct ZS {
   using T = T_;
-  static constexpr int L = L_, RA = RA_, NY2 = NY2_, V = V_;
+  static constexpr int L = L_, RA = RA_, NY2 = NY2_, V = V_, P = P_;
   static constexpr int E = PlanV<L, V>::E, TPC = L / E;
   static constexpr int NPR = RA * NY2 / 2, NT = NPR * TPC, NZH = L / 2 + 1;
-  // Half-spectrum tile [kz][y1][y2]: rows padded by 32 bytes, so that the NY2-wide pieces which
-  // lanes write down consecutive kz fall in different banks.
-  static constexpr int HP = RA * NY2 + 32 / (int)sizeof(cplx<T>);
-  static constexpr int FP = NPR, SP = NPR + 1;  // transform tile pitch; pitch of the split's copy
+  // Half-spectrum tile [kz][part of the y1][y1][y2]: the parts PH apart and rows HP, so that the
+  // pieces which lanes write (P parts x NY2 x consecutive kz) fall in different banks: 8 banks from
+  // part to part, 8 P from row to row.
+  static constexpr int DW = sizeof(cplx<T>) / 4;  // banks of a value
+  static constexpr int pad_to(int n, int banks) {
+    while (n * DW % 64 != banks) ++n;
+    return n;
+  }
+  static constexpr int H = RA / P;
+  static constexpr int PH = P == 2 ? pad_to(H * NY2, 8) : 0, HP = pad_to(PH + H * NY2, 8 * P);
+  static constexpr int FP = NPR, SP = NPR + NY2 / 2;  // transform tile pitch; pitch of the split's copy
+  // Items of the y part, H values each: one kz, one y2 and (P = 2) one parity of k1, half of the y1.
+  static constexpr int ITEMS = NZH * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
   static constexpr int LDS = (NZH * HP > L * SP ? NZH * HP : L * SP);
   static constexpr int RED = (NT % 64 == 0) ? NT / 64 : NT;
   static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
@@ -128,35 +152,104 @@ __device__ __forceinline__ void split_project(cplx<T>* r, const PParams<T>& p, i
   }
 }
 
+// The value of the neighbouring lane (lane ^ 1).
+__device__ __forceinline__ float lane_xor1(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_xor1(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, 0xB1, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), 0xB1, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// w[y] times e^{SIGN 2 pi i y / R}
+template <int R, int SIGN, int Y, int N, typename T>
+__device__ __forceinline__ void rot_all(cplx<T>* w) {
+  if constexpr (Y < N) {
+    w[Y] = rot<R, Y, SIGN>(w[Y]);
+    rot_all<R, SIGN, Y + 1, N>(w);
+  }
+}
+// Radix 2 H of one line held by two adjacent lanes: even and odd inputs (SIGN > 0: lane parity = k1
+// parity in, half of the y1 out) or the other way round (SIGN < 0).  The pair and its neighbours load
+// and store whole lines' halves together, and every thread of the block has a part of the work.
+template <int H, int SIGN, typename T>
+__device__ __forceinline__ void pair_dft(cplx<T>* w, int lo) {
+  const T sgn = lo ? (T)-1 : (T)1;
+  auto cross = [&]() {
+#pragma unroll
+    for (int y = 0; y < H; ++y) {
+      const cplx<T> o = mk(lane_xor1(w[y].x), lane_xor1(w[y].y));
+      w[y] = mk(o.x + sgn * w[y].x, o.y + sgn * w[y].y);
+    }
+  };
+  if constexpr (SIGN > 0) {
+    dft<H, +1>(w);
+    if (lo) rot_all<2 * H, +1, 0, H>(w);
+    cross();
+  } else {
+    cross();
+    if (lo) rot_all<2 * H, -1, 0, H>(w);
+    dft<H, -1>(w);
+  }
+}
+
+// Byte offset of an item's value k: every other k1 (P = 2) or every k1; step: two k1 apart.
+template <typename Z>
+__device__ __forceinline__ uint32_t zs_leg(int k, uint32_t step, uint32_t cb) {
+  return Z::P == 2 ? (uint32_t)k * step : (uint32_t)(k / 2) * step + (uint32_t)((k & 1) * kSplitYC) * cb;
+}
+
 // Inverse half: radix RA over k1 of the tile's rows and the C2R along z; v receives (psi_a, psi_b) of
-// the column pair q at z = pos_in<inv_last>.  TI: type of the stage array (float: widened).
+// the column pair q at z = pos_in<inv_last>.  TI: type of the stage array (float: widened).  kzm: k_z
+// table of the spectral d/dz (rows times i k_z, Nyquist +pi/dz, pf3d.cpp:184), or nullptr.  twg: the
+// z twiddles in memory, copied to twl behind the tile's loads, or nullptr if they are there.
 template <typename Z, typename TI, typename T = typename Z::T>
-__device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, int rb, int yc, cplx<T>* F,
-                                           const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v) {
+__device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F,
+                                           const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v,
+                                           const T* kzm = nullptr, const cplx<T>* twg = nullptr) {
   constexpr int L = Z::L, RA = Z::RA;
   constexpr uint32_t CB = sizeof(cplx<TI>);
-  for (int i = tid; i < Z::NZH * Z::NY2; i += Z::NT) {
-    const int m = i / Z::NY2, c = i - m * Z::NY2;
-    cplx<T> w[RA];
-    const uint32_t o = (uint32_t)m * rowb + (uint32_t)c * CB, step = (uint32_t)(2 * rb) * CB, odd = (uint32_t)yc * CB;
+  cplx<T> w[Z::IPT][Z::H];
 #pragma unroll
-    for (int k = 0; k < RA; ++k) {
-      const cplx<TI> g = ld_off(src, o + (uint32_t)(k / 2) * step + (k & 1) * odd);
-      w[k] = mk((T)g.x, (T)g.y);
+  for (int it = 0; it < Z::IPT; ++it) {  // every load is issued before the first is used
+    const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, m = i / Z::P / Z::NY2;
+    if (i < Z::ITEMS) {
+      const uint32_t o = (uint32_t)m * rowb + (uint32_t)(c + lo * kSplitYC) * CB, step = (uint32_t)(2 * rb) * CB;
+#pragma unroll
+      for (int k = 0; k < Z::H; ++k) {
+        const cplx<TI> g = ld_off(src, o + zs_leg<Z>(k, step, CB));
+        w[it][k] = mk((T)g.x, (T)g.y);
+      }
     }
-    dft<RA, +1>(w);
-    // only the real parts of kz = 0 and nz/2 enter (the half-complex stage of an FFTW c2r)
-    const T im = (m == 0 || m == L / 2) ? (T)0 : (T)1;
+  }
+  if (twg != nullptr) tw_lds<L, Z::NT>(const_cast<cplx<T>*>(twl), twg, tid);
 #pragma unroll
-    for (int k = 0; k < RA; ++k) F[m * Z::HP + k * Z::NY2 + c] = mk(w[k].x, im * w[k].y);
+  for (int it = 0; it < Z::IPT; ++it) {
+    const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, m = i / Z::P / Z::NY2;
+    if (i < Z::ITEMS) {
+      if constexpr (Z::P == 2) pair_dft<Z::H, +1>(w[it], lo);
+      else dft<Z::H, +1>(w[it]);
+      if (kzm != nullptr) {
+        const T kz = kzm[m];
+#pragma unroll
+        for (int k = 0; k < Z::H; ++k) w[it][k] = mk(-kz * w[it][k].y, kz * w[it][k].x);
+      }
+      // only the real parts of kz = 0 and nz/2 enter (the half-complex stage of an FFTW c2r)
+      const T im = (m == 0 || m == L / 2) ? (T)0 : (T)1;
+      cplx<T>* f = &F[m * Z::HP + lo * Z::PH + c];
+#pragma unroll
+      for (int k = 0; k < Z::H; ++k) f[k * Z::NY2] = mk(w[it][k].x, im * w[it][k].y);
+    }
   }
   __syncthreads();
+  const int qa = Z::P == 1 || q < Z::NPR / 2 ? 2 * q : 2 * q - Z::NPR + Z::PH;
 #pragma unroll
   for (int e = 0; e < Z::E; ++e) {
     const int n = Tile<T, L, Z::E, Z::FP>::template pos_in<inv_first<L, Z::V>()>(tc, e);
     const bool lo = n <= L / 2;
     const int m = lo ? n : L - n;
-    const cplx<T> A = F[m * Z::HP + 2 * q], B = F[m * Z::HP + 2 * q + 1];
+    const cplx<T> A = F[m * Z::HP + qa], B = F[m * Z::HP + qa + 1];
     v[e] = lo ? mk(A.x - B.y, A.y + B.x) : mk(A.x + B.y, B.x - A.y);
   }
   InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
@@ -164,7 +257,7 @@ __device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, i
 
 // Forward half: the R2C along z of the pairs in v and radix RA over y1 of the half spectra.
 template <typename Z, typename T = typename Z::T>
-__device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t rowb, int rb, int yc, cplx<T>* F,
+__device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t rowb, int rb, cplx<T>* F,
                                            const cplx<T>* twl, int tid, int q, int tc) {
   constexpr int L = Z::L, RA = Z::RA;
   constexpr uint32_t CB = sizeof(cplx<T>);
@@ -172,22 +265,26 @@ __device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t ro
   __syncthreads();
   Tile<T, L, Z::E, Z::SP>::template store<fwd_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
-  for (int i = tid; i < Z::NZH * Z::NY2; i += Z::NT) {
-    const int m = i / Z::NY2, c = i - m * Z::NY2;
-    const int mm = m == 0 ? 0 : L - m;
-    cplx<T> w[RA];
 #pragma unroll
-    for (int k = 0; k < RA; ++k) {
-      const int col = k * (Z::NY2 / 2) + c / 2;
-      const cplx<T> W = F[m * Z::SP + col], Wm = F[mm * Z::SP + col];
-      // W = X + iY:  X = (W_k + conj W_{-k})/2,  Y = (W_k - conj W_{-k})/(2i)
-      w[k] = (c & 1) == 0 ? mk((T)0.5 * (W.x + Wm.x), (T)0.5 * (W.y - Wm.y))
-                          : mk((T)0.5 * (W.y + Wm.y), (T)0.5 * (Wm.x - W.x));
+  for (int it = 0; it < Z::IPT; ++it) {
+    const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, m = i / Z::P / Z::NY2;
+    if (i < Z::ITEMS) {
+      const int mm = m == 0 ? 0 : L - m;
+      cplx<T> w[Z::H];
+#pragma unroll
+      for (int k = 0; k < Z::H; ++k) {
+        const int col = (lo * Z::H + k) * (Z::NY2 / 2) + c / 2;
+        const cplx<T> W = F[m * Z::SP + col], Wm = F[mm * Z::SP + col];
+        // W = X + iY:  X = (W_k + conj W_{-k})/2,  Y = (W_k - conj W_{-k})/(2i)
+        w[k] = (c & 1) == 0 ? mk((T)0.5 * (W.x + Wm.x), (T)0.5 * (W.y - Wm.y))
+                            : mk((T)0.5 * (W.y + Wm.y), (T)0.5 * (Wm.x - W.x));
+      }
+      if constexpr (Z::P == 2) pair_dft<Z::H, -1>(w, lo);
+      else dft<Z::H, -1>(w);
+      const uint32_t o = (uint32_t)m * rowb + (uint32_t)(c + lo * kSplitYC) * CB, step = (uint32_t)(2 * rb) * CB;
+#pragma unroll
+      for (int k = 0; k < Z::H; ++k) st_off(dst, o + zs_leg<Z>(k, step, CB), w[k]);
     }
-    dft<RA, -1>(w);
-    const uint32_t o = (uint32_t)m * rowb + (uint32_t)c * CB, step = (uint32_t)(2 * rb) * CB, odd = (uint32_t)yc * CB;
-#pragma unroll
-    for (int k = 0; k < RA; ++k) st_off(dst, o + (uint32_t)(k / 2) * step + (k & 1) * odd, w[k]);
   }
 }
 
@@ -214,15 +311,13 @@ __device__ __forceinline__ void zsplit_tile(cplx<T>* a, cplx<T>* r, int op, cons
     return;
   }
   const int bz = bx - nproj;
-  const cplx<T>* twl = tw_lds<L, Z::NT>(TW, p.twz, tid);
   const int rb = p.ny / RA;
   int x, yg;
   zs_tile(bz, rb / Z::NY2, x, yg);
   const uint32_t rowb = (uint32_t)p.nxy * (uint32_t)sizeof(cplx<T>);
-  const int yc = split_yc<T>(rb);
-  cplx<T>* base = a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb, yc);
+  cplx<T>* base = a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb);
   cplx<T> v[E];
-  zs_inverse<Z>((const cplx<T>*)base, rowb, rb, yc, F, twl, tid, q, tc, v);
+  zs_inverse<Z>((const cplx<T>*)base, rowb, rb, F, TW, tid, q, tc, v, (const T*)nullptr, p.twz);
   constexpr int RP = fwd_first<L, Z::V>();
   static_assert(fwd_first<L, Z::V>() == inv_last<L, Z::V>(), "plan symmetry");
   // column pair q: y = (q / (NY2/2)) rb + yg NY2 + 2 (q % (NY2/2)) and the next
@@ -254,7 +349,7 @@ __device__ __forceinline__ void zsplit_tile(cplx<T>* a, cplx<T>* r, int op, cons
     }
   }
   if (p.partial != nullptr) zs_partial<T, E, Z::NT>(v, red, tid);
-  zs_forward<Z>(v, base, rowb, rb, yc, F, twl, tid, q, tc);  // its barriers order red[]
+  zs_forward<Z>(v, base, rowb, rb, F, TW, tid, q, tc);  // its barriers order red[]
   if (p.partial != nullptr && tid == 0) {
     double s = 0.0;
     for (int w = 0; w < Z::RED; ++w) s += red[w];
@@ -279,14 +374,13 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_real(const cplx<TI>* a, double
   __shared__ cplx<double> F[Z::LDS];
   __shared__ cplx<double> TW[L];
   const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
-  const cplx<double>* twl = tw_lds<L, Z::NT>(TW, p.twz, tid);
   const int rb = p.ny / RA;
   int x, yg;
   zs_tile(blockIdx.x, rb / Z::NY2, x, yg);
   cplx<double> v[Z::E];
-  const int yc = split_yc<TI>(rb);
-  zs_inverse<Z, TI>(a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb, yc),
-                    (uint32_t)p.nxy * (uint32_t)sizeof(cplx<TI>), rb, yc, F, twl, tid, q, tc, v);
+  zs_inverse<Z, TI>(a + (int64_t)x * p.ny + split_pos(0, yg * Z::NY2, rb),
+                    (uint32_t)p.nxy * (uint32_t)sizeof(cplx<TI>), rb, F, TW, tid, q, tc, v,
+                    (const double*)nullptr, p.twz);
   __syncthreads();
   Tile<double, L, Z::E, Z::SP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
@@ -332,62 +426,30 @@ struct RowFFT<LB, T, L, E, AD, SIGN, Radices<R, Rest...>> {
   }
 };
 
-template <typename T_, int L_, int RB_, int NC_ = split_nc(RB_), int V_ = split_v<L_>(), int ORD_ = 0>
+template <typename T_, int L_, int RB_, int NC_ = split_nc<T_>(RB_), int V_ = split_v<L_>(),
+          bool PRE_ = split_pre<T_, L_>()>
 struct XS {
   using T = T_;
-  static constexpr int L = L_, RB = RB_, NC = NC_, V = V_, ORD = ORD_;
+  static constexpr int L = L_, RB = RB_, NC = NC_, V = V_;
+  static constexpr bool PRE = PRE_;  // the carry is read with the stage rows
   static constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NC * TPC, NCP = NC + 1, NK = NC / RB;
+  using AD = RowAddr<NCP>;
   static constexpr bool fits =
-      NT <= 1024 && (size_t)(L * (NC + 2) + NC) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
+      NT <= 1024 && (size_t)(L * (NCP + 1) + NC) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
 };
 
-template <typename X, typename T = typename X::T>
-__device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rbuf, const cplx<T>* __restrict__ twy,
-                                            const PParams<T> p, int bx, int kz) {
-  constexpr int L = X::L, RB = X::RB, NC = X::NC, V = X::V, ORD = X::ORD;
-  constexpr int E = X::E, TPC = X::TPC, NT = X::NT, NCP = X::NCP, NK = X::NK;
-  constexpr uint32_t CB = sizeof(cplx<T>);
-  using AD = RowAddr<NCP>;
-  __shared__ cplx<T> S[L * NCP];
-  __shared__ cplx<T> TW[L];
-  __shared__ T KX[L];
-  __shared__ cplx<T> TWY[NC];  // w_ny^{y2 k1} of the tile's columns
-  const int tid = threadIdx.x, col = tid % NC, tc = tid / NC;
-  const cplx<T>* twl = tw_lds<L, NT>(TW, p.twx, tid);
-  for (int i = tid; i < L; i += NT) KX[i] = p.kx[i];
-  const int ra = p.ny / RB;
-  for (int i = tid; i < NC; i += NT) TWY[i] = twy[(bx * NK + i / RB) * (i % RB)];
-  const int ky = bx * NK + col / RB + ra * (col % RB);
-  const int64_t plane = (int64_t)kz * p.nxy;
-  const uint32_t rowb = (uint32_t)p.ny * CB;
-  const uint32_t cofs = (uint32_t)(bx * NC + col) * CB;  // in the carry's rows
-  const uint32_t aofs = (uint32_t)split_pos(bx * NK + col / RB, col % RB, RB, split_yc<T>(RB)) * CB;
-  cplx<T>* src = a + plane;
-  cplx<T>* rb = rbuf + plane;
-  cplx<T> v[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e)
-    v[e] = ld_off<cplx<T>>(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<fwd_first<L, V>()>(tc, e) * rowb + aofs);
-  // FP64 mean mode (mixed path): the block owning k = 0 sums the z kernel's partials.
-  double nsum = 0.0;
-  const bool owner0 = (p.partial != nullptr) && kz == 0 && bx == 0;
-  if (owner0) {
-    double* red = reinterpret_cast<double*>(S);  // NT doubles fit: NT <= L NC
-    double s = 0.0;
-    for (int i = tid; i < p.npartial; i += NT) s += p.partial[i];
-    red[tid] = s;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-      if (tid < w && tid + w < NT) red[tid] += red[tid + w];
-      __syncthreads();
-    }
-    nsum = red[0];
-  }
-  auto fwd_row = [&]() {
+// The x tile's part of the y transform on its rows: y2 -> k2 (twiddles, then radix RB) and back.
+// Lanes run down the rows; TWY: w_ny^{y2 k1} of the tile's columns.
+template <typename X>
+struct XRow {
+  using T = typename X::T;
+  using AD = typename X::AD;
+  static constexpr int L = X::L, RB = X::RB, NK = X::NK, NT = X::NT;
+  __device__ static __forceinline__ void fwd(cplx<T>* S, const cplx<T>* TWY, int tid) {
     for (int i = tid; i < L * NK; i += NT) {
       const int g = i / L, row = i - g * L;
       cplx<T> w[RB];
-      cplx<T>* s = &S[row * NCP + g * RB];
+      cplx<T>* s = &S[AD::at(row, g * RB)];
       w[0] = s[0];
 #pragma unroll
       for (int c = 1; c < RB; ++c) w[c] = cmul(s[c], TWY[g * RB + c]);
@@ -395,12 +457,12 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
 #pragma unroll
       for (int c = 0; c < RB; ++c) s[c] = w[c];
     }
-  };
-  auto inv_row = [&]() {
+  }
+  __device__ static __forceinline__ void inv(cplx<T>* S, const cplx<T>* TWY, int tid) {
     for (int i = tid; i < L * NK; i += NT) {
       const int g = i / L, row = i - g * L;
       cplx<T> w[RB];
-      cplx<T>* s = &S[row * NCP + g * RB];
+      cplx<T>* s = &S[AD::at(row, g * RB)];
 #pragma unroll
       for (int c = 0; c < RB; ++c) w[c] = s[c];
       dft<RB, +1>(w);
@@ -408,15 +470,66 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
 #pragma unroll
       for (int c = 1; c < RB; ++c) s[c] = cmul(w[c], conjg(TWY[g * RB + c]));
     }
-  };
-  cplx<T> cr[(ORD == 2) ? E : 1];
-  RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(v, S, col, tc, twl, fwd_row);
-  const T kyv = p.ky[ky], kzv = p.kz[kz];
-  if constexpr (ORD == 2) {
+  }
+};
+
+// Sum of the z kernel's FP64 partials over the block, in a fixed order; S is free.
+template <typename X, typename T = typename X::T>
+__device__ __forceinline__ double xs_partial_sum(const PParams<T>& p, cplx<T>* S, int tid) {
+  double* red = reinterpret_cast<double*>(S);  // NT doubles fit: NT <= L NC
+  double s = 0.0;
+  for (int i = tid; i < p.npartial; i += X::NT) s += p.partial[i];
+  red[tid] = s;
+  __syncthreads();
+  for (int w = 512; w > 0; w >>= 1) {
+    if (tid < w && tid + w < X::NT) red[tid] += red[tid + w];
+    __syncthreads();
+  }
+  return red[0];
+}
+
+template <typename X, typename T = typename X::T>
+__device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rbuf, const cplx<T>* __restrict__ twy,
+                                            const PParams<T> p, int bx, int kz) {
+  constexpr int L = X::L, RB = X::RB, NC = X::NC, V = X::V;
+  constexpr int E = X::E, TPC = X::TPC, NT = X::NT, NCP = X::NCP, NK = X::NK;
+  constexpr uint32_t CB = sizeof(cplx<T>);
+  using AD = typename X::AD;
+  __shared__ cplx<T> S[L * NCP];
+  __shared__ cplx<T> TW[L];
+  __shared__ T KX[L];
+  __shared__ cplx<T> TWY[NC];  // w_ny^{y2 k1} of the tile's columns
+  const int tid = threadIdx.x, col = tid % NC, tc = tid / NC;
+  const int ra = p.ny / RB;
+  const int ky = bx * NK + col / RB + ra * (col % RB);
+  const int64_t plane = (int64_t)kz * p.nxy;
+  const uint32_t rowb = (uint32_t)p.ny * CB;
+  const uint32_t cofs = (uint32_t)(bx * NC + col) * CB;  // in the carry's rows
+  const uint32_t aofs = (uint32_t)split_pos(bx * NK + col / RB, col % RB, RB) * CB;
+  cplx<T>* src = a + plane;
+  cplx<T>* rb = rbuf + plane;
+  cplx<T> v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    v[e] = ld_off<cplx<T>>(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<fwd_first<L, V>()>(tc, e) * rowb + aofs);
+  cplx<T> cr[X::PRE ? E : 1];
+  if constexpr (X::PRE) {
 #pragma unroll
     for (int e = 0; e < E; ++e)
       cr[e] = ld_off<cplx<T>>(rb, (uint32_t)Tile<T, L, E, NCP>::template pos_in<fwd_last<L, V>()>(tc, e) * rowb + cofs);
   }
+  // the tables behind the tile's loads, so that their latencies overlap
+  const cplx<T>* twl = tw_lds<L, NT>(TW, p.twx, tid);
+  for (int i = tid; i < L; i += NT) KX[i] = p.kx[i];
+  for (int i = tid; i < NC; i += NT) TWY[i] = twy[(bx * NK + i / RB) * (i % RB)];
+  const T kyv = p.ky[ky], kzv = p.kz[kz];
+  // FP64 mean mode (mixed path): the block owning k = 0 sums the z kernel's partials.
+  double nsum = 0.0;
+  const bool owner0 = (p.partial != nullptr) && kz == 0 && bx == 0;
+  if (owner0) nsum = xs_partial_sum<X>(p, S, tid);
+  auto fwd_row = [&]() { XRow<X>::fwd(S, TWY, tid); };
+  auto inv_row = [&]() { XRow<X>::inv(S, TWY, tid); };
+  RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(v, S, col, tc, twl, fwd_row);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int kxi = Tile<T, L, E, NCP>::template pos_in<fwd_last<L, V>()>(tc, e);
@@ -428,7 +541,7 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
     const T C1 = (T)1 + p.dtd2 * aLin, C2 = (T)1 - p.dtd2 * aLin;  // :214-215
     const cplx<T> nn = p.scale * v[e];
     // psi_new = (R + 3 dt/2 N)/C2, R' = C1 psi_new - dt/2 N (pf3d.cpp:476-478, as xpass_tile)
-    const cplx<T> r = (ORD == 2) ? cr[e] : ld_off<cplx<T>>(rb, o);
+    const cplx<T> r = X::PRE ? cr[X::PRE ? e : 0] : ld_off<cplx<T>>(rb, o);
     const T ic2 = recip(C2);
     cplx<T> ps = mk(ic2 * (r.x + (T)3 * p.dtd2 * nn.x), ic2 * (r.y + (T)3 * p.dtd2 * nn.y));
     cplx<T> rn = mk(C1 * ps.x - p.dtd2 * nn.x, C1 * ps.y - p.dtd2 * nn.y);
@@ -475,13 +588,12 @@ __global__ __launch_bounds__(X::NT) void k_xsplit_grp(const SplitArgs<typename X
 //   to standard: ky = k1 + RA k2 from radix RB over y2 with the twiddles, divided by RB (the split
 //   form's y2-space values are an unnormalised inverse); from standard: the inverse of it.
 //   perm: the carry's rows, an order of entries only.
+// kmul: k_y table of a standard-form input's d/dy, or nullptr.
 enum FormDir { FORM_TO_STD = 0, FORM_FROM_STD = 1, FORM_PERM_TO_STD = 2, FORM_PERM_FROM_STD = 3 };
-// YT: the type whose split_yc orders the stage rows (an FP32 array widened to FP64 keeps its order).
-template <typename T, int RB, typename YT = T>
+template <typename T, int RB>
 __global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny,
-                                              const cplx<T>* __restrict__ twy, int dir) {
+                                              const cplx<T>* __restrict__ twy, int dir, const T* __restrict__ kmul) {
   constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
-  constexpr int YC = split_yc<YT>(RB);
   __shared__ cplx<T> S[CAP + CAP / 16];
   auto at = [](int i) { return i + (i >> 4); };
   const int ra = ny / RB, rows = CAP / ny, tid = threadIdx.x;
@@ -490,7 +602,14 @@ __global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, i
   const int n = nr * ny;
   const cplx<T>* src = in + r0 * ny;
   cplx<T>* dst = out + r0 * ny;
-  for (int i = tid; i < n; i += 256) S[at(i)] = src[i];
+  for (int i = tid; i < n; i += 256) {
+    cplx<T> e = src[i];
+    if (kmul != nullptr) {  // i k_y of the spectral d/dy (pf3d.cpp:405)
+      const T k = kmul[i % ny];
+      e = mk(-k * e.y, k * e.x);
+    }
+    S[at(i)] = e;
+  }
   __syncthreads();
   if (dir == FORM_PERM_TO_STD || dir == FORM_PERM_FROM_STD) {
     for (int i = tid; i < n; i += 256) {
@@ -508,7 +627,7 @@ __global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, i
     if (i < nr * ra) {
 #pragma unroll
       for (int c = 0; c < RB; ++c)
-        w[it][c] = dir == FORM_TO_STD ? cmul(S[at(row * ny + split_pos(k1, c, RB, YC))], twy[k1 * c])
+        w[it][c] = dir == FORM_TO_STD ? cmul(S[at(row * ny + split_pos(k1, c, RB))], twy[k1 * c])
                                       : S[at(row * ny + k1 + ra * c)];
       if (dir == FORM_TO_STD) {
         dft<RB, -1>(w[it]);
@@ -528,7 +647,7 @@ __global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, i
     if (i < nr * ra) {
 #pragma unroll
       for (int c = 0; c < RB; ++c)
-        S[at(row * ny + (dir == FORM_TO_STD ? k1 + ra * c : split_pos(k1, c, RB, YC)))] = w[it][c];
+        S[at(row * ny + (dir == FORM_TO_STD ? k1 + ra * c : split_pos(k1, c, RB)))] = w[it][c];
     }
   }
   __syncthreads();

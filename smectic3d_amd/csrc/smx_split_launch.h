@@ -158,22 +158,21 @@ hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, hip
 }
 template <typename T, int RB>
 static void split_form_launch(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
-                              bool wide, hipStream_t st) {
+                              const T* kmul, hipStream_t st) {
   const int rows = 1024 / ny;
   const dim3 grid((unsigned)((nrows + rows - 1) / rows));
-  if (wide) SMX_LAUNCH((k_form<T, RB, float>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir);
-  else SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir);
+  SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul);
 }
 template <typename T>
-hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir, bool wide,
-                      hipStream_t st) {
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+                      const T* kmul, hipStream_t st) {
   const int ra = split_ra(ny);
   if (ra == 0) return hipErrorInvalidValue;
   switch (ny / ra) {
-    case 4: split_form_launch<T, 4>(in, out, nrows, ny, twy, dir, wide, st); break;
-    case 8: split_form_launch<T, 8>(in, out, nrows, ny, twy, dir, wide, st); break;
-    case 12: split_form_launch<T, 12>(in, out, nrows, ny, twy, dir, wide, st); break;
-    case 16: split_form_launch<T, 16>(in, out, nrows, ny, twy, dir, wide, st); break;
+    case 4: split_form_launch<T, 4>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 8: split_form_launch<T, 8>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 12: split_form_launch<T, 12>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 16: split_form_launch<T, 16>(in, out, nrows, ny, twy, dir, kmul, st); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

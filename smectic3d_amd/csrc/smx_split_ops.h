@@ -22,9 +22,9 @@ template <typename TI>
 hipError_t split_real(const cplx<TI>* a, double* out, const PParams<double>& p, hipStream_t st);
 bool split_real_fits(int ny, int nz);
 // Rows of a stage array (or, with the perm directions, of the carry) between the two forms, in place
-// allowed.  wide: FP64 rows that were widened from FP32 ones (which have another order).
+// allowed.  kmul: k_y table of the d/dy of a standard-form input, or nullptr.
 template <typename T>
-hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir, bool wide,
-                      hipStream_t st);
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+                      const T* kmul, hipStream_t st);
 
 }  // namespace smx

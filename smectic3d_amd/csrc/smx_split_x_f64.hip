@@ -5,4 +5,4 @@ template bool smx::split_x_fits<double>(int, int);
 template hipError_t smx::split_x<double>(const smx::SplitArgs<double>&, hipStream_t);
 template hipError_t smx::split_x_grp<double>(const smx::SplitArgs<double>*, int, const smx::PParams<double>&, hipStream_t);
 template hipError_t smx::split_form<double>(const smx::cplx<double>*, smx::cplx<double>*, int64_t, int, const smx::cplx<double>*,
-                                         int, bool, hipStream_t);
+                                         int, const double*, hipStream_t);
