@@ -1603,8 +1603,8 @@ static int autotune_T(smx_handle* h, int reps_in, PassSched* best) {
 // (one thread, which also takes the page faults) and 5.2 ms the other way.  Here a large field goes
 // through a ring of pinned slots: each worker thread moves its own chunks between its two slots and the
 // caller's array while the device copy of its other slot runs, 4.4, 3.6 and 4.0 ms.  Short of kRingToHost
-// (96^3, 7 MB: 0.43 -> 0.37 ms; 2 MB: the same) and kRingToDevice bytes (25 MB: the same; 57 MB: 2.2 ->
-// 1.8 ms) the runtime's copy is as fast.  One ring per process, used by one transfer at a time (another
+// (96^3, 7 MB: 0.48 -> 0.38 ms; 64^3, 2 MB: 0.17 -> 0.22) and kRingToDevice bytes (25 MB: the same; 57 MB:
+// 2.2 -> 1.8 ms) the runtime's copy is as fast.  One ring per process, used by one transfer at a time (another
 // one, from another thread, takes the runtime's copy); allocated by the first large transfer (2 ms), freed
 // with the last handle.
 constexpr size_t kRingSlot = 2u << 20;
@@ -1630,16 +1630,16 @@ static void ring_release() {
 }
 
 // Chunks w, w + nw, ... of one transfer through two slots, on the handle's stream.
-static hipError_t ring_worker(int device, hipStream_t st, char* dev, char* host, size_t bytes, bool to_host, int w,
-                              int nw, char* slots) {
+static hipError_t ring_worker(int device, hipStream_t st, char* dev, char* host, size_t bytes, size_t chunk,
+                              bool to_host, int w, int nw, char* slots) {
   hipError_t e = hipSetDevice(device);
   hipEvent_t ev[2] = {nullptr, nullptr};
   for (auto& x : ev)
     if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
-  const size_t nchunks = (bytes + kRingSlot - 1) / kRingSlot;
-  auto size = [&](size_t c) { return std::min(kRingSlot, bytes - c * kRingSlot); };
+  const size_t nchunks = (bytes + chunk - 1) / chunk;
+  auto size = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
   auto issue = [&](size_t c, int s) {
-    char* d = dev + c * kRingSlot;
+    char* d = dev + c * chunk;
     char* b = slots + s * kRingSlot;
     e = to_host ? hipMemcpyAsync(b, d, size(c), hipMemcpyDeviceToHost, st)
                 : hipMemcpyAsync(d, b, size(c), hipMemcpyHostToDevice, st);
@@ -1652,14 +1652,14 @@ static hipError_t ring_worker(int device, hipStream_t st, char* dev, char* host,
     for (size_t c = w; c < nchunks && e == hipSuccess; c += nw, s ^= 1) {
       e = hipEventSynchronize(ev[s]);
       if (e != hipSuccess) break;
-      std::memcpy(host + c * kRingSlot, slots + s * kRingSlot, size(c));
+      std::memcpy(host + c * chunk, slots + s * kRingSlot, size(c));
       if (c + 2 * nw < nchunks) issue(c + 2 * nw, s);
     }
   } else {
     for (size_t c = w; c < nchunks && e == hipSuccess; c += nw, s ^= 1) {
       if (c >= (size_t)w + 2 * nw) e = hipEventSynchronize(ev[s]);
       if (e != hipSuccess) break;
-      std::memcpy(slots + s * kRingSlot, host + c * kRingSlot, size(c));
+      std::memcpy(slots + s * kRingSlot, host + c * chunk, size(c));
       issue(c, s);
     }
   }
@@ -1687,10 +1687,14 @@ static int field_copy(smx_handle* h, void* dev, void* host, size_t bytes, bool t
     HIPCHK(hipStreamSynchronize(h->st));  // the host array is borrowed for the duration of the call only
     return SMX_OK;
   }
-  const int nw = (int)std::min<size_t>(kRingWorkers, 1 + bytes / (2 * kRingSlot));  // two chunks or more each
+  // Worker threads meet the caller's own (an OpenMP team that still spins behind its last loop): 96^3 and
+  // 128^3 into fresh arrays take 0.38 and 0.9-1.2 ms with one worker, 0.48 and 0.9-1.5 with four, so that
+  // each further one has 32 MB to move.
+  const size_t chunk = std::min(kRingSlot, (bytes / 8 + 4095) & ~(size_t)4095);
+  const int nw = (int)std::min<size_t>(kRingWorkers, 1 + bytes / (16 * kRingSlot));
   std::atomic<int> err{hipSuccess};
   auto work = [&](int w) {
-    const hipError_t e = ring_worker(h->cfg.device, h->st, (char*)dev, (char*)host, bytes, to_host, w, nw,
+    const hipError_t e = ring_worker(h->cfg.device, h->st, (char*)dev, (char*)host, bytes, chunk, to_host, w, nw,
                                      g_ring.buf + 2 * kRingSlot * w);
     if (e != hipSuccess) err = e;
   };
