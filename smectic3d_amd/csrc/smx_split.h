@@ -44,10 +44,11 @@ __host__ __device__ __forceinline__ int split_pos(int k1, int y2, int rb) {
 // y2 of a z tile: a whole piece or half of one (the tile's two parities of k1 share a line).  Whole pieces
 // where two blocks of the tile still fit a CU (192 x 96 x 384 FP64: 37.6 us with halves, 48.6 with one
 // block of whole pieces; 256^3 FP32: 34 with whole, 42 with halves), except in the shortest boxes, which
-// want more blocks (96^3 FP64 10.9 against 12.1 us, 128^3 FP32 11.7 against 10.2).
+// want more blocks (96^3 FP64 10.9 against 12.1 us, 128^3 FP32 11.7 against 10.2), and the shortest
+// lines, where half a piece would leave a wave mostly empty.
 template <typename T>
 constexpr int split_ny2(int l, int ra) {
-  return (l > 96 || ra == 4) && l * (2 * ra + 2) * 2 * (int)sizeof(T) <= 80 * 1024 && (ra <= 8 || sizeof(T) == 4) ? 4 : 2;
+  return (l > 96 || l <= 32 || ra == 4) && l * (2 * ra + 2) * 2 * (int)sizeof(T) <= 80 * 1024 && (ra <= 8 || sizeof(T) == 4) ? 4 : 2;
 }
 // Lanes that share one y line in the z kernel (pair_dft): two from radix 16 on, where one lane's 16
 // values make its loads the longest part (256^3 FP32: 40.6 -> 34.0 us; 192^3 FP32: 22.3 with one, 27.7).
@@ -70,10 +71,10 @@ constexpr bool split_pre() {
   return L <= 96 || (sizeof(T) == 4 && L <= 128);
 }
 // Columns per x tile: whole k1 groups of RB, rows of 128 bytes or more (96^3 FP32 with 12 columns 10.2
-// us, with 24 9.3; FP64 keeps 12, twice the blocks).
-template <typename T>
+// us, with 24 9.3; FP64 and long lines, whose blocks would pass 512 threads, keep 12).
+template <typename T, int L>
 constexpr int split_nc(int rb) {
-  return rb <= 8 ? 16 : (rb == 12 && sizeof(T) == 4 ? 24 : rb);
+  return rb <= 8 ? 16 : (rb == 12 && sizeof(T) == 4 && L <= 192 ? 24 : rb);
 }
 
 template <typename T>
@@ -426,7 +427,7 @@ struct RowFFT<LB, T, L, E, AD, SIGN, Radices<R, Rest...>> {
   }
 };
 
-template <typename T_, int L_, int RB_, int NC_ = split_nc<T_>(RB_), int V_ = split_v<L_>(),
+template <typename T_, int L_, int RB_, int NC_ = split_nc<T_, L_>(RB_), int V_ = split_v<L_>(),
           bool PRE_ = split_pre<T_, L_>()>
 struct XS {
   using T = T_;
@@ -435,40 +436,28 @@ struct XS {
   static constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NC * TPC, NCP = NC + 1, NK = NC / RB;
   using AD = RowAddr<NCP>;
   static constexpr bool fits =
-      NT <= 1024 && (size_t)(L * (NCP + 1) + NC) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
+      NT <= 1024 && (size_t)L * (NCP + 1) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
 };
 
-// The x tile's part of the y transform on its rows: y2 -> k2 (twiddles, then radix RB) and back.
-// Lanes run down the rows; TWY: w_ny^{y2 k1} of the tile's columns.
-template <typename X>
+// The x tile's part of the y transform on its rows, radix RB between y2 and k2 (SIGN -1: y2 -> k2).
+// Lanes run down the rows.  The twiddles w_ny^{y2 k1} are one factor per column, so a thread applies
+// its column's in registers as it loads (and, conjugated, as it stores) the stage rows: taken here they
+// were 15 LDS reads per row each way (256^3 FP32 47.5 -> 45.9 us, 64^3 4.8 -> 4.4).
+template <typename X, int SIGN>
 struct XRow {
   using T = typename X::T;
   using AD = typename X::AD;
   static constexpr int L = X::L, RB = X::RB, NK = X::NK, NT = X::NT;
-  __device__ static __forceinline__ void fwd(cplx<T>* S, const cplx<T>* TWY, int tid) {
-    for (int i = tid; i < L * NK; i += NT) {
-      const int g = i / L, row = i - g * L;
-      cplx<T> w[RB];
-      cplx<T>* s = &S[AD::at(row, g * RB)];
-      w[0] = s[0];
-#pragma unroll
-      for (int c = 1; c < RB; ++c) w[c] = cmul(s[c], TWY[g * RB + c]);
-      dft<RB, -1>(w);
-#pragma unroll
-      for (int c = 0; c < RB; ++c) s[c] = w[c];
-    }
-  }
-  __device__ static __forceinline__ void inv(cplx<T>* S, const cplx<T>* TWY, int tid) {
+  __device__ static __forceinline__ void run(cplx<T>* S, int tid) {
     for (int i = tid; i < L * NK; i += NT) {
       const int g = i / L, row = i - g * L;
       cplx<T> w[RB];
       cplx<T>* s = &S[AD::at(row, g * RB)];
 #pragma unroll
       for (int c = 0; c < RB; ++c) w[c] = s[c];
-      dft<RB, +1>(w);
-      s[0] = w[0];
+      dft<RB, SIGN>(w);
 #pragma unroll
-      for (int c = 1; c < RB; ++c) s[c] = cmul(w[c], conjg(TWY[g * RB + c]));
+      for (int c = 0; c < RB; ++c) s[c] = w[c];
     }
   }
 };
@@ -498,7 +487,6 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
   __shared__ cplx<T> S[L * NCP];
   __shared__ cplx<T> TW[L];
   __shared__ T KX[L];
-  __shared__ cplx<T> TWY[NC];  // w_ny^{y2 k1} of the tile's columns
   const int tid = threadIdx.x, col = tid % NC, tc = tid / NC;
   const int ra = p.ny / RB;
   const int ky = bx * NK + col / RB + ra * (col % RB);
@@ -521,15 +509,15 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
   // the tables behind the tile's loads, so that their latencies overlap
   const cplx<T>* twl = tw_lds<L, NT>(TW, p.twx, tid);
   for (int i = tid; i < L; i += NT) KX[i] = p.kx[i];
-  for (int i = tid; i < NC; i += NT) TWY[i] = twy[(bx * NK + i / RB) * (i % RB)];
+  const cplx<T> tw = twy[(bx * NK + col / RB) * (col % RB)];  // w_ny^{y2 k1}
   const T kyv = p.ky[ky], kzv = p.kz[kz];
   // FP64 mean mode (mixed path): the block owning k = 0 sums the z kernel's partials.
   double nsum = 0.0;
   const bool owner0 = (p.partial != nullptr) && kz == 0 && bx == 0;
   if (owner0) nsum = xs_partial_sum<X>(p, S, tid);
-  auto fwd_row = [&]() { XRow<X>::fwd(S, TWY, tid); };
-  auto inv_row = [&]() { XRow<X>::inv(S, TWY, tid); };
-  RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(v, S, col, tc, twl, fwd_row);
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = cmul(v[e], tw);
+  RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(v, S, col, tc, twl, [&]() { XRow<X, -1>::run(S, tid); });
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const int kxi = Tile<T, L, E, NCP>::template pos_in<fwd_last<L, V>()>(tc, e);
@@ -556,10 +544,11 @@ __device__ __forceinline__ void xsplit_tile(cplx<T>* a, cplx<T>* __restrict__ rb
     st_off(rb, o, rn);
     v[e] = ps;
   }
-  RowFFT<true, T, L, E, AD, +1, typename PlanV<L, V>::Inv>::run(v, S, col, tc, twl, inv_row);
+  RowFFT<true, T, L, E, AD, +1, typename PlanV<L, V>::Inv>::run(v, S, col, tc, twl, [&]() { XRow<X, +1>::run(S, tid); });
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    st_off(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<inv_last<L, V>()>(tc, e) * rowb + aofs, v[e]);
+    st_off(src, (uint32_t)Tile<T, L, E, NCP>::template pos_in<inv_last<L, V>()>(tc, e) * rowb + aofs,
+           cmul(v[e], conjg(tw)));
 }
 // Tile of linear block b of g column groups a plane: with one k1 per tile, the two tiles that share
 // the stage rows' lines are neighbours on one XCD (whole groups of 16 blocks; the rest in order).
