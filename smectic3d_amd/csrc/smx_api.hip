@@ -371,6 +371,7 @@ static int bootstrap(smx_handle* h) {
 // Kernel slots of one step, in launch order.
 static const char* kSlotNamesP[] = {"k_ypass_inv", "k_zpass_nl", "k_ypass_fwd", "k_xpass_step"};
 static const char* kSlotNamesS[] = {"k_zsplit", "k_xsplit"};
+static const char* kSlotNamesSA[] = {"k_zsplit_force", "k_xsplit_stokes", "k_zsplit_advnl", "k_xsplit_adv"};
 static const char* kSlotNamesN[] = {"k_dct_ypass_inv", "k_dct_zpass_nl", "k_dct_ypass_fwd", "k_dct_xpass_step"};
 static const char* kSlotNamesA[] = {"k_ypass_inv_dy", "k_ypass_inv_psi", "k_ypass_inv_dx", "k_ypass_inv_sh",
                                     "k_zpass_force", "k_ypass_fwd_s0", "k_ypass_fwd_s1", "k_ypass_fwd_s2",
@@ -381,9 +382,9 @@ static const char* kSlotNamesNA[] = {"k_dct_ypass_inv_dy", "k_dct_ypass_inv_psi"
                                      "k_dct_ypass_fwd_s1", "k_dct_ypass_fwd_s2", "k_dctx_stokes",
                                      "k_dct_ypass_inv_u0", "k_dct_ypass_inv_u1", "k_dct_ypass_inv_u2",
                                      "k_dctz_advnl", "k_dct_ypass_fwd_n", "k_dctx_adv"};
-static int num_slots(const smx_handle* h) { return h->cfg.advect ? 15 : (h->split ? 2 : 4); }
+static int num_slots(const smx_handle* h) { return h->cfg.advect ? (h->split ? 4 : 15) : (h->split ? 2 : 4); }
 static const char* slot_name(const smx_handle* h, int s) {
-  if (h->cfg.advect) return h->neumann ? kSlotNamesNA[s] : kSlotNamesA[s];
+  if (h->cfg.advect) return h->neumann ? kSlotNamesNA[s] : (h->split ? kSlotNamesSA[s] : kSlotNamesA[s]);
   return h->neumann ? kSlotNamesN[s] : (h->split ? kSlotNamesS[s] : kSlotNamesP[s]);
 }
 
@@ -510,6 +511,23 @@ static int step_advect(smx_handle* h, const AParams<T>& ap, hipEvent_t* ev) {
 
 template <typename T>
 static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
+  if (h->cfg.advect && h->split) {  // four launches (smx_split_adv.h)
+    SlotTimer tm(ev);
+    SplitAdvArgs<T> sa{(cplx<T>*)h->A,  (cplx<T>*)h->Ax, (cplx<T>*)h->By, (cplx<T>*)h->As, (cplx<T>*)h->S1,
+                       (cplx<T>*)h->S2, (cplx<T>*)h->R,  tables<T>(h).twy, aparams<T>(h, h->fp32)};
+    sa.ap.p.partial = p.partial;
+    sa.ap.p.npartial = split_z_blocks<T>(p);
+    tm.arm(0);
+    hipError_t e = split_adv_force<T>(sa, h->st);
+    tm.arm(1);
+    if (e == hipSuccess) e = split_adv_stokes<T>(sa, h->st);
+    tm.arm(2);
+    if (e == hipSuccess) e = split_adv_advnl<T>(sa, h->st);
+    tm.arm(3);
+    if (e == hipSuccess) e = split_adv_update<T>(sa, h->st);
+    if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("advected step: ") + hipGetErrorString(e));
+    return SMX_OK;
+  }
   if (h->cfg.advect) {
     AParams<T> ap = aparams<T>(h, h->fp32);
     ap.p.partial = p.partial;  // the caller's partial-sum region (the handle's, or the device scratch)
@@ -570,6 +588,10 @@ static bool use_split(const smx_handle* h) { return h->auto_path && h->split_ok;
 template <typename T>
 static int ensure_form_T(smx_handle* h, bool split) {
   cplx<T>*A = (cplx<T>*)h->A, *R = (cplx<T>*)h->R;
+  if (h->cfg.advect) {  // in the split form d_y psi is carried too (a work array in the standard one)
+    if (split) CHK(form_rows<T>(h, A, (cplx<T>*)h->By, FORM_FROM_STD, tables<T>(h).ky));
+    for (void* x : {h->Ax, h->As}) CHK(form_rows<T>(h, (cplx<T>*)x, (cplx<T>*)x, split ? FORM_FROM_STD : FORM_TO_STD));
+  }
   CHK(form_rows<T>(h, A, A, split ? FORM_FROM_STD : FORM_TO_STD));
   CHK(form_rows<T>(h, R, R, split ? FORM_PERM_FROM_STD : FORM_PERM_TO_STD));
   h->split = split;
@@ -1788,11 +1810,12 @@ static int64_t split_layout(const smx_handle* h) {
   return ra ? ra * 65536 + kSplitYC : 0;
 }
 
-static std::vector<void*> carried_arrays(smx_handle* h) {
+static std::vector<void*> carried_arrays(smx_handle* h, bool split) {
   std::vector<void*> v = {h->A, h->R};
   if (h->cfg.advect) {
     v.push_back(h->Ax);
     v.push_back(h->As);
+    if (split) v.push_back(h->By);
   }
   return v;
 }
@@ -1864,6 +1887,9 @@ int smx_create(const smx_config* cfg, smx_handle** out) {
   if (!h->neumann && !c.advect)
     h->split_ok = h->fp32 ? split_z_fits<float>(c.ny, c.nz) && split_x_fits<float>(c.nx, c.ny)
                           : split_z_fits<double>(c.ny, c.nz) && split_x_fits<double>(c.nx, c.ny);
+  else if (!h->neumann)
+    h->split_ok = h->fp32 ? split_adv_fits_z<float>(c.ny, c.nz) && split_adv_fits_x<float>(c.nx, c.ny)
+                          : split_adv_fits_z<double>(c.ny, c.nz) && split_adv_fits_x<double>(c.nx, c.ny);
   if (h->split_ok) h->split_ok = split_real_fits(c.ny, c.nz);
   if (h->neumann) {  // the default widths; the x pass's tile must divide ny (else 16 columns)
     const int ncd = h->fp32 ? neumann_nc<float>() : neumann_nc<double>();
@@ -2005,7 +2031,7 @@ int smx_save_checkpoint(smx_handle* h, const char* path) {
   if (!h || !path) return fail(SMX_ERR_INVALID, "null argument");
   if (!h->has_state) return fail(SMX_ERR_STATE, "no state: call smx_set_psi first");
   HIPCHK(hipSetDevice(h->cfg.device));
-  const std::vector<void*> arrs = carried_arrays(h);
+  const std::vector<void*> arrs = carried_arrays(h, h->split);
   const size_t abytes = h->wbytes * (size_t)h->nspec;
   CkptHeader hd;
   std::memset(&hd, 0, sizeof(hd));
@@ -2052,7 +2078,6 @@ int smx_load_checkpoint(smx_handle* h, const char* path) {
   FILE* f = std::fopen(path, "rb");
   if (!f) return fail(SMX_ERR_INVALID, std::string("cannot open ") + path);
   CkptHeader hd;
-  const std::vector<void*> arrs = carried_arrays(h);
   const size_t abytes = h->wbytes * (size_t)h->nspec;
   auto bad = [&](const std::string& why) {
     std::fclose(f);
@@ -2062,6 +2087,7 @@ int smx_load_checkpoint(smx_handle* h, const char* path) {
       (std::memcmp(hd.magic, "SMXCKPT1", 8) != 0 && std::memcmp(hd.magic, "SMXCKPT2", 8) != 0))
     return bad("not a checkpoint");
   const bool in_split = hd.magic[7] == '2';
+  const std::vector<void*> arrs = carried_arrays(h, in_split);
   if (hd.abi_version != SMX_ABI_VERSION || hd.narrays != (int32_t)arrs.size() || hd.wbytes != (int64_t)h->wbytes ||
       hd.nspec != h->nspec || !same_operator(hd.cfg, h->cfg))
     return bad("checkpoint of a different grid, precision or operator");
@@ -2809,7 +2835,9 @@ int smx_profile_step(smx_handle* h, int64_t nsteps, int max_slots, int* nslots, 
   CHK(h->fp32 ? profile_T<float>(h, nsteps, acc) : profile_T<double>(h, nsteps, acc));
   const double sc = (double)h->wbytes * (double)h->nspec;  // bytes of one spectral-stage array
   std::vector<double> bytes;
-  if (h->cfg.advect)  // reads + writes of spectral-stage arrays per launch
+  if (h->cfg.advect && h->split)  // reads + writes of spectral-stage arrays per launch
+    bytes = {7 * sc, 6 * sc, 7 * sc, 7 * sc};
+  else if (h->cfg.advect)
     bytes = {2 * sc, 2 * sc, 2 * sc, 2 * sc, 7 * sc, 2 * sc, 2 * sc, 2 * sc,
              6 * sc, 2 * sc, 2 * sc, 2 * sc, 7 * sc, 2 * sc, 6 * sc};
   else if (h->split)

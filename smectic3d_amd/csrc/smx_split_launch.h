@@ -40,6 +40,12 @@ hipError_t split_x_dispatch(int nx, int rb, F&& f) {
   return hipErrorInvalidValue;
 }
 
+// Blocks that project the carry: 8 pairs' entries per thread.
+template <typename Z, typename T>
+static int split_nproj(const PParams<T>& p) {
+  return (int)((2 * p.nxy + 8 * Z::NT - 1) / (8 * Z::NT));
+}
+
 #ifdef SMX_SPLIT_Z
 template <typename T>
 bool split_z_fits(int ny, int nz) {
@@ -58,11 +64,6 @@ int split_z_blocks(const PParams<T>& p) {
     return hipSuccess;
   });
   return n;
-}
-// Blocks that project the carry: 8 pairs' entries per thread.
-template <typename Z, typename T>
-static int split_nproj(const PParams<T>& p) {
-  return (int)((2 * p.nxy + 8 * Z::NT - 1) / (8 * Z::NT));
 }
 template <typename T>
 hipError_t split_z(const SplitArgs<T>& s, int op, hipStream_t st) {
@@ -90,6 +91,81 @@ hipError_t split_z_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, int
       const int np = split_nproj<Z>(p);
       SMX_LAUNCH((k_zsplit_grp<Z>), dim3((unsigned)(np + split_z_blocks(p)), (unsigned)nbox), dim3(Z::NT), 0, st,
                  g, op, np);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_ADV_Z
+template <typename T>
+bool split_adv_fits_z(int ny, int nz) {
+  const int ra = split_ra(ny);
+  return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
+           using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
+           return zsa_fits<Z>() && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+hipError_t split_adv_force(const SplitAdvArgs<T>& s, hipStream_t st) {
+  const PParams<T>& p = s.ap.p;
+  return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!zsa_fits<Z>()) {
+      return hipErrorInvalidValue;
+    } else {
+      const int np = split_nproj<Z>(p), nb = p.nx * (p.ny / Z::RA / Z::NY2);
+      SMX_LAUNCH((k_zsplit_force<Z>), dim3((unsigned)(np + nb)), dim3(Z::NT), 0, st, s, np);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename T>
+hipError_t split_adv_advnl(const SplitAdvArgs<T>& s, hipStream_t st) {
+  const PParams<T>& p = s.ap.p;
+  return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!zsa_fits<Z>()) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_zsplit_advnl<Z>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, s);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_ADV_X
+template <typename T>
+bool split_adv_fits_x(int nx, int ny) {
+  const int ra = split_ra(ny);
+  return ra != 0 && split_x_dispatch(nx, ny / ra, [&](auto l, auto r) -> hipError_t {
+           using X = XS<T, decltype(l)::value, decltype(r)::value>;
+           return xsa_fits<X>() && ny % X::NC == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+hipError_t split_adv_stokes(const SplitAdvArgs<T>& s, hipStream_t st) {
+  const PParams<T>& p = s.ap.p;
+  return split_x_dispatch(p.nx, p.ny / split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    using X = XS<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!xsa_fits<X>()) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_xsplit_stokes<X>), dim3((unsigned)(p.ny / X::NC * p.nzh)), dim3(X::NT), 0, st, s);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename T>
+hipError_t split_adv_update(const SplitAdvArgs<T>& s, hipStream_t st) {
+  const PParams<T>& p = s.ap.p;
+  return split_x_dispatch(p.nx, p.ny / split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    using X = XS<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!xsa_fits<X>()) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_xsplit_adv<X>), dim3((unsigned)(p.ny / X::NC * p.nzh)), dim3(X::NT), 0, st, s);
       return hipGetLastError();
     }
   });

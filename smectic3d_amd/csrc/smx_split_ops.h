@@ -1,7 +1,7 @@
 // smx_split_ops.h -- host launchers of the two-launch step (smx_split.h).  The definitions are in
 // smx_split_launch.h, instantiated per precision in smx_split_z_*.hip and smx_split_x_*.hip.
 #pragma once
-#include "smx_split.h"
+#include "smx_split_adv.h"
 
 namespace smx {
 
@@ -20,6 +20,13 @@ template <typename T> hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, co
 // FP64 real field of a split-form stage array of type TI.
 template <typename TI>
 hipError_t split_real(const cplx<TI>* a, double* out, const PParams<double>& p, hipStream_t st);
+// The advected step's four launches (smx_split_adv.h).
+template <typename T> bool split_adv_fits_z(int ny, int nz);
+template <typename T> bool split_adv_fits_x(int nx, int ny);
+template <typename T> hipError_t split_adv_force(const SplitAdvArgs<T>& s, hipStream_t st);
+template <typename T> hipError_t split_adv_stokes(const SplitAdvArgs<T>& s, hipStream_t st);
+template <typename T> hipError_t split_adv_advnl(const SplitAdvArgs<T>& s, hipStream_t st);
+template <typename T> hipError_t split_adv_update(const SplitAdvArgs<T>& s, hipStream_t st);
 bool split_real_fits(int ny, int nz);
 // Rows of a stage array (or, with the perm directions, of the carry) between the two forms, in place
 // allowed.  kmul: k_y table of the d/dy of a standard-form input, or nullptr.
