@@ -368,11 +368,20 @@ static int bootstrap(smx_handle* h) {
   return SMX_OK;
 }
 
+// The default schedule.  Neumann passes have their own widths; the x pass's tile must divide ny (else 16
+// columns).
+static PassSched default_sched(const smx_handle* h, int slot) {
+  if (!h->neumann) return PassSched{};
+  const int nc = h->fp32 ? neumann_nc<float>() : neumann_nc<double>();
+  return PassSched{slot == SLOT_X && h->cfg.ny % nc != 0 ? 16 : nc, 0};
+}
+
 // Kernel slots of one step, in launch order.
 static const char* kSlotNamesP[] = {"k_ypass_inv", "k_zpass_nl", "k_ypass_fwd", "k_xpass_step"};
 static const char* kSlotNamesS[] = {"k_zsplit", "k_xsplit"};
 static const char* kSlotNamesSA[] = {"k_zsplit_force", "k_xsplit_stokes", "k_zsplit_advnl", "k_xsplit_adv"};
 static const char* kSlotNamesN[] = {"k_dct_ypass_inv", "k_dct_zpass_nl", "k_dct_ypass_fwd", "k_dct_xpass_step"};
+static const char* kSlotNamesNS[] = {"k_nsplit_z", "k_nsplit_x"};
 static const char* kSlotNamesA[] = {"k_ypass_inv_dy", "k_ypass_inv_psi", "k_ypass_inv_dx", "k_ypass_inv_sh",
                                     "k_zpass_force", "k_ypass_fwd_s0", "k_ypass_fwd_s1", "k_ypass_fwd_s2",
                                     "k_xpass_stokes", "k_ypass_inv_u0", "k_ypass_inv_u1", "k_ypass_inv_u2",
@@ -385,7 +394,8 @@ static const char* kSlotNamesNA[] = {"k_dct_ypass_inv_dy", "k_dct_ypass_inv_psi"
 static int num_slots(const smx_handle* h) { return h->cfg.advect ? (h->split ? 4 : 15) : (h->split ? 2 : 4); }
 static const char* slot_name(const smx_handle* h, int s) {
   if (h->cfg.advect) return h->neumann ? kSlotNamesNA[s] : (h->split ? kSlotNamesSA[s] : kSlotNamesA[s]);
-  return h->neumann ? kSlotNamesN[s] : (h->split ? kSlotNamesS[s] : kSlotNamesP[s]);
+  if (h->neumann) return h->split ? kSlotNamesNS[s] : kSlotNamesN[s];
+  return h->split ? kSlotNamesS[s] : kSlotNamesP[s];
 }
 
 // Per-kernel timing of a step chain: slot k's kernel is launched with the event pair
@@ -536,6 +546,17 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
     return step_advect<T>(h, ap, ev);
   }
   SlotTimer tm(ev);
+  if (h->neumann && h->split) {  // the two-launch step (smx_split_neu.h)
+    const DevTables<T>& t = tables<T>(h);
+    SplitNeuArgs<T> sa{(cplx<T>*)h->A, (cplx<T>*)h->R, t.twy, t.qtwx, t.qtwy, t.qtwz, p};
+    sa.p.npartial = nsplit_z_blocks<T>(p);
+    tm.arm(0);
+    hipError_t e = nsplit_z<T>(sa, h->st);
+    tm.arm(1);
+    if (e == hipSuccess) e = nsplit_x<T>(sa, h->st);
+    if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("two-launch step: ") + hipGetErrorString(e));
+    return SMX_OK;
+  }
   if (h->neumann) {  // the handle's tile widths; the x pass sums one FP64 partial per z tile
     PParams<T> q = p;
     q.npartial = NeumannOps<T>::zpass_blocks(p, h->sched[SLOT_Z].nc);
@@ -574,11 +595,19 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
   return SMX_OK;  // the x pass projects the self-conjugate planes of R itself
 }
 
-// ---- the two forms of a periodic state (smx_split.h) ----
+// ---- the two forms of a state (smx_split.h, smx_split_neu.h) ----
 // Rows of a stage array or carry from one form to the other on the handle's stream, in place allowed.
 template <typename T>
 static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
   const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
+  if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
+  return SMX_OK;
+}
+// The same for a Neumann box, out of place.
+template <typename TI, typename TO>
+static int nform_rows(smx_handle* h, const void* in, void* out, int dir) {
+  const hipError_t e = nsplit_form<TI, TO>((const TI*)in, (TO*)out, h->cfg.nx, h->cfg.ny, h->cfg.nz, h->t64.twy,
+                                           h->t64.qtwy, dir, h->st);
   if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
   return SMX_OK;
 }
@@ -588,6 +617,16 @@ static bool use_split(const smx_handle* h) { return h->auto_path && h->split_ok;
 template <typename T>
 static int ensure_form_T(smx_handle* h, bool split) {
   cplx<T>*A = (cplx<T>*)h->A, *R = (cplx<T>*)h->R;
+  if (h->neumann) {  // through real_io, which holds nothing between calls
+    for (void* x : {h->A, h->R}) {
+      const bool perm = x == h->R;
+      HIPCHK(hipMemcpyAsync(h->real_io, x, sizeof(T) * (size_t)h->N, hipMemcpyDeviceToDevice, h->st));
+      CHK((nform_rows<T, T>(h, h->real_io, x, split ? (perm ? FORM_PERM_FROM_STD : FORM_FROM_STD)
+                                                    : (perm ? FORM_PERM_TO_STD : FORM_TO_STD))));
+    }
+    h->split = split;
+    return SMX_OK;
+  }
   if (h->cfg.advect) {  // in the split form d_y psi is carried too (a work array in the standard one)
     if (split) CHK(form_rows<T>(h, A, (cplx<T>*)h->By, FORM_FROM_STD, tables<T>(h).ky));
     for (void* x : {h->Ax, h->As}) CHK(form_rows<T>(h, (cplx<T>*)x, (cplx<T>*)x, split ? FORM_FROM_STD : FORM_TO_STD));
@@ -609,6 +648,9 @@ static int ensure_form(smx_handle* h, bool split) {
 // split: the stage buffer holds the split form; the copy is in the standard one.
 static int stage_to_f64(smx_handle* h, const void* stage, void* dst, bool split) {
   const int64_t ncomp = h->neumann ? h->nspec : 2 * h->nspec;  // real components
+  if (h->neumann && split)
+    return h->fp32 ? nform_rows<float, double>(h, stage, dst, FORM_TO_STD)
+                   : nform_rows<double, double>(h, stage, dst, FORM_TO_STD);
   if (h->fp32) {
     hipLaunchKernelGGL(k_f32_to_f64, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, (const float*)stage,
                        (double*)dst, ncomp);
@@ -634,7 +676,10 @@ static int state_to_d1(smx_handle* h) { return stage_to_f64(h, h->A, h->D1, h->s
 static int c2r_stage(smx_handle* h, const void* stage, bool split, double* out) {
   PParams<double> p = params<double>(h, false);
   if (split) {  // one kernel: y and z inverse of the split form, FP32 widened as it is read
-    const hipError_t e = h->fp32 ? split_real<float>((const cplx<float>*)stage, out, p, h->st)
+    const hipError_t e =
+        h->neumann ? (h->fp32 ? nsplit_real<float>((const cplx<float>*)stage, out, p, h->t64.qtwz, h->st)
+                              : nsplit_real<double>((const cplx<double>*)stage, out, p, h->t64.qtwz, h->st))
+        : h->fp32 ? split_real<float>((const cplx<float>*)stage, out, p, h->st)
                                  : split_real<double>((const cplx<double>*)stage, out, p, h->st);
     if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("real field: ") + hipGetErrorString(e));
     return SMX_OK;
@@ -1540,7 +1585,10 @@ static int autotune_T(smx_handle* h, int reps_in, PassSched* best) {
   T* wr = (T*)h->D2;
   auto reset = [&]() -> int {
     if (h->has_state) {
-      if (h->split) {
+      if (h->split && h->neumann) {
+        CHK((nform_rows<T, T>(h, h->A, wa, FORM_TO_STD)));
+        CHK((nform_rows<T, T>(h, h->R, wr, FORM_PERM_TO_STD)));
+      } else if (h->split) {
         CHK(form_rows<T>(h, (const cplx<T>*)h->A, (cplx<T>*)wa, FORM_TO_STD));
         CHK(form_rows<T>(h, (const cplx<T>*)h->R, (cplx<T>*)wr, FORM_PERM_TO_STD));
       } else {
@@ -1806,7 +1854,7 @@ static bool same_operator(const smx_config& a, const smx_config& b) {
 }
 
 static int64_t split_layout(const smx_handle* h) {
-  const int ra = split_ra(h->cfg.ny);
+  const int ra = h->neumann ? nsplit_ra(h->cfg.ny, h->cfg.nx) : split_ra(h->cfg.ny);
   return ra ? ra * 65536 + kSplitYC : 0;
 }
 
@@ -1887,15 +1935,18 @@ int smx_create(const smx_config* cfg, smx_handle** out) {
   if (!h->neumann && !c.advect)
     h->split_ok = h->fp32 ? split_z_fits<float>(c.ny, c.nz) && split_x_fits<float>(c.nx, c.ny)
                           : split_z_fits<double>(c.ny, c.nz) && split_x_fits<double>(c.nx, c.ny);
+  else if (h->neumann && !c.advect)
+    h->split_ok = (h->fp32 ? nsplit_z_fits<float>(c.nx, c.ny, c.nz) && nsplit_x_fits<float>(c.nx, c.ny)
+                           : nsplit_z_fits<double>(c.nx, c.ny, c.nz) && nsplit_x_fits<double>(c.nx, c.ny)) &&
+                  nsplit_real_fits(c.nx, c.ny, c.nz) &&
+                  // FP64 256 x 256 x 384: one block of 512 threads a CU in either kernel, 405 us a step and 387 in
+                  // four passes (256 x 256 x 512, 1024 threads in z: 513 and 581; 192 x 256 x 384: 265 and 288)
+                  !(!h->fp32 && c.nx == 256 && c.ny == 256 && c.nz == 384);
   else if (!h->neumann)
     h->split_ok = h->fp32 ? split_adv_fits_z<float>(c.ny, c.nz) && split_adv_fits_x<float>(c.nx, c.ny)
                           : split_adv_fits_z<double>(c.ny, c.nz) && split_adv_fits_x<double>(c.nx, c.ny);
-  if (h->split_ok) h->split_ok = split_real_fits(c.ny, c.nz);
-  if (h->neumann) {  // the default widths; the x pass's tile must divide ny (else 16 columns)
-    const int ncd = h->fp32 ? neumann_nc<float>() : neumann_nc<double>();
-    for (PassSched& ps : h->sched) ps = PassSched{ncd, 0};
-    if (c.ny % ncd != 0) h->sched[SLOT_X].nc = 16;
-  }
+  if (h->split_ok && !h->neumann) h->split_ok = split_real_fits(c.ny, c.nz);
+  for (int k = 0; k < NSLOTS; ++k) h->sched[k] = default_sched(h, k);
   auto bail = [&](int code) {
     smx_destroy(h);
     return code;
@@ -2248,9 +2299,9 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   const int ns = surf_nsplit(h->neumann, h->cfg.nx, h->cfg.nz);
   // An FP64 state is its own x stage, and an FP32 Neumann stage is read as it is (widened on
   // load); a periodic FP32 stage is copied to FP64 and projected (stage_to_f64) first.
-  // An FP64 split-form state is brought to the standard form there.
-  const bool f32in = h->fp32 && h->neumann, w0copy = !h->neumann && (h->fp32 || h->split);
-  const bool w0room = !h->neumann && (h->fp32 || h->split_ok);
+  // A split-form state is brought to the standard form there.
+  const bool f32in = h->fp32 && h->neumann && !h->split, w0copy = h->split || (!h->neumann && h->fp32);
+  const bool w0room = h->split_ok || (!h->neumann && h->fp32);
   // real psi, the FP64 x stage copy, the field values at each column's evaluation index (ns
   // parts per field), the z evaluation's trigonometric table, and the crossing and evaluation
   // indices of each column
@@ -2490,7 +2541,7 @@ int smx_adjoint_info(const smx_handle* h, int64_t* resident_steps, int64_t* reco
 int smx_get_schedule(const smx_handle* h, smx_schedule* s) {
   if (!h || !s) return fail(SMX_ERR_INVALID, "null argument");
   for (int k = 0; k < NSLOTS; ++k) {
-    const PassSched ps = use_split(h) ? PassSched{} : h->sched[k];
+    const PassSched ps = use_split(h) ? default_sched(h, k) : h->sched[k];
     s->nc[k] = ps.nc;
     s->variant[k] = ps.v;
   }
@@ -2511,7 +2562,8 @@ int smx_set_schedule(smx_handle* h, const smx_schedule* s) {
   h->auto_path = true;  // the default schedule leaves the choice of the path to the library
   for (int k = 0; k < NSLOTS; ++k) {
     h->sched[k] = c[k];
-    if (c[k].nc != kNC || c[k].v != 0) h->auto_path = false;
+    const PassSched d = default_sched(h, k);
+    if (c[k].nc != d.nc || c[k].v != d.v) h->auto_path = false;
   }
   return SMX_OK;
 }

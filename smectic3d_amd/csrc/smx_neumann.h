@@ -2,7 +2,8 @@
 // (cosFFT/mesabi/cosNoAdvMorph.cpp:483-530).
 //
 // Every stage array is real, layout [kz][x or kx][y or ky] (y fastest), N entries.
-// A step is four in-place launches on the stage buffer A plus the carry R:
+// A step of a grid without the two-launch form (smx_split_neu.h), or with a schedule of its own, is four
+// in-place launches on the stage buffer A plus the carry R:
 //   k_dct_ypass<inv>   (x,ky,kz) -> (x,y,kz)    DCT-III along y
 //   k_dct_zpass        (x,y,kz)  -> (x,y,kz)    DCT-III along z, N(psi), DCT-II along z
 //   k_dct_ypass<fwd>   (x,y,kz)  -> (x,ky,kz)   DCT-II along y

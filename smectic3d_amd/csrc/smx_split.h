@@ -171,10 +171,11 @@ __device__ __forceinline__ void rot_all(cplx<T>* w) {
     rot_all<R, SIGN, Y + 1, N>(w);
   }
 }
-// Radix 2 H of one line held by two adjacent lanes: even and odd inputs (SIGN > 0: lane parity = k1
-// parity in, half of the y1 out) or the other way round (SIGN < 0).  The pair and its neighbours load
-// and store whole lines' halves together, and every thread of the block has a part of the work.
-template <int H, int SIGN, typename T>
+// Radix 2 H of one line held by two adjacent lanes: even and odd inputs in, the two halves of the outputs
+// out, or (HALVES) the other way round.  Here even and odd k1, and halves of the y1, so SIGN decides.  The
+// pair and its neighbours load and store whole lines' halves together, and every thread of the block has
+// a part of the work.
+template <int H, int SIGN, bool HALVES = (SIGN < 0), typename T>
 __device__ __forceinline__ void pair_dft(cplx<T>* w, int lo) {
   const T sgn = lo ? (T)-1 : (T)1;
   auto cross = [&]() {
@@ -184,14 +185,14 @@ __device__ __forceinline__ void pair_dft(cplx<T>* w, int lo) {
       w[y] = mk(o.x + sgn * w[y].x, o.y + sgn * w[y].y);
     }
   };
-  if constexpr (SIGN > 0) {
-    dft<H, +1>(w);
-    if (lo) rot_all<2 * H, +1, 0, H>(w);
+  if constexpr (!HALVES) {
+    dft<H, SIGN>(w);
+    if (lo) rot_all<2 * H, SIGN, 0, H>(w);
     cross();
   } else {
     cross();
-    if (lo) rot_all<2 * H, -1, 0, H>(w);
-    dft<H, -1>(w);
+    if (lo) rot_all<2 * H, SIGN, 0, H>(w);
+    dft<H, SIGN>(w);
   }
 }
 

@@ -255,4 +255,95 @@ hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, co
 }
 #endif
 
+#ifdef SMX_SPLIT_NEU_Z
+template <typename T>
+bool nsplit_z_fits(int nx, int ny, int nz) {
+  const int ra = nsplit_ra(ny, nx);
+  return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
+           using Z = NZ<T, decltype(l)::value, decltype(r)::value>;
+           return Z::fits && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+int nsplit_z_blocks(const PParams<T>& p) {
+  const int ra = nsplit_ra(p.ny, p.nx);
+  int n = 0;
+  (void)split_z_dispatch(p.nz, ra, [&](auto l, auto r) -> hipError_t {
+    n = p.nx * (p.ny / ra / NZ<T, decltype(l)::value, decltype(r)::value>::NY2);
+    return hipSuccess;
+  });
+  return n;
+}
+template <typename T>
+hipError_t nsplit_z(const SplitNeuArgs<T>& s, hipStream_t st) {
+  return split_z_dispatch(s.p.nz, nsplit_ra(s.p.ny, s.p.nx), [&](auto l, auto r) -> hipError_t {
+    using Z = NZ<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!Z::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_nsplit_z<Z>), dim3((unsigned)(s.p.nx * (s.p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, s);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_NEU_X
+template <typename T>
+bool nsplit_x_fits(int nx, int ny) {
+  const int ra = nsplit_ra(ny, nx);
+  return ra != 0 && split_x_dispatch(nx, ny / ra, [&](auto l, auto r) -> hipError_t {
+           using X = NX<T, decltype(l)::value, decltype(r)::value>;
+           return X::fits && ny % X::NC == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename T>
+hipError_t nsplit_x(const SplitNeuArgs<T>& s, hipStream_t st) {
+  return split_x_dispatch(s.p.nx, s.p.ny / nsplit_ra(s.p.ny, s.p.nx), [&](auto l, auto r) -> hipError_t {
+    using X = NX<T, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!X::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_nsplit_x<X>), dim3((unsigned)(s.p.ny / X::NC * (s.p.nz / 2))), dim3(X::NT), 0, st, s);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_NEU_REAL
+// FP64 tiles also of the grids whose FP32 step fits: one y2 where two do not.
+template <int L, int RA>
+using NZReal = NZ<double, L, RA, NZ<double, L, RA>::fits ? nsplit_ny2<double>(L, RA) : 1>;
+bool nsplit_real_fits(int nx, int ny, int nz) {
+  const int ra = nsplit_ra(ny, nx);
+  return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
+           using Z = NZReal<decltype(l)::value, decltype(r)::value>;
+           return Z::fits && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+         }) == hipSuccess;
+}
+template <typename TI>
+hipError_t nsplit_real(const cplx<TI>* a, double* out, const PParams<double>& p, const cplx<double>* qtz,
+                       hipStream_t st) {
+  return split_z_dispatch(p.nz, nsplit_ra(p.ny, p.nx), [&](auto l, auto r) -> hipError_t {
+    using Z = NZReal<decltype(l)::value, decltype(r)::value>;
+    if constexpr (!Z::fits) {
+      return hipErrorInvalidValue;
+    } else {
+      SMX_LAUNCH((k_nsplit_real<Z, TI>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, a, out, p,
+                 qtz);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename TI, typename TO>
+hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
+                       int dir, hipStream_t st) {
+  if (nsplit_ra(ny, nx) == 0 || ny > 384 || nz % 2 != 0) return hipErrorInvalidValue;
+  SMX_LAUNCH((k_nform<TI, TO>), dim3((unsigned)(nx * (nz / 2))), dim3(256), 0, st, in, out, nx, ny, nz, nsplit_ra(ny, nx), twy,
+             qty, dir);
+  return hipGetLastError();
+}
+#endif
+
 }  // namespace smx

@@ -2,6 +2,7 @@
 // smx_split_launch.h, instantiated per precision in smx_split_z_*.hip and smx_split_x_*.hip.
 #pragma once
 #include "smx_split_adv.h"
+#include "smx_split_neu.h"
 
 namespace smx {
 
@@ -28,6 +29,18 @@ template <typename T> hipError_t split_adv_stokes(const SplitAdvArgs<T>& s, hipS
 template <typename T> hipError_t split_adv_advnl(const SplitAdvArgs<T>& s, hipStream_t st);
 template <typename T> hipError_t split_adv_update(const SplitAdvArgs<T>& s, hipStream_t st);
 bool split_real_fits(int ny, int nz);
+// The Neumann step's two launches, its real field and its change of form (smx_split_neu.h).
+template <typename T> bool nsplit_z_fits(int nx, int ny, int nz);
+template <typename T> bool nsplit_x_fits(int nx, int ny);
+template <typename T> int nsplit_z_blocks(const PParams<T>& p);
+template <typename T> hipError_t nsplit_z(const SplitNeuArgs<T>& s, hipStream_t st);
+template <typename T> hipError_t nsplit_x(const SplitNeuArgs<T>& s, hipStream_t st);
+bool nsplit_real_fits(int nx, int ny, int nz);
+template <typename TI>
+hipError_t nsplit_real(const cplx<TI>* a, double* out, const PParams<double>& p, const cplx<double>* qtz, hipStream_t st);
+template <typename TI, typename TO>
+hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
+                       int dir, hipStream_t st);
 // Rows of a stage array (or, with the perm directions, of the carry) between the two forms, in place
 // allowed.  kmul: k_y table of the d/dy of a standard-form input, or nullptr.
 template <typename T>
