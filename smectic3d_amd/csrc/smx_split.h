@@ -13,8 +13,12 @@
 // and the carry R(kx, ky = k1 + RA k2, kz) is at [kz][kx][k1 RB + k2] (the split form; the four-pass
 // kernels of smx_periodic.h and the diagnostics use the standard one, ky at its index).
 //
-// Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 64 + 98 us and
-// 33 + 47 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
+// In the z kernel a lane has both lines of a column pair, so that it combines their half spectra into the
+// transform's input (and the other way back) in registers; a tile of half spectra, combined as it is read,
+// took two reads per value each way (64 -> 59 us at 256^3 FP64, 39.4 -> 37.0 at 192 x 96 x 384).
+//
+// Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 59 + 98 us and
+// 33 + 46 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
 // from two launches in place of four as well: 64^3 FP32 3.71 -> 2.97 ms for 200 steps and their checks.
 #pragma once
 #include "smx_periodic.h"
@@ -42,13 +46,17 @@ __host__ __device__ __forceinline__ int split_pos(int k1, int y2, int rb) {
   return (k1 >> 1) * 2 * rb + (y2 / YC) * 2 * YC + (k1 & 1) * YC + y2 % YC;
 }
 // y2 of a z tile: a whole piece or half of one (the tile's two parities of k1 share a line).  Whole pieces
-// where two blocks of the tile still fit a CU (192 x 96 x 384 FP64: 37.6 us with halves, 48.6 with one
-// block of whole pieces; 256^3 FP32: 34 with whole, 42 with halves), except in the shortest boxes, which
-// want more blocks (96^3 FP64 10.9 against 12.1 us, 128^3 FP32 11.7 against 10.2), and the shortest
-// lines, where half a piece would leave a wave mostly empty.
+// on long lines of a power of two (256^3 FP32: 32.9 us, 34.3 with halves; 128^3 FP32 9.7 and 11.4, FP64 15.0
+// and 15.2), where two blocks of the tile still fit a CU, and on the shortest, where half a piece would
+// leave a wave mostly empty.  Half pieces, twice the blocks, in all others (192^3 FP32 20.4 us, 23.3 with
+// whole; 96^3 FP64 10.1 and 11.0; 192 x 96 x 384 FP64 37.0 and 46.8; 64 x 64 x 256 FP64 10.4 and 11.6).
 template <typename T>
 constexpr int split_ny2(int l, int ra) {
-  return (l > 96 || l <= 32 || ra == 4) && l * (2 * ra + 2) * 2 * (int)sizeof(T) <= 80 * 1024 && (ra <= 8 || sizeof(T) == 4) ? 4 : 2;
+  const bool fp32 = sizeof(T) == 4;
+  return (l <= 32 || ra == 4 || (l > 96 && l % 3 != 0 && (fp32 || l <= 128))) && (ra <= 8 || fp32) &&
+                 l * (2 * ra + 4) * 2 * (int)sizeof(T) <= 80 * 1024
+             ? 4
+             : 2;
 }
 // Lanes that share one y line in the z kernel (pair_dft): two from radix 16 on, where one lane's 16
 // values make its loads the longest part (256^3 FP32: 40.6 -> 34.0 us; 192^3 FP32: 22.3 with one, 27.7).
@@ -94,20 +102,13 @@ struct ZS {
   static constexpr int L = L_, RA = RA_, NY2 = NY2_, V = V_, P = P_;
   static constexpr int E = PlanV<L, V>::E, TPC = L / E;
   static constexpr int NPR = RA * NY2 / 2, NT = NPR * TPC, NZH = L / 2 + 1;
-  // Half-spectrum tile [kz][part of the y1][y1][y2]: the parts PH apart and rows HP, so that the
-  // pieces which lanes write (P parts x NY2 x consecutive kz) fall in different banks: 8 banks from
-  // part to part, 8 P from row to row.
-  static constexpr int DW = sizeof(cplx<T>) / 4;  // banks of a value
-  static constexpr int pad_to(int n, int banks) {
-    while (n * DW % 64 != banks) ++n;
-    return n;
-  }
-  static constexpr int H = RA / P;
-  static constexpr int PH = P == 2 ? pad_to(H * NY2, 8) : 0, HP = pad_to(PH + H * NY2, 8 * P);
-  static constexpr int FP = NPR, SP = NPR + NY2 / 2;  // transform tile pitch; pitch of the split's copy
+  static constexpr int H = RA / P, HC = H / 2;
+  // Tile pitch of the transform, and of the items, whose lanes write runs of NY2 columns of successive rows:
+  // those fall in other banks.  Column q: the lines y1 = 2 (q / NY2) and the next, y2 = q % NY2.
+  static constexpr int FP = NPR, HP = NPR + NY2;
   // Items of the y part, H values each: one kz, one y2 and (P = 2) one parity of k1, half of the y1.
   static constexpr int ITEMS = NZH * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
-  static constexpr int LDS = (NZH * HP > L * SP ? NZH * HP : L * SP);
+  static constexpr int LDS = L * HP;
   static constexpr int RED = (NT % 64 == 0) ? NT / 64 : NT;
   static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
 };
@@ -237,23 +238,23 @@ __device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, i
 #pragma unroll
         for (int k = 0; k < Z::H; ++k) w[it][k] = mk(-kz * w[it][k].y, kz * w[it][k].x);
       }
-      // only the real parts of kz = 0 and nz/2 enter (the half-complex stage of an FFTW c2r)
+      // A + iB of two lines at m, and at L - m from the conjugates; only the real parts of kz = 0 and
+      // nz/2 enter (the half-complex stage of an FFTW c2r)
       const T im = (m == 0 || m == L / 2) ? (T)0 : (T)1;
-      cplx<T>* f = &F[m * Z::HP + lo * Z::PH + c];
+      cplx<T>* fa = &F[m * Z::HP + lo * Z::HC * Z::NY2 + c];
+      cplx<T>* fb = &F[(m == 0 ? 0 : L - m) * Z::HP + lo * Z::HC * Z::NY2 + c];
 #pragma unroll
-      for (int k = 0; k < Z::H; ++k) f[k * Z::NY2] = mk(w[it][k].x, im * w[it][k].y);
+      for (int h = 0; h < Z::HC; ++h) {
+        const cplx<T> A = mk(w[it][2 * h].x, im * w[it][2 * h].y), B = mk(w[it][2 * h + 1].x, im * w[it][2 * h + 1].y);
+        fa[h * Z::NY2] = mk(A.x - B.y, A.y + B.x);
+        fb[h * Z::NY2] = mk(A.x + B.y, B.x - A.y);
+      }
     }
   }
   __syncthreads();
-  const int qa = Z::P == 1 || q < Z::NPR / 2 ? 2 * q : 2 * q - Z::NPR + Z::PH;
 #pragma unroll
-  for (int e = 0; e < Z::E; ++e) {
-    const int n = Tile<T, L, Z::E, Z::FP>::template pos_in<inv_first<L, Z::V>()>(tc, e);
-    const bool lo = n <= L / 2;
-    const int m = lo ? n : L - n;
-    const cplx<T> A = F[m * Z::HP + qa], B = F[m * Z::HP + qa + 1];
-    v[e] = lo ? mk(A.x - B.y, A.y + B.x) : mk(A.x + B.y, B.x - A.y);
-  }
+  for (int e = 0; e < Z::E; ++e)
+    v[e] = F[Tile<T, L, Z::E, Z::HP>::template pos_in<inv_first<L, Z::V>()>(tc, e) * Z::HP + q];
   InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
 }
 
@@ -265,21 +266,21 @@ __device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t ro
   constexpr uint32_t CB = sizeof(cplx<T>);
   FwdFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
   __syncthreads();
-  Tile<T, L, Z::E, Z::SP>::template store<fwd_last<L, Z::V>()>(v, F, q, tc);
+  Tile<T, L, Z::E, Z::HP>::template store<fwd_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < Z::IPT; ++it) {
     const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, m = i / Z::P / Z::NY2;
     if (i < Z::ITEMS) {
-      const int mm = m == 0 ? 0 : L - m;
+      const cplx<T>* fa = &F[m * Z::HP + lo * Z::HC * Z::NY2 + c];
+      const cplx<T>* fb = &F[(m == 0 ? 0 : L - m) * Z::HP + lo * Z::HC * Z::NY2 + c];
       cplx<T> w[Z::H];
 #pragma unroll
-      for (int k = 0; k < Z::H; ++k) {
-        const int col = (lo * Z::H + k) * (Z::NY2 / 2) + c / 2;
-        const cplx<T> W = F[m * Z::SP + col], Wm = F[mm * Z::SP + col];
+      for (int h = 0; h < Z::HC; ++h) {
+        const cplx<T> W = fa[h * Z::NY2], Wm = fb[h * Z::NY2];
         // W = X + iY:  X = (W_k + conj W_{-k})/2,  Y = (W_k - conj W_{-k})/(2i)
-        w[k] = (c & 1) == 0 ? mk((T)0.5 * (W.x + Wm.x), (T)0.5 * (W.y - Wm.y))
-                            : mk((T)0.5 * (W.y + Wm.y), (T)0.5 * (Wm.x - W.x));
+        w[2 * h] = mk((T)0.5 * (W.x + Wm.x), (T)0.5 * (W.y - Wm.y));
+        w[2 * h + 1] = mk((T)0.5 * (W.y + Wm.y), (T)0.5 * (Wm.x - W.x));
       }
       if constexpr (Z::P == 2) pair_dft<Z::H, -1>(w, lo);
       else dft<Z::H, -1>(w);
@@ -322,7 +323,6 @@ __device__ __forceinline__ void zsplit_tile(cplx<T>* a, cplx<T>* r, int op, cons
   zs_inverse<Z>((const cplx<T>*)base, rowb, rb, F, TW, tid, q, tc, v, (const T*)nullptr, p.twz);
   constexpr int RP = fwd_first<L, Z::V>();
   static_assert(fwd_first<L, Z::V>() == inv_last<L, Z::V>(), "plan symmetry");
-  // column pair q: y = (q / (NY2/2)) rb + yg NY2 + 2 (q % (NY2/2)) and the next
   const bool pen = (op == Z_OP_NL) && p.mid > 0 && p.mid < L - 1;
   if (pen) {
     __syncthreads();
@@ -384,16 +384,16 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_real(const cplx<TI>* a, double
                     (uint32_t)p.nxy * (uint32_t)sizeof(cplx<TI>), rb, F, TW, tid, q, tc, v,
                     (const double*)nullptr, p.twz);
   __syncthreads();
-  Tile<double, L, Z::E, Z::SP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
+  Tile<double, L, Z::E, Z::HP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
   // lanes run along z of one column pair: two coalesced rows
   for (int i = tid; i < Z::NPR * L; i += Z::NT) {
     const int qq = i / L, n = i - qq * L;
-    const int y = (qq / (Z::NY2 / 2)) * rb + yg * Z::NY2 + 2 * (qq % (Z::NY2 / 2));
-    const cplx<double> w = F[n * Z::SP + qq];
+    const int y = 2 * (qq / Z::NY2) * rb + yg * Z::NY2 + qq % Z::NY2;
+    const cplx<double> w = F[n * Z::HP + qq];
     double* row = out + ((int64_t)x * p.ny + y) * L;
     row[n] = w.x;
-    row[L + n] = w.y;
+    row[(int64_t)rb * L + n] = w.y;
   }
 }
 

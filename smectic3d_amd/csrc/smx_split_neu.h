@@ -84,7 +84,9 @@ struct NZ {
   static constexpr int E = PlanV<L, V>::E, TPC = L / E;
   static constexpr int NPR = RA * NY2 / 2, NT = NPR * TPC;
   static constexpr int H = RA / P, HC = H / 2;
-  static constexpr int HP = NPR + NY2;  // tile pitch: the runs of NY2 values of successive rows in other banks
+  // Tile pitches of the items and of the transform, as in ZS; one in FP32, where the second costs the registers
+  // that let a second block of 1024 threads on the CU (256^3: 40 -> 53 us).
+  static constexpr int HP = NPR + NY2, FP = sizeof(T) == 8 ? NPR : HP;
   static constexpr int ITEMS = L / 2 * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
   static constexpr int LDS = L * HP, RED = (NT % 64 == 0) ? NT / 64 : NT;
   static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
@@ -152,7 +154,7 @@ __device__ __forceinline__ void nz_inverse(const cplx<TI>* src, uint32_t rowb, i
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < Z::E; ++e) v[e] = F[Tile<T, L, Z::E, Z::HP>::template pos_in<inv_first<L, Z::V>()>(tc, e) * Z::HP + q];
-  InvFFT<T, L, Z::HP, Z::V>::run(v, F, q, tc, twl);
+  InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
 }
 
 // Forward half: the DCT-II along z of the pairs in v and radix RA over y1.
@@ -161,7 +163,7 @@ __device__ __forceinline__ void nz_forward(cplx<T>* v, cplx<T>* dst, uint32_t ro
                                            const cplx<T>* TW, const cplx<T> (*qw)[2], int tid, int q, int tc) {
   constexpr int L = Z::L;
   constexpr uint32_t CB = sizeof(cplx<T>);
-  FwdFFT<T, L, Z::HP, Z::V>::run(v, F, q, tc, TW);
+  FwdFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, TW);
   __syncthreads();
   Tile<T, L, Z::E, Z::HP>::template store<fwd_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
