@@ -597,9 +597,9 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
 
 // ---- the two forms of a state (smx_split.h, smx_split_neu.h) ----
 // Rows of a stage array or carry from one form to the other on the handle's stream, in place allowed.
-template <typename T>
-static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
-  const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
+template <typename T, typename TI = T>
+static int form_rows(smx_handle* h, const cplx<TI>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
+  const hipError_t e = split_form<T, TI>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
   if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
   return SMX_OK;
 }
@@ -652,11 +652,13 @@ static int stage_to_f64(smx_handle* h, const void* stage, void* dst, bool split)
     return h->fp32 ? nform_rows<float, double>(h, stage, dst, FORM_TO_STD)
                    : nform_rows<double, double>(h, stage, dst, FORM_TO_STD);
   if (h->fp32) {
-    hipLaunchKernelGGL(k_f32_to_f64, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, (const float*)stage,
-                       (double*)dst, ncomp);
-    HIPCHK(hipGetLastError());
-    if (split)
-      CHK(form_rows<double>(h, (const cplx<double>*)dst, (cplx<double>*)dst, FORM_TO_STD));
+    if (split) {
+      CHK((form_rows<double, float>(h, (const cplx<float>*)stage, (cplx<double>*)dst, FORM_TO_STD)));
+    } else {
+      hipLaunchKernelGGL(k_f32_to_f64, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, (const float*)stage,
+                         (double*)dst, ncomp);
+      HIPCHK(hipGetLastError());
+    }
     if (!h->neumann) {
       const int64_t pairs = 2 * (int64_t)h->cfg.nx * (h->cfg.ny / 2 + 1);
       hipLaunchKernelGGL(k_herm_stage, dim3((unsigned)std::min<int64_t>((pairs + 255) / 256, 4096)), dim3(256), 0,
@@ -2299,7 +2301,9 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   const int ns = surf_nsplit(h->neumann, h->cfg.nx, h->cfg.nz);
   // An FP64 state is its own x stage, and an FP32 Neumann stage is read as it is (widened on
   // load); a periodic FP32 stage is copied to FP64 and projected (stage_to_f64) first.
-  // A split-form state is brought to the standard form there.
+  // A split-form state is brought to the standard form there, in FP64 (an FP32 Neumann box of 256 x 256 x
+  // 384 then takes 0.96 ms a call, 0.81 from a standard-form state; an FP32 copy was no faster and lost
+  // the second derivatives' accuracy).
   const bool f32in = h->fp32 && h->neumann && !h->split, w0copy = h->split || (!h->neumann && h->fp32);
   const bool w0room = h->split_ok || (!h->neumann && h->fp32);
   // real psi, the FP64 x stage copy, the field values at each column's evaluation index (ns

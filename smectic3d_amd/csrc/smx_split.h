@@ -580,8 +580,9 @@ __global__ __launch_bounds__(X::NT) void k_xsplit_grp(const SplitArgs<typename X
 //   perm: the carry's rows, an order of entries only.
 // kmul: k_y table of a standard-form input's d/dy, or nullptr.
 enum FormDir { FORM_TO_STD = 0, FORM_FROM_STD = 1, FORM_PERM_TO_STD = 2, FORM_PERM_FROM_STD = 3 };
-template <typename T, int RB>
-__global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny,
+// TI: the input's type (float rows widened into an FP64 copy).
+template <typename T, int RB, typename TI = T>
+__global__ __launch_bounds__(256) void k_form(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny,
                                               const cplx<T>* __restrict__ twy, int dir, const T* __restrict__ kmul) {
   constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
   __shared__ cplx<T> S[CAP + CAP / 16];
@@ -590,10 +591,11 @@ __global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, i
   const int64_t r0 = (int64_t)blockIdx.x * rows;
   const int nr = (int)(nrows - r0 < rows ? nrows - r0 : rows);
   const int n = nr * ny;
-  const cplx<T>* src = in + r0 * ny;
+  const cplx<TI>* src = in + r0 * ny;
   cplx<T>* dst = out + r0 * ny;
   for (int i = tid; i < n; i += 256) {
-    cplx<T> e = src[i];
+    const cplx<TI> g = src[i];
+    cplx<T> e = mk((T)g.x, (T)g.y);
     if (kmul != nullptr) {  // i k_y of the spectral d/dy (pf3d.cpp:405)
       const T k = kmul[i % ny];
       e = mk(-k * e.y, k * e.x);

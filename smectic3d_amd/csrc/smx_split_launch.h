@@ -232,23 +232,23 @@ hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, hip
     }
   });
 }
-template <typename T, int RB>
-static void split_form_launch(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+template <typename T, int RB, typename TI>
+static void split_form_launch(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
                               const T* kmul, hipStream_t st) {
   const int rows = 1024 / ny;
   const dim3 grid((unsigned)((nrows + rows - 1) / rows));
-  SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul);
+  SMX_LAUNCH((k_form<T, RB, TI>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul);
 }
-template <typename T>
-hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+template <typename T, typename TI>
+hipError_t split_form(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
                       const T* kmul, hipStream_t st) {
   const int ra = split_ra(ny);
   if (ra == 0) return hipErrorInvalidValue;
   switch (ny / ra) {
-    case 4: split_form_launch<T, 4>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 8: split_form_launch<T, 8>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 12: split_form_launch<T, 12>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 16: split_form_launch<T, 16>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 4: split_form_launch<T, 4, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 8: split_form_launch<T, 8, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 12: split_form_launch<T, 12, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    case 16: split_form_launch<T, 16, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -339,9 +339,17 @@ hipError_t nsplit_real(const cplx<TI>* a, double* out, const PParams<double>& p,
 template <typename TI, typename TO>
 hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
                        int dir, hipStream_t st) {
-  if (nsplit_ra(ny, nx) == 0 || ny > 384 || nz % 2 != 0) return hipErrorInvalidValue;
-  SMX_LAUNCH((k_nform<TI, TO>), dim3((unsigned)(nx * (nz / 2))), dim3(256), 0, st, in, out, nx, ny, nz, nsplit_ra(ny, nx), twy,
-             qty, dir);
+  const int ra = nsplit_ra(ny, nx);
+  if (ra == 0) return hipErrorInvalidValue;
+  const int rows = 1024 / ny;
+  const dim3 grid((unsigned)((nx * (nz / 2) + rows - 1) / rows));
+#define SMX_CASE(RB)                                                                                           \
+  case RB: SMX_LAUNCH((k_nform<TI, TO, RB>), grid, dim3(256), 0, st, in, out, nx, ny, nz, twy, qty, dir); break;
+  switch (ny / ra) {
+    SMX_CASE(4) SMX_CASE(8) SMX_CASE(12) SMX_CASE(16)
+    default: return hipErrorInvalidValue;
+  }
+#undef SMX_CASE
   return hipGetLastError();
 }
 #endif

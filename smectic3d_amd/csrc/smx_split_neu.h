@@ -403,65 +403,83 @@ __global__ __launch_bounds__(X::NT) void k_nsplit_x(SplitNeuArgs<typename X::T> 
 }
 
 // ---------------------------------------------------------------------------
-// Between the two forms, out of place, in FP64; one block per row (j, x).  Runs when a step path is changed
-// and where a diagnostic reads the standard form, so it sums directly (ny RB terms a row).
-template <typename TI, typename TO>
+// Between the two forms, out of place, in FP64; whole rows (j, x) per block of 256 threads, an item the RB
+// values of one row and k1 (as k_form).
+template <typename TI, typename TO, int RB>
 __global__ __launch_bounds__(256) void k_nform(const TI* __restrict__ in, TO* __restrict__ out, int nx, int ny, int nz,
-                                               int ra, const cplx<double>* __restrict__ twy,
+                                               const cplx<double>* __restrict__ twy,
                                                const cplx<double>* __restrict__ qty, int dir) {
   using C = cplx<double>;
-  __shared__ C S[384];
-  __shared__ C W[384];
-  const int j = blockIdx.x / nx, x = blockIdx.x % nx, rb = ny / ra, tid = threadIdx.x;
-  const int kz[2] = {j, j == 0 ? nz / 2 : nz - j};
-  const int64_t std0 = ((int64_t)kz[0] * nx + x) * ny, std1 = ((int64_t)kz[1] * nx + x) * ny;
-  const int64_t row = 2 * ((int64_t)j * nx + x) * ny;  // words of the split-form row
+  constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
+  static_assert(CAP / RB <= 256, "one item per thread");
+  __shared__ C S[CAP + CAP / 16];
+  auto at = [](int i) { return i + (i >> 4); };
+  const int ra = ny / RB, rows = CAP / ny, tid = threadIdx.x, nrows = nx * (nz / 2);
+  const int r0 = blockIdx.x * rows, nr = nrows - r0 < rows ? nrows - r0 : rows, n = nr * ny;
+  // words of row r: its two planes in the standard form, and the split form's row
+  auto plane = [&](int r, int b) {
+    const int j = r / nx, kz = b == 0 ? j : (j == 0 ? nz / 2 : nz - j);
+    return ((int64_t)kz * nx + (r - j * nx)) * ny;
+  };
   if (dir == FORM_PERM_TO_STD || dir == FORM_PERM_FROM_STD) {
-    for (int i = tid; i < ny; i += 256) {
-      const int t = i / (2 * rb), b = i / rb % 2, u = i % rb;
-      const int ka = nsplit_ky(t, u, ra, rb), k = b == 0 ? ka : (ka == 0 ? ny / 2 : ny - ka);
+    for (int i = tid; i < n; i += 256) {
+      const int r = r0 + i / ny, c = i % ny;
+      const int t = c / (2 * RB), b = c / RB % 2, u = c % RB;
+      const int ka = nsplit_ky(t, u, ra, RB), k = b == 0 ? ka : (ka == 0 ? ny / 2 : ny - ka);
+      const int64_t o = 2 * ((int64_t)r * ny + c);
       if (dir == FORM_PERM_TO_STD) {
-        out[std0 + k] = (TO)in[row + 2 * i];
-        out[std1 + k] = (TO)in[row + 2 * i + 1];
+        out[plane(r, 0) + k] = (TO)in[o];
+        out[plane(r, 1) + k] = (TO)in[o + 1];
       } else {
-        out[row + 2 * i] = (TO)in[std0 + k];
-        out[row + 2 * i + 1] = (TO)in[std1 + k];
+        out[o] = (TO)in[plane(r, 0) + k];
+        out[o + 1] = (TO)in[plane(r, 1) + k];
       }
     }
     return;
   }
-  if (dir == FORM_FROM_STD) {
-    for (int k = tid; k < ny; k += 256) S[k] = mk((double)in[std0 + k], (double)in[std1 + k]);
-    __syncthreads();
-    for (int k = tid; k < ny; k += 256) W[k] = dct3_in(S[k], k == 0 ? mk<double>(0, 0) : S[ny - k], qty[k]);
-    __syncthreads();
-    for (int i = tid; i < ny; i += 256) {
-      const int k1 = i % ra, y2 = i / ra;
-      C a = mk<double>(0, 0);
-      for (int k2 = 0; k2 < rb; ++k2) {
-        const int k = k1 + ra * k2;
-        a = a + cmul(W[k], conjg(twy[y2 * k % ny]));
-      }
-      const int o = nsplit_pos(k1, y2, ra, rb);
-      out[row + 2 * o] = (TO)a.x;
-      out[row + 2 * o + 1] = (TO)a.y;
+  const bool from = dir == FORM_FROM_STD;
+  for (int i = tid; i < n; i += 256) {
+    const int r = r0 + i / ny, c = i % ny;
+    const int64_t o = 2 * ((int64_t)r * ny + c);
+    S[at(i)] = from ? mk((double)in[plane(r, 0) + c], (double)in[plane(r, 1) + c]) : mk((double)in[o], (double)in[o + 1]);
+  }
+  __syncthreads();
+  const int row = tid / ra, k1 = tid - row * ra;
+  const bool item = tid < nr * ra;
+  C w[RB];
+  if (item) {
+#pragma unroll
+    for (int c = 0; c < RB; ++c) {
+      const int k = k1 + ra * c;
+      w[c] = from ? dct3_in(S[at(row * ny + k)], k == 0 ? mk<double>(0, 0) : S[at(row * ny + ny - k)], qty[k])
+                  : cmul(S[at(row * ny + nsplit_pos(k1, c, ra, RB))], twy[k1 * c]);
     }
-  } else {
-    for (int i = tid; i < ny; i += 256) {
-      const int o = nsplit_pos(i % ra, i / ra, ra, rb);
-      S[i] = mk((double)in[row + 2 * o], (double)in[row + 2 * o + 1]);
+    if (from) {
+      dft<RB, +1>(w);
+#pragma unroll
+      for (int c = 0; c < RB; ++c) w[c] = cmul(w[c], conjg(twy[k1 * c]));
+    } else {
+      dft<RB, -1>(w);
+#pragma unroll
+      for (int c = 0; c < RB; ++c) w[c] = (1.0 / RB) * w[c];
     }
-    __syncthreads();
-    for (int k = tid; k < ny; k += 256) {
-      C a = mk<double>(0, 0);
-      for (int y2 = 0; y2 < rb; ++y2) a = a + cmul(S[y2 * ra + k % ra], twy[y2 * k % ny]);
-      W[k] = (1.0 / rb) * a;
-    }
-    __syncthreads();
-    for (int k = tid; k < ny; k += 256) {
-      const C y = dct2_out(W[k], W[k == 0 ? 0 : ny - k], qty[k]);
-      out[std0 + k] = (TO)(0.5 * y.x);
-      out[std1 + k] = (TO)(0.5 * y.y);
+  }
+  __syncthreads();
+  if (item) {
+#pragma unroll
+    for (int c = 0; c < RB; ++c) S[at(row * ny + (from ? nsplit_pos(k1, c, ra, RB) : k1 + ra * c))] = w[c];
+  }
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) {
+    const int rr = i / ny, r = r0 + rr, c = i - rr * ny;
+    if (from) {
+      const int64_t o = 2 * ((int64_t)r * ny + c);
+      out[o] = (TO)S[at(i)].x;
+      out[o + 1] = (TO)S[at(i)].y;
+    } else {
+      const C y = dct2_out(S[at(i)], S[at(rr * ny + (c == 0 ? 0 : ny - c))], qty[c]);
+      out[plane(r, 0) + c] = (TO)(0.5 * y.x);
+      out[plane(r, 1) + c] = (TO)(0.5 * y.y);
     }
   }
 }
