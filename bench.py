@@ -475,6 +475,12 @@ def measured_traffic(slot, schedule, n, real="double"):
             kernels = json.load(f)["kernels"]
     except (OSError, ValueError, KeyError):
         return None
+    if slot in ("k_zsplit", "k_xsplit"):  # the two-launch step: one instantiation per grid and precision
+        tile = {"k_zsplit": "ZS", "k_xsplit": "XS"}[slot]
+        hits = [k for name, k in kernels.items() if name.startswith(f"smx::{slot}<smx::{tile}<{real}, {n},")]
+        if len(hits) != 1 or "FETCH_SIZE_bytes" not in hits[0] or "WRITE_SIZE_bytes" not in hits[0]:
+            return None
+        return hits[0]["FETCH_SIZE_bytes"] + hits[0]["WRITE_SIZE_bytes"]
     slots = ["k_ypass_inv", "k_zpass_nl", "k_ypass_fwd", "k_xpass_step"]
     if slot not in slots:
         return None
@@ -615,7 +621,8 @@ def main():
         },
         "schedule_fp64": r64["schedule"],
         "schedule_source": sched_src,
-        "schedule_note": "(columns per tile, plan variant) of the y-inverse, z, y-forward and x kernels",
+        "schedule_note": "(columns per tile, plan variant) of the y-inverse, z, y-forward and x kernels; the "
+                         "default schedule leaves the step to the two-launch kernels where the grid has them",
         "kernel_sum_ms_fp64": ksum64,
         "ms_per_step_over_kernel_sum_fp64": r64["ms_per_step"] / ksum64,
         "kernels_fp64": kernel_table(r64["kernels"]),
