@@ -274,9 +274,9 @@ int smx_batch_adjoint_nodes(smx_batch *b, int64_t *nodes);
  * its eleven y passes.  Neumann handles: the tile width only (variant 0): 32 (default) or 16
  * columns in FP32, 16 (default) or 8 in FP64; the advected Neumann step keeps the defaults.
  * The step's result depends on the schedule only through rounding.  While the default schedule is
- * in place a periodic handle steps in two launches instead of four (four instead of fifteen with
- * advection) where its grid allows it (the y transforms divided between the z and the x kernels: every
- * grid with ny <= 384 whose tiles fit a workgroup's LDS); any other schedule selects the kernels it names.
+ * in place a handle steps in two launches instead of four (a periodic advected one in four instead of
+ * fifteen) where its grid allows it (the y transforms divided between the z and the x kernels: grids with
+ * ny <= 384 whose tiles fit a workgroup's LDS); any other schedule selects the kernels it names.
  */
 typedef struct smx_schedule {
   int nc[4];
