@@ -19,7 +19,7 @@
 //
 // Measured at 256^3: four passes 213 us FP64 and 112 us FP32 a step; the two kernels 59 + 98 us and
 // 33 + 46 us (6 moves of a stage array at the copy rate would take 118 and 59 us).  Smaller boxes gain
-// from two launches in place of four as well: 64^3 FP32 3.71 -> 2.97 ms for 200 steps and their checks.
+// from two launches in place of four as well: 64^3 FP32 3.75 -> 2.56 ms for 200 steps and their checks.
 #pragma once
 #include "smx_periodic.h"
 
