@@ -236,11 +236,12 @@ int smx_batch_create(int nbox, const smx_config *cfgs, smx_batch **out);
 void smx_batch_destroy(smx_batch *b);
 /* Per-box handle for set/get/diagnostics; owned by the batch. */
 int smx_batch_handle(smx_batch *b, int box, smx_handle **h);
-/* Advance every box by nsteps: launches of a graph of `graph_steps` steps, or of up to four times as
- * many where that divides nsteps / graph_steps (captured once and kept while it fits the calls), plus a
- * direct remainder. */
+/* Advance every box by nsteps: launches of a graph of two to four times `graph_steps` steps (a number that
+ * the first such call divides into) and of one of `graph_steps` for what that leaves, plus a direct
+ * remainder.  Each graph is captured when a call first needs it and kept while graph_steps and the boxes'
+ * schedules stay the same. */
 int smx_batch_run(smx_batch *b, int64_t nsteps, int64_t graph_steps);
-/* Number of kernel nodes in the captured graph (0 before the first run). */
+/* Number of kernel nodes in the captured graph, the longer of two (0 before the first run). */
 int smx_batch_graph_nodes(smx_batch *b, int64_t *nodes);
 
 /*

@@ -1311,13 +1311,18 @@ struct smx_batch {
   hipStream_t st = nullptr;  // capture / launch stream
   hipEvent_t fork = nullptr;
   std::vector<hipEvent_t> joins;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  // captured steps: one stretch of graph_steps, and m stretches; each made when a call first needs it
+  struct Graph {
+    hipGraph_t g = nullptr;
+    hipGraphExec_t x = nullptr;
+    int64_t m = 0;
+  } one, many;
   int64_t graph_steps = 0;
   // boxes that share precision, grid and tile schedules (periodic, no advection) advance in
   // the graph with one grouped launch per pass: member indices, and each group's GrpArgs
   // array in device memory (built at capture, freed with the graph)
   std::vector<std::vector<int>> groups;
+  std::vector<int> single;  // the boxes of no group
   std::vector<void*> grp_args;
   std::vector<std::array<PassSched, NSLOTS>> cap_sched;  // every box's schedules at capture
   std::vector<bool> cap_split;                           // and its path
@@ -1358,6 +1363,7 @@ static void batch_free_groups(smx_batch* b) {
     if (d) (void)hipFree(d);
   b->grp_args.clear();
   b->groups.clear();
+  b->single.clear();
 }
 
 static bool same_sched(const smx_handle* a, const smx_handle* b) {
@@ -1441,32 +1447,43 @@ static int group_steps(smx_batch* b, const std::vector<int>& members, const void
   return SMX_OK;
 }
 
-static int batch_capture(smx_batch* b, int64_t gsteps) {
-  if (b->exec) {
-    (void)hipGraphExecDestroy(b->exec);
-    b->exec = nullptr;
-  }
-  if (b->graph) {
-    (void)hipGraphDestroy(b->graph);
-    b->graph = nullptr;
+static void batch_drop_graphs(smx_batch* b) {
+  for (smx_batch::Graph* q : {&b->one, &b->many}) {
+    if (q->x) (void)hipGraphExecDestroy(q->x);
+    if (q->g) (void)hipGraphDestroy(q->g);
+    *q = smx_batch::Graph{};
   }
   batch_free_groups(b);
   b->cap_sched.clear();
   b->cap_split.clear();
-  for (const smx_handle* h : b->boxes) {
-    std::array<PassSched, NSLOTS> s;
-    for (int k = 0; k < NSLOTS; ++k) s[k] = h->sched[k];
-    b->cap_sched.push_back(s);
-    b->cap_split.push_back(h->split);
-  }
+  b->graph_steps = 0;
+}
+
+// Groups of the boxes as they are now, for stretches of gsteps; the graphs of another grouping go.
+static int batch_plan(smx_batch* b, int64_t gsteps) {
+  batch_drop_graphs(b);
   std::vector<int> single;
   batch_make_groups(b, single);
+  b->single = single;
   b->grp_args.assign(b->groups.size(), nullptr);
   for (size_t k = 0; k < b->groups.size(); ++k) {
     const smx_handle* h = b->boxes[b->groups[k][0]];
     CHK(h->fp32 ? group_args<float>(b, b->groups[k], &b->grp_args[k])
                 : group_args<double>(b, b->groups[k], &b->grp_args[k]));
   }
+  for (const smx_handle* h : b->boxes) {
+    std::array<PassSched, NSLOTS> s;
+    for (int k = 0; k < NSLOTS; ++k) s[k] = h->sched[k];
+    b->cap_sched.push_back(s);
+    b->cap_split.push_back(h->split);
+  }
+  b->graph_steps = gsteps;
+  return SMX_OK;
+}
+
+// A graph of m stretches.
+static int batch_capture(smx_batch* b, int64_t m, smx_batch::Graph* out) {
+  const int64_t gsteps = m * b->graph_steps;
   HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
   int rc = SMX_OK;
   hipError_t e = hipEventRecord(b->fork, b->st);
@@ -1481,8 +1498,8 @@ static int batch_capture(smx_batch* b, int64_t gsteps) {
     if (rc == SMX_OK && e == hipSuccess) e = hipEventRecord(b->joins[i0], h->st);
     if (rc == SMX_OK && e == hipSuccess) e = hipStreamWaitEvent(b->st, b->joins[i0], 0);
   }
-  for (size_t k = 0; k < single.size() && rc == SMX_OK && e == hipSuccess; ++k) {
-    const int i = single[k];
+  for (size_t k = 0; k < b->single.size() && rc == SMX_OK && e == hipSuccess; ++k) {
+    const int i = b->single[k];
     smx_handle* h = b->boxes[i];
     e = hipStreamWaitEvent(h->st, b->fork, 0);
     if (e == hipSuccess) rc = box_steps(h, gsteps);
@@ -1495,11 +1512,16 @@ static int batch_capture(smx_batch* b, int64_t gsteps) {
     if (g) (void)hipGraphDestroy(g);
     return rc;
   }
-  if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("batch capture: ") + hipGetErrorString(e));
-  if (e2 != hipSuccess) return fail(SMX_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e2));
-  b->graph = g;
-  HIPCHK(hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0));
-  b->graph_steps = gsteps;
+  if (e == hipSuccess) e = e2;
+  hipGraphExec_t x = nullptr;
+  if (e == hipSuccess) e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+  if (e != hipSuccess) {
+    if (g) (void)hipGraphDestroy(g);
+    return fail(SMX_ERR_HIP, std::string("batch capture: ") + hipGetErrorString(e));
+  }
+  out->g = g;
+  out->x = x;
+  out->m = m;
   return SMX_OK;
 }
 
@@ -2630,9 +2652,7 @@ void smx_batch_destroy(smx_batch* b) {
   if (!b) return;
   if (b->st) (void)hipStreamSynchronize(b->st);
   batch_drop_adj_graph(b);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  batch_free_groups(b);
+  batch_drop_graphs(b);
   for (auto e : b->joins)
     if (e) (void)hipEventDestroy(e);
   if (b->fork) (void)hipEventDestroy(b->fork);
@@ -2658,25 +2678,30 @@ int smx_batch_run(smx_batch* b, int64_t nsteps, int64_t graph_steps) {
     CHK(ensure_form(h, use_split(h)));
     HIPCHK(hipStreamSynchronize(h->st));
   }
-  // One graph carries up to four stretches of graph_steps where their number divides evenly (the
-  // kernels of a small box last a few microseconds, as long as the gap between two graphs); a
-  // captured graph that fits is kept.
+  // One launch takes up to four stretches of graph_steps (the kernels of a small box last a few
+  // microseconds, as long as the gap between two graphs): the number that the first call of several
+  // stretches divides into.  It is kept beside a graph of one stretch, which does what is left of a call
+  // that it does not divide, so that calls of other lengths capture nothing again.
   const int64_t ng = nsteps / graph_steps, rem = nsteps - ng * graph_steps;
-  int64_t m = b->graph_steps / graph_steps;
-  bool stale = !b->exec || m < 1 || b->graph_steps != m * graph_steps || ng % m != 0 ||
-               b->cap_sched.size() != b->boxes.size();
+  bool stale = b->graph_steps != graph_steps || b->cap_sched.size() != b->boxes.size();
   for (size_t i = 0; !stale && i < b->boxes.size(); ++i) {  // a box's schedule or path set since the capture
     if (b->cap_split[i] != b->boxes[i]->split) stale = true;
     for (int k = 0; k < NSLOTS; ++k)
       if (b->cap_sched[i][k].nc != b->boxes[i]->sched[k].nc || b->cap_sched[i][k].v != b->boxes[i]->sched[k].v)
         stale = true;
   }
-  if (ng > 0 && stale) {
-    for (m = 4; ng % m != 0;) --m;
-    CHK(batch_capture(b, m * graph_steps));
+  if (ng > 0) {
+    if (stale) CHK(batch_plan(b, graph_steps));
+    if (!b->many.x) {
+      int64_t m = 4;
+      while (ng % m != 0) --m;
+      if (m > 1) CHK(batch_capture(b, m, &b->many));
+    }
+    const int64_t nm = b->many.x ? ng / b->many.m : 0, n1 = b->many.x ? ng % b->many.m : ng;
+    if (n1 > 0 && !b->one.x) CHK(batch_capture(b, 1, &b->one));
+    for (int64_t g = 0; g < nm; ++g) HIPCHK(hipGraphLaunch(b->many.x, b->st));
+    for (int64_t g = 0; g < n1; ++g) HIPCHK(hipGraphLaunch(b->one.x, b->st));
   }
-  if (ng > 0)
-    for (int64_t g = 0; g < ng / m; ++g) HIPCHK(hipGraphLaunch(b->exec, b->st));
   HIPCHK(hipStreamSynchronize(b->st));
   for (smx_handle* h : b->boxes) {
     if (rem > 0) CHK(box_steps(h, rem));
@@ -2693,21 +2718,15 @@ int smx_batch_autotune(smx_batch* b, int reps) {
     CHK(smx_autotune(h, reps, nullptr));
   // the captured graphs hold the old schedules: capture again on the next run
   batch_drop_adj_graph(b);
-  if (b->exec) {
-    (void)hipGraphExecDestroy(b->exec);
-    b->exec = nullptr;
-  }
-  if (b->graph) {
-    (void)hipGraphDestroy(b->graph);
-    b->graph = nullptr;
-  }
+  batch_drop_graphs(b);
   return SMX_OK;
 }
 
 int smx_batch_graph_nodes(smx_batch* b, int64_t* nodes) {
   if (!b || !nodes) return fail(SMX_ERR_INVALID, "null argument");
   size_t n = 0;
-  if (b->graph) HIPCHK(hipGraphGetNodes(b->graph, nullptr, &n));
+  const hipGraph_t g = b->many.g ? b->many.g : b->one.g;
+  if (g) HIPCHK(hipGraphGetNodes(g, nullptr, &n));
   *nodes = (int64_t)n;
   return SMX_OK;
 }
