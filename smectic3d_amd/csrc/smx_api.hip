@@ -1318,9 +1318,9 @@ struct smx_batch {
     int64_t m = 0;
   } one, many;
   int64_t graph_steps = 0;
-  // boxes that share precision, grid and tile schedules (periodic, no advection) advance in
-  // the graph with one grouped launch per pass: member indices, and each group's GrpArgs
-  // array in device memory (built at capture, freed with the graph)
+  // boxes that batch_make_groups finds alike advance in the graphs with one grouped launch per
+  // pass: member indices, and each group's array of arguments in device memory (batch_plan,
+  // freed with the graphs)
   std::vector<std::vector<int>> groups;
   std::vector<int> single;  // the boxes of no group
   std::vector<void*> grp_args;
@@ -1373,7 +1373,7 @@ static bool same_sched(const smx_handle* a, const smx_handle* b) {
 }
 
 // Boxes that can share the grouped step kernels: periodic, no advection, same precision,
-// grid and schedules.  Groups of one box keep the single-box kernels.
+// grid, path and (four-pass steps only) schedules.  Groups of one box keep the single-box kernels.
 static void batch_make_groups(smx_batch* b, std::vector<int>& single) {
   const int n = (int)b->boxes.size();
   std::vector<bool> used(n, false);
@@ -1382,11 +1382,11 @@ static void batch_make_groups(smx_batch* b, std::vector<int>& single) {
     const smx_handle* h = b->boxes[i];
     std::vector<int> g{i};
     used[i] = true;
-    if (!h->neumann && !h->cfg.advect)  // (equal schedules and paths: equal forms)
+    if (!h->neumann && !h->cfg.advect)
       for (int j = i + 1; j < n; ++j) {
         const smx_handle* o = b->boxes[j];
         if (used[j] || o->neumann || o->cfg.advect || o->fp32 != h->fp32 || o->cfg.nx != h->cfg.nx ||
-            o->cfg.ny != h->cfg.ny || o->cfg.nz != h->cfg.nz || o->split != h->split || !same_sched(o, h))
+            o->cfg.ny != h->cfg.ny || o->cfg.nz != h->cfg.nz || o->split != h->split || !(h->split || same_sched(o, h)))
           continue;
         g.push_back(j);
         used[j] = true;
@@ -2686,7 +2686,7 @@ int smx_batch_run(smx_batch* b, int64_t nsteps, int64_t graph_steps) {
   bool stale = b->graph_steps != graph_steps || b->cap_sched.size() != b->boxes.size();
   for (size_t i = 0; !stale && i < b->boxes.size(); ++i) {  // a box's schedule or path set since the capture
     if (b->cap_split[i] != b->boxes[i]->split) stale = true;
-    for (int k = 0; k < NSLOTS; ++k)
+    for (int k = 0; k < NSLOTS && !b->boxes[i]->split; ++k)
       if (b->cap_sched[i][k].nc != b->boxes[i]->sched[k].nc || b->cap_sched[i][k].v != b->boxes[i]->sched[k].v)
         stale = true;
   }

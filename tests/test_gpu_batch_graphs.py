@@ -61,3 +61,24 @@ def test_another_stretch_captures_again():
         assert b.graph_nodes() == 18
         got = [s.get_psi() for s in b.boxes]
     check(cfgs, psis, got, 22)
+
+
+@pytest.mark.parametrize("prec", [A.SMX_FP64, A.SMX_FP32_MIXED])
+def test_tiles_of_the_four_passes_do_not_divide_a_group(prec):
+    """Boxes that step in two launches share them whatever their adjoint's tiles are: one box tuned, the
+    group and its graph stay (two launches a step in all, four grids to have tiles other than the default)."""
+    for shape in ((32, 32, 32), (64, 64, 64), (64, 96, 48), (96, 128, 64)):
+        cfgs = [cfg_reference(*shape, eps=0.5, beta=0.3, dt=0.05, nl_model=A.SMX_NL_CUBIC, precision=prec)] * 3
+        psi = O.ic_noise(*shape, 5, 0.3)
+        with Batch(cfgs) as b:
+            for s in b.boxes:
+                s.set_psi(psi)
+            b.boxes[0].autotune(3)
+            b.run(4, graph_steps=4)
+            print(shape, "nodes", b.graph_nodes(), flush=True)
+            assert b.graph_nodes() == 2 * 4
+            b.boxes[1].autotune(3)
+            b.run(4, graph_steps=4)
+            assert b.graph_nodes() == 2 * 4
+            # boxes stepped in one group from equal states stay equal
+            assert rel_l2(b.boxes[0].get_psi(), b.boxes[2].get_psi()) == 0.0
