@@ -298,7 +298,8 @@ int smx_set_schedule(smx_handle *h, const smx_schedule *s);
  * pf3d.cpp:226-291 (which times candidate FFT algorithms at set-up).  An advected Neumann
  * handle keeps its fixed tiles (the call returns them); not callable during stream capture.  On a
  * grid that steps in two launches the tuned tiles serve the adjoint's four-pass chains and *chosen is
- * the default schedule. */
+ * the default schedule; where such a handle has no adjoint (Neumann, advected or with the mid-plane
+ * penalty) nothing is timed. */
 int smx_autotune(smx_handle *h, int reps, smx_schedule *chosen);
 /* smx_autotune on every box (boxes of one shape are tuned once; advected Neumann boxes keep
  * their fixed tiles); the next smx_batch_run captures its graph again with the new schedules. */

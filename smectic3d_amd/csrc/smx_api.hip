@@ -1297,9 +1297,9 @@ static int adj_finish(smx_handle* h, double* loss, double* deps, double* dq0) {
   return SMX_OK;
 }
 
+static bool adj_covers(const smx_handle* h) { return !h->neumann && !h->cfg.advect && h->cfg.w_mid == 0.0; }
 static int adj_check(const smx_handle* h) {
-  const smx_config& c = h->cfg;
-  if (h->neumann || c.advect || c.w_mid != 0.0)
+  if (!adj_covers(h))
     return fail(SMX_ERR_UNSUPPORTED, "the adjoint covers the periodic, non-advected, penalty-free step");
   return SMX_OK;
 }
@@ -1540,6 +1540,19 @@ struct TuneKey {
 };
 static std::mutex g_tune_mu;
 static std::map<TuneKey, std::array<PassSched, NSLOTS>> g_tune_cache;
+static TuneKey tune_key(const smx_handle* h) {
+  return TuneKey{h->cfg.device, h->fp32 ? 1 : 0, h->cfg.bc, h->cfg.nx, h->cfg.ny, h->cfg.nz};
+}
+static bool tuned_tiles(const smx_handle* h, std::array<PassSched, NSLOTS>* best) {
+  std::lock_guard<std::mutex> lk(g_tune_mu);
+  const auto it = g_tune_cache.find(tune_key(h));
+  if (it == g_tune_cache.end()) return false;
+  *best = it->second;
+  return true;
+}
+// Whether some call of the handle launches four-pass kernels while its schedule is the library's choice:
+// the step of a grid without the two-launch form, and the adjoint.
+static bool auto_uses_tiles(const smx_handle* h) { return !h->split_ok || adj_covers(h); }
 
 template <typename T>
 static hipError_t launch_slot(smx_handle* h, const PParams<T>& p, int slot, PassSched s, bool dry, void* a,
@@ -2602,21 +2615,13 @@ int smx_autotune(smx_handle* h, int reps, smx_schedule* chosen) {
     return SMX_OK;
   }
   HIPCHK(hipSetDevice(h->cfg.device));
-  const TuneKey key{h->cfg.device, h->fp32 ? 1 : 0, h->cfg.bc, h->cfg.nx, h->cfg.ny, h->cfg.nz};
   std::array<PassSched, NSLOTS> best;
-  bool hit = false;
-  {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tune_cache.find(key);
-    if (it != g_tune_cache.end()) {
-      best = it->second;
-      hit = true;
-    }
-  }
-  if (!hit) {
+  if (!auto_uses_tiles(h)) {  // nothing to time
+    for (int k = 0; k < NSLOTS; ++k) best[k] = default_sched(h, k);
+  } else if (!tuned_tiles(h, &best)) {
     CHK(h->fp32 ? autotune_T<float>(h, reps, best.data()) : autotune_T<double>(h, reps, best.data()));
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    g_tune_cache[key] = best;
+    g_tune_cache[tune_key(h)] = best;
   }
   for (int k = 0; k < NSLOTS; ++k) h->sched[k] = best[k];
   h->auto_path = true;
