@@ -2604,6 +2604,10 @@ int smx_set_schedule(smx_handle* h, const smx_schedule* s) {
     const PassSched d = default_sched(h, k);
     if (c[k].nc != d.nc || c[k].v != d.v) h->auto_path = false;
   }
+  // ... and with the two-launch step the adjoint's tiles, which smx_get_schedule does not report there
+  std::array<PassSched, NSLOTS> best;
+  if (use_split(h) && auto_uses_tiles(h) && tuned_tiles(h, &best))
+    for (int k = 0; k < NSLOTS; ++k) h->sched[k] = best[k];
   return SMX_OK;
 }
 
