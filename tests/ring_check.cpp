@@ -19,7 +19,6 @@ int copies = 0, records = 0, creates = 0, mallocs = 0;
 int fail_record = -1, fail_copy = -1, fail_create = -1;  // the call that fails
 bool fail_malloc = false;
 hipMemoryType host_type = hipMemoryTypeUnregistered;
-const void* last_host = nullptr;  // the host side of the last copy
 struct Ev { size_t at = 0; };
 void run_to(size_t n) {
   for (; done < n; ++done) std::memcpy(ops[done].dst, ops[done].src, ops[done].n);
@@ -65,11 +64,10 @@ hipError_t hipStreamSynchronize(hipStream_t) {
   run_to(ops.size());
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t) {
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
   std::lock_guard<std::mutex> lk(mu);
   if (copies++ == fail_copy) return hipErrorUnknown;
   ops.push_back(Op{dst, src, n});
-  last_host = kind == hipMemcpyDeviceToHost ? dst : src;
   return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
@@ -118,6 +116,12 @@ int main(int, char** argv) {
             *f = -1;
             rc |= transfer(n, to_host, hipSuccess, k);  // the ring is free again
           }
+      }
+    } else if (what == "known") {
+      for (hipMemoryType t : {hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged}) {
+        host_type = t;
+        rc |= transfer(70000008, to_host, hipSuccess, (int)t);
+        if (copies != 1 || mallocs != 0) rc |= bad("not one copy of the runtime", 70000008, copies);
       }
     } else if (what == "nomemory") {
       fail_malloc = true;

@@ -16,10 +16,11 @@ def ring_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["bytes", "errors", "nomemory"])
+@pytest.mark.parametrize("scenario", ["bytes", "errors", "nomemory", "known"])
 def test_ring(ring_check, scenario):
     """bytes: every byte arrives, at sizes about the thresholds, with one and several workers.  errors: after a
     call of the runtime failed, no copy is in flight that still uses the slots or the caller's array.
-    nomemory: without the ring's memory the runtime's copy is taken."""
+    nomemory: without the ring's memory the runtime's copy is taken.  known: memory that the runtime knows
+    (pinned, managed, device) goes in one copy of its own."""
     r = subprocess.run([ring_check, scenario], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
