@@ -108,7 +108,8 @@ struct smx_handle {
   int64_t steps = 0;
   PassSched sched[NSLOTS];  // tile schedules of the four-pass kernels (Neumann: tile widths, variant 0)
   bool auto_path = true;    // no schedule was installed: the two-launch step where the grid has it
-  bool split_ok = false;    // the grid has the two-launch step (smx_split.h)
+  bool split_form = false;  // the grid has the split form of a state and the kernels that read it (smx_split.h)
+  bool split_ok = false;    // and steps in two launches
   bool split = false;       // A and R hold the split form
   bool prev_split = false;  // Aprev does
   // device bytes the adjoint may spend on resident record sets: -1 (default) = a share of
@@ -592,6 +593,17 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
   tm.arm(3);
   CHK(xpass<T>(h, q, X_STEP, h->A, h->A, h->R, nullptr, h->sched[SLOT_X]));
   return SMX_OK;  // the x pass projects the self-conjugate planes of R itself
+}
+
+// Whether the two-launch Neumann step is the faster one where it fits.  In FP64, 21 grids have tiles that leave
+// one block a CU in both kernels, 0.74 to 1.03 of the four passes' time.  Those behind are x lines of 256 (16
+// values and 190 registers a thread, 8.9 ns per thousand points where lines of 192 and 384 take 7.2 and 8.2):
+// 256 x 256 x 384 402 us and 390 in four passes, 256 x 384 x 192 299 and 294, 256 x 384 x 256 387 and 388, but not
+// with z lines of 512 (256 x 256 x 512 505 and 584), whose four-pass kernels have one block a CU as well.  192 x
+// 256 x 384 261 and 292, 384 x 128 x 384 280 and 302, 384 x 192 x 192 211 and 209.
+static bool nsplit_pays(bool fp32, int nx, int ny, int nz) {
+  return fp32 || !(nx == 256 && nz < 512 && nsplit_z_per_cu<double>(nx, ny, nz) == 1 &&
+                   nsplit_x_per_cu<double>(nx, ny) == 1);
 }
 
 // ---- the two forms of a state (smx_split.h, smx_split_neu.h) ----
@@ -1865,14 +1877,13 @@ int smx_create(const smx_config* cfg, smx_handle** out) {
   else if (h->neumann && !c.advect)
     h->split_ok = (h->fp32 ? nsplit_z_fits<float>(c.nx, c.ny, c.nz) && nsplit_x_fits<float>(c.nx, c.ny)
                            : nsplit_z_fits<double>(c.nx, c.ny, c.nz) && nsplit_x_fits<double>(c.nx, c.ny)) &&
-                  nsplit_real_fits(c.nx, c.ny, c.nz) &&
-                  // FP64 256 x 256 x 384: one block of 512 threads a CU in either kernel, 405 us a step and 387 in
-                  // four passes (256 x 256 x 512, 1024 threads in z: 513 and 581; 192 x 256 x 384: 265 and 288)
-                  !(!h->fp32 && c.nx == 256 && c.ny == 256 && c.nz == 384);
+                  nsplit_real_fits(c.nx, c.ny, c.nz);
   else if (!h->neumann)
     h->split_ok = h->fp32 ? split_adv_fits_z<float>(c.ny, c.nz) && split_adv_fits_x<float>(c.nx, c.ny)
                           : split_adv_fits_z<double>(c.ny, c.nz) && split_adv_fits_x<double>(c.nx, c.ny);
   if (h->split_ok && !h->neumann) h->split_ok = split_real_fits(c.ny, c.nz);
+  h->split_form = h->split_ok;
+  if (h->split_ok && h->neumann) h->split_ok = nsplit_pays(h->fp32, c.nx, c.ny, c.nz);
   for (int k = 0; k < NSLOTS; ++k) h->sched[k] = default_sched(h, k);
   auto bail = [&](int code) {
     smx_destroy(h);
@@ -2073,7 +2084,7 @@ int smx_load_checkpoint(smx_handle* h, const char* path) {
   if (in_split) {
     int64_t lay = 0;
     if (std::fread(&lay, sizeof(lay), 1, f) != 1) return bad("truncated");
-    if (!h->split_ok || lay != split_layout(h)) return bad("checkpoint of another state layout");
+    if (!h->split_form || lay != split_layout(h)) return bad("checkpoint of another state layout");
     hsh = fnv1a(hsh, &lay, sizeof(lay));
   }
   std::vector<std::vector<char>> data(arrs.size(), std::vector<char>(abytes));
@@ -2230,7 +2241,7 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   // 384 then takes 0.96 ms a call, 0.81 from a standard-form state; an FP32 copy was no faster and lost
   // the second derivatives' accuracy).
   const bool f32in = h->fp32 && h->neumann && !h->split, w0copy = h->split || (!h->neumann && h->fp32);
-  const bool w0room = h->split_ok || (!h->neumann && h->fp32);
+  const bool w0room = h->split_form || (!h->neumann && h->fp32);
   // real psi, the FP64 x stage copy, the field values at each column's evaluation index (ns
   // parts per field), the z evaluation's trigonometric table, and the crossing and evaluation
   // indices of each column

@@ -265,6 +265,15 @@ bool nsplit_z_fits(int nx, int ny, int nz) {
          }) == hipSuccess;
 }
 template <typename T>
+int nsplit_z_per_cu(int nx, int ny, int nz) {
+  int n = 0;
+  (void)split_z_dispatch(nz, nsplit_ra(ny, nx), [&](auto l, auto r) -> hipError_t {
+    n = (int)(160 * 1024 / NZ<T, decltype(l)::value, decltype(r)::value>::BYTES);
+    return hipSuccess;
+  });
+  return n;
+}
+template <typename T>
 int nsplit_z_blocks(const PParams<T>& p) {
   const int ra = nsplit_ra(p.ny, p.nx);
   int n = 0;
@@ -296,6 +305,17 @@ bool nsplit_x_fits(int nx, int ny) {
            using X = NX<T, decltype(l)::value, decltype(r)::value>;
            return X::fits && ny % X::NC == 0 ? hipSuccess : hipErrorInvalidValue;
          }) == hipSuccess;
+}
+template <typename T>
+int nsplit_x_per_cu(int nx, int ny) {
+  const int ra = nsplit_ra(ny, nx);
+  int n = 0;
+  if (ra != 0)
+    (void)split_x_dispatch(nx, ny / ra, [&](auto l, auto r) -> hipError_t {
+      n = (int)(160 * 1024 / NX<T, decltype(l)::value, decltype(r)::value>::BYTES);
+      return hipSuccess;
+    });
+  return n;
 }
 template <typename T>
 hipError_t nsplit_x(const SplitNeuArgs<T>& s, hipStream_t st) {

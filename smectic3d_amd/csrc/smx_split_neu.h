@@ -89,7 +89,8 @@ struct NZ {
   static constexpr int HP = NPR + NY2, FP = sizeof(T) == 8 ? NPR : HP;
   static constexpr int ITEMS = L / 2 * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
   static constexpr int LDS = L * HP, RED = (NT % 64 == 0) ? NT / 64 : NT;
-  static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
+  static constexpr size_t BYTES = (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8;
+  static constexpr bool fits = NT <= 1024 && BYTES <= 160 * 1024;
 };
 
 // Byte offset of an item's value k: k1 = k (P = 1), or k + H lo.
@@ -263,7 +264,8 @@ struct NX {
   static constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NC * TPC, NCP = NC + 1, NK = NC / RB;
   using AD = RowAddr<NCP>;
   static constexpr int NIT = (L / 2 + 2 * TPC - 1) / (2 * TPC);  // row pairs per thread
-  static constexpr bool fits = NT <= 1024 && (size_t)L * (NCP + 2) * sizeof(cplx<T>) + L * sizeof(T) <= 160 * 1024;
+  static constexpr size_t BYTES = (size_t)L * (NCP + 2) * sizeof(cplx<T>) + L * sizeof(T);
+  static constexpr bool fits = NT <= 1024 && BYTES <= 160 * 1024;
 };
 
 template <typename X>

@@ -3,3 +3,4 @@
 #include "smx_split_launch.h"
 template bool smx::nsplit_x_fits<double>(int, int);
 template hipError_t smx::nsplit_x<double>(const smx::SplitNeuArgs<double>&, hipStream_t);
+template int smx::nsplit_x_per_cu<double>(int, int);

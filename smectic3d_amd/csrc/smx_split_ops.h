@@ -32,6 +32,8 @@ bool split_real_fits(int ny, int nz);
 // The Neumann step's two launches, its real field and its change of form (smx_split_neu.h).
 template <typename T> bool nsplit_z_fits(int nx, int ny, int nz);
 template <typename T> bool nsplit_x_fits(int nx, int ny);
+template <typename T> int nsplit_z_per_cu(int nx, int ny, int nz);  // blocks whose tiles fit a CU (0: none)
+template <typename T> int nsplit_x_per_cu(int nx, int ny);
 template <typename T> int nsplit_z_blocks(const PParams<T>& p);
 template <typename T> hipError_t nsplit_z(const SplitNeuArgs<T>& s, hipStream_t st);
 template <typename T> hipError_t nsplit_x(const SplitNeuArgs<T>& s, hipStream_t st);
