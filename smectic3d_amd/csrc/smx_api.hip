@@ -608,9 +608,9 @@ static bool nsplit_pays(bool fp32, int nx, int ny, int nz) {
 
 // ---- the two forms of a state (smx_split.h, smx_split_neu.h) ----
 // Rows of a stage array or carry from one form to the other on the handle's stream, in place allowed.
-template <typename T, typename TI = T>
-static int form_rows(smx_handle* h, const cplx<TI>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
-  const hipError_t e = split_form<T, TI>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
+template <typename T>
+static int form_rows(smx_handle* h, const cplx<T>* in, cplx<T>* out, int dir, const T* kmul = nullptr) {
+  const hipError_t e = split_form<T>(in, out, h->npencils, h->cfg.ny, tables<T>(h).twy, dir, kmul, h->st);
   if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
   return SMX_OK;
 }
@@ -664,7 +664,9 @@ static int stage_to_f64(smx_handle* h, const void* stage, void* dst, bool split)
                    : nform_rows<double, double>(h, stage, dst, FORM_TO_STD);
   if (h->fp32) {
     if (split) {
-      CHK((form_rows<double, float>(h, (const cplx<float>*)stage, (cplx<double>*)dst, FORM_TO_STD)));
+      const hipError_t e = split_form_std<double, float>((const cplx<float>*)stage, (cplx<double>*)dst, h->npencils,
+                                                         h->cfg.ny, h->t64.twy, h->st);
+      if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("state form: ") + hipGetErrorString(e));
     } else {
       hipLaunchKernelGGL(k_f32_to_f64, dim3(kRedBlocks), dim3(kRedThreads), 0, h->st, (const float*)stage,
                          (double*)dst, ncomp);

@@ -40,6 +40,9 @@ hipError_t split_x_dispatch(int nx, int rb, F&& f) {
   return hipErrorInvalidValue;
 }
 
+// The y lengths with a division (split_ra, nsplit_ra).
+#define SMX_FOR_EACH_SPLIT(X) X(16) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384)
+
 // Blocks that project the carry: 8 pairs' entries per thread.
 template <typename Z, typename T>
 static int split_nproj(const PParams<T>& p) {
@@ -232,25 +235,36 @@ hipError_t split_x_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, hip
     }
   });
 }
-template <typename T, int RB, typename TI>
-static void split_form_launch(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
-                              const T* kmul, hipStream_t st) {
+template <typename T, typename TI>
+hipError_t split_form_std(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy,
+                          hipStream_t st) {
+  if (nrows < 1) return hipErrorInvalidValue;
+#define SMX_CASE(NY)                                                                                         \
+  if (ny == NY) {                                                                                            \
+    constexpr int RA = split_ra(NY), ROWS = 256 / RA;                                                        \
+    SMX_LAUNCH((k_form_std<T, RA, NY / RA, TI>), dim3((unsigned)((nrows + ROWS - 1) / ROWS)), dim3(256), 0, st, in, \
+               out, nrows, twy);                                                                             \
+    return hipGetLastError();                                                                                \
+  }
+  SMX_FOR_EACH_SPLIT(SMX_CASE)
+#undef SMX_CASE
+  return hipErrorInvalidValue;
+}
+template <typename T>
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+                      const T* kmul, hipStream_t st) {
+  if (dir == FORM_TO_STD) return kmul == nullptr ? split_form_std<T, T>(in, out, nrows, ny, twy, st) : hipErrorInvalidValue;
+  const int ra = split_ra(ny);
+  if (ra == 0 || nrows < 1) return hipErrorInvalidValue;
   const int rows = 1024 / ny;
   const dim3 grid((unsigned)((nrows + rows - 1) / rows));
-  SMX_LAUNCH((k_form<T, RB, TI>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul);
-}
-template <typename T, typename TI>
-hipError_t split_form(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
-                      const T* kmul, hipStream_t st) {
-  const int ra = split_ra(ny);
-  if (ra == 0) return hipErrorInvalidValue;
+#define SMX_CASE(RB)                                                                                            \
+  case RB: SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul); break;
   switch (ny / ra) {
-    case 4: split_form_launch<T, 4, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 8: split_form_launch<T, 8, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 12: split_form_launch<T, 12, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
-    case 16: split_form_launch<T, 16, TI>(in, out, nrows, ny, twy, dir, kmul, st); break;
+    SMX_CASE(4) SMX_CASE(8) SMX_CASE(12) SMX_CASE(16)
     default: return hipErrorInvalidValue;
   }
+#undef SMX_CASE
   return hipGetLastError();
 }
 #endif
@@ -356,11 +370,30 @@ hipError_t nsplit_real(const cplx<TI>* a, double* out, const PParams<double>& p,
     }
   });
 }
+template <typename TI, typename TO, int NY, int RA>
+static hipError_t nsplit_form_std(const TI* in, TO* out, int nx, int nz, const cplx<double>* twy,
+                                  const cplx<double>* qty, hipStream_t st) {
+  constexpr int ROWS = 128 / RA;
+  SMX_LAUNCH((k_nform_std<TI, TO, RA, NY / RA>), dim3((unsigned)((nx * (nz / 2) + ROWS - 1) / ROWS)), dim3(128), 0, st,
+             in, out, nx, nz, twy, qty);
+  return hipGetLastError();
+}
 template <typename TI, typename TO>
 hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
                        int dir, hipStream_t st) {
   const int ra = nsplit_ra(ny, nx);
   if (ra == 0) return hipErrorInvalidValue;
+  if (dir == FORM_TO_STD) {
+#define SMX_CASE(NY)                                                                                              \
+  if (ny == NY) {                                                                                                 \
+    constexpr int R0 = nsplit_ra(NY, 1), R3 = nsplit_ra(NY, 3);                                                   \
+    return ra == R0 ? nsplit_form_std<TI, TO, NY, R0>(in, out, nx, nz, twy, qty, st)                              \
+                    : nsplit_form_std<TI, TO, NY, R3>(in, out, nx, nz, twy, qty, st);                             \
+  }
+    SMX_FOR_EACH_SPLIT(SMX_CASE)
+#undef SMX_CASE
+    return hipErrorInvalidValue;
+  }
   const int rows = 1024 / ny;
   const dim3 grid((unsigned)((nx * (nz / 2) + rows - 1) / rows));
 #define SMX_CASE(RB)                                                                                           \

@@ -405,8 +405,60 @@ __global__ __launch_bounds__(X::NT) void k_nsplit_x(SplitNeuArgs<typename X::T> 
 }
 
 // ---------------------------------------------------------------------------
-// Between the two forms, out of place, in FP64; whole rows (j, x) per block of 256 threads, an item the RB
-// values of one row and k1 (as k_form).
+// Between the two forms, out of place, in FP64.  Rows (j, x) of the split form, two planes of the standard one.
+// To standard as k_form_std, but with the lines' untangling from LDS (ky and ny - ky of a row are two threads')
+// and real rows stored 8 bytes a lane (256 x 256 x 384 from FP32: 151 -> 67 us).
+template <typename TI, typename TO, int RA, int RB>
+__global__ __launch_bounds__(128) void k_nform_std(const TI* __restrict__ in, TO* __restrict__ out, int nx, int nz,
+                                                   const cplx<double>* __restrict__ twy,
+                                                   const cplx<double>* __restrict__ qty) {
+  using C = cplx<double>;
+  constexpr int NT = 128, NY = RA * RB, ROWS = NT / RA, N = ROWS * NY, YC = kSplitYC;
+  __shared__ C S[N + N / 16];
+  __shared__ C TW[NY];
+  __shared__ int64_t PL[ROWS][2];  // where the two planes' rows are
+  auto at = [](int i) { return i + (i >> 4); };
+  const int tid = threadIdx.x, row = tid / RA, k1 = tid - row * RA;
+  const int nrows = nx * (nz / 2), r0 = blockIdx.x * ROWS, nr = nrows - r0 < ROWS ? nrows - r0 : ROWS;
+  const bool item = row < nr;
+  C w[RB];
+  if (item) {
+    const cplx<TI>* src = reinterpret_cast<const cplx<TI>*>(in) + (int64_t)(r0 + row) * NY + nsplit_pos(k1, 0, RA, RB);
+#pragma unroll
+    for (int c = 0; c < RB; c += 2) {
+      const cplx2<TI> g = *reinterpret_cast<const cplx2<TI>*>(src + c / YC * 2 * YC + c % YC);
+      w[c] = mk((double)g.a.x, (double)g.a.y);
+      w[c + 1] = mk((double)g.b.x, (double)g.b.y);
+    }
+  }
+  tw_lds<NY, NT>(TW, twy, tid);
+  if (tid < nr) {
+    const int j = (r0 + tid) / nx, x = r0 + tid - j * nx;
+    PL[tid][0] = ((int64_t)j * nx + x) * NY;
+    PL[tid][1] = ((int64_t)(j == 0 ? nz / 2 : nz - j) * nx + x) * NY;
+  }
+  __syncthreads();
+  if (item) {
+#pragma unroll
+    for (int c = 1; c < RB; ++c) w[c] = cmul(w[c], TW[k1 * c]);
+    dft<RB, -1>(w);
+#pragma unroll
+    for (int c = 0; c < RB; ++c) S[at(row * NY + k1 + RA * c)] = (0.5 / RB) * w[c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < (N + NT - 1) / NT; ++u) {
+    const int i = tid + u * NT, rr = i / NY, c = i - rr * NY;
+    if (rr < nr) {
+      const C y = dct2_out(S[at(i)], S[at(rr * NY + (c == 0 ? 0 : NY - c))], qty[c]);
+      out[PL[rr][0] + c] = (TO)y.x;
+      out[PL[rr][1] + c] = (TO)y.y;
+    }
+  }
+}
+
+// From standard and the carry's orders; whole rows per block of 256 threads, an item the RB values of one row
+// and k1 (as k_form).
 template <typename TI, typename TO, int RB>
 __global__ __launch_bounds__(256) void k_nform(const TI* __restrict__ in, TO* __restrict__ out, int nx, int ny, int nz,
                                                const cplx<double>* __restrict__ twy,
@@ -439,11 +491,9 @@ __global__ __launch_bounds__(256) void k_nform(const TI* __restrict__ in, TO* __
     }
     return;
   }
-  const bool from = dir == FORM_FROM_STD;
   for (int i = tid; i < n; i += 256) {
     const int r = r0 + i / ny, c = i % ny;
-    const int64_t o = 2 * ((int64_t)r * ny + c);
-    S[at(i)] = from ? mk((double)in[plane(r, 0) + c], (double)in[plane(r, 1) + c]) : mk((double)in[o], (double)in[o + 1]);
+    S[at(i)] = mk((double)in[plane(r, 0) + c], (double)in[plane(r, 1) + c]);
   }
   __syncthreads();
   const int row = tid / ra, k1 = tid - row * ra;
@@ -453,36 +503,23 @@ __global__ __launch_bounds__(256) void k_nform(const TI* __restrict__ in, TO* __
 #pragma unroll
     for (int c = 0; c < RB; ++c) {
       const int k = k1 + ra * c;
-      w[c] = from ? dct3_in(S[at(row * ny + k)], k == 0 ? mk<double>(0, 0) : S[at(row * ny + ny - k)], qty[k])
-                  : cmul(S[at(row * ny + nsplit_pos(k1, c, ra, RB))], twy[k1 * c]);
+      w[c] = dct3_in(S[at(row * ny + k)], k == 0 ? mk<double>(0, 0) : S[at(row * ny + ny - k)], qty[k]);
     }
-    if (from) {
-      dft<RB, +1>(w);
+    dft<RB, +1>(w);
 #pragma unroll
-      for (int c = 0; c < RB; ++c) w[c] = cmul(w[c], conjg(twy[k1 * c]));
-    } else {
-      dft<RB, -1>(w);
-#pragma unroll
-      for (int c = 0; c < RB; ++c) w[c] = (1.0 / RB) * w[c];
-    }
+    for (int c = 0; c < RB; ++c) w[c] = cmul(w[c], conjg(twy[k1 * c]));
   }
   __syncthreads();
   if (item) {
 #pragma unroll
-    for (int c = 0; c < RB; ++c) S[at(row * ny + (from ? nsplit_pos(k1, c, ra, RB) : k1 + ra * c))] = w[c];
+    for (int c = 0; c < RB; ++c) S[at(row * ny + nsplit_pos(k1, c, ra, RB))] = w[c];
   }
   __syncthreads();
   for (int i = tid; i < n; i += 256) {
     const int rr = i / ny, r = r0 + rr, c = i - rr * ny;
-    if (from) {
-      const int64_t o = 2 * ((int64_t)r * ny + c);
-      out[o] = (TO)S[at(i)].x;
-      out[o + 1] = (TO)S[at(i)].y;
-    } else {
-      const C y = dct2_out(S[at(i)], S[at(rr * ny + (c == 0 ? 0 : ny - c))], qty[c]);
-      out[plane(r, 0) + c] = (TO)(0.5 * y.x);
-      out[plane(r, 1) + c] = (TO)(0.5 * y.y);
-    }
+    const int64_t o = 2 * ((int64_t)r * ny + c);
+    out[o] = (TO)S[at(i)].x;
+    out[o + 1] = (TO)S[at(i)].y;
   }
 }
 

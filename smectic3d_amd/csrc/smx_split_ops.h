@@ -44,9 +44,13 @@ template <typename TI, typename TO>
 hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
                        int dir, hipStream_t st);
 // Rows of a stage array (or, with the perm directions, of the carry) between the two forms, in place
-// allowed (TI = T).  kmul: k_y table of the d/dy of a standard-form input, or nullptr.
-template <typename T, typename TI = T>
-hipError_t split_form(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
+// allowed.  kmul: k_y table of the d/dy of a standard-form input, or nullptr.
+template <typename T>
+hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
                       const T* kmul, hipStream_t st);
+// To the standard form from rows of type TI (in place allowed for TI = T).
+template <typename T, typename TI>
+hipError_t split_form_std(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy,
+                          hipStream_t st);
 
 }  // namespace smx
