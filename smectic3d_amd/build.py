@@ -22,7 +22,7 @@ UNITS = ["smx_inst_f32.hip", "smx_inst_f64.hip", "smx_api.hip", "smx_split_z_f32
          "smx_split_x_f32.hip", "smx_split_x_f64.hip", "smx_split_real.hip", "smx_split_adv_z_f32.hip",
          "smx_split_adv_z_f64.hip", "smx_split_adv_x_f32.hip", "smx_split_adv_x_f64.hip",
          "smx_split_neu_z_f32.hip", "smx_split_neu_z_f64.hip", "smx_split_neu_x_f32.hip", "smx_split_neu_x_f64.hip",
-         "smx_split_neu_real.hip"]
+         "smx_split_neu_real.hip", "smx_split_surf_f32.hip", "smx_split_surf_f64.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", INCLUDE]

@@ -2239,9 +2239,8 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   const int ns = surf_nsplit(h->neumann, h->cfg.nx, h->cfg.nz);
   // An FP64 state is its own x stage, and an FP32 Neumann stage is read as it is (widened on
   // load); a periodic FP32 stage is copied to FP64 and projected (stage_to_f64) first.
-  // A split-form state is brought to the standard form there, in FP64 (an FP32 Neumann box of 256 x 256 x
-  // 384 then takes 0.96 ms a call, 0.81 from a standard-form state; an FP32 copy was no faster and lost
-  // the second derivatives' accuracy).
+  // A split-form state is brought to the standard form there, in FP64, for the multipliers (an FP32 copy would
+  // lose the second derivatives' accuracy); psi comes from the state itself.
   const bool f32in = h->fp32 && h->neumann && !h->split, w0copy = h->split || (!h->neumann && h->fp32);
   const bool w0room = h->split_form || (!h->neumann && h->fp32);
   // real psi, the FP64 x stage copy, the field values at each column's evaluation index (ns
@@ -2264,7 +2263,7 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   int* kev = kcol + nxy;
   PParams<double> p = params<double>(h, false);
   const DevTables<double>& t = h->t64;
-  // psi into f (through its y inverse in D1) and, where an x multiplier needs it, psi_hat into D2:
+  // psi into f and, where an x multiplier needs it, psi_hat into D2:
   // the plain Neumann step's two (the rate and psi_xx) are applied from the x stage itself
   // (X_MUL2, below)
   const void* x_stage = h->A;
@@ -2276,32 +2275,44 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
   // itself is not needed
   const bool xmul2 = !h->cfg.advect;
   const double xscale = h->neumann ? 0.5 / (double)h->cfg.nx : 1.0 / (double)h->cfg.nx;  // undo the x inverse
-  {
+  if (!xmul2) {
     PParams<double> px = p;
     px.scale = xscale;
-    if (f32in) {
-      hipError_t e = xmul2 ? hipSuccess : surf_dct_xfwd_f32((const float*)x_stage, (double*)h->D2, px, t.qtwx, h->st);
-      if (e == hipSuccess)
-        e = surf_dct_yinv_f32((const float*)x_stage, (double*)h->D1, h->cfg.ny, h->npencils, t.twy, t.qtwy, h->st);
-      if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("surfTrack transforms: ") + hipGetErrorString(e));
-    } else {
-      if (!xmul2) CHK(xpass<double>(h, px, X_FWD_SCALED, x_stage, h->D2, nullptr, nullptr));
-      CHK(ypass<double>(h, x_stage, h->D1, +1));
-    }
+    const hipError_t e = f32in ? surf_dct_xfwd_f32((const float*)x_stage, (double*)h->D2, px, t.qtwx, h->st) : hipSuccess;
+    if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("surfTrack transforms: ") + hipGetErrorString(e));
+    if (!f32in) CHK(xpass<double>(h, px, X_FWD_SCALED, x_stage, h->D2, nullptr, nullptr));
   }
   // psi, the crossing of every column and the index its fields are taken at; a grid whose z
   // blocks are whole waves also gets psi_zz (Neumann) or psi_z (periodic) there from the same
-  // pass (k_dct_zinv_scan, k_zinv_scan)
-  bool zfused = false;
-  {
-    hipError_t e =
-        h->neumann ? surf_dct_zinv_scan((const double*)h->D1, f, nxy, h->cfg.nz, t.twz, t.qtwz, t.kz, trig, opts->arm,
-                                        kcol, kev, ns, val + (size_t)SV_DZZ * ns * nxy, h->st)
-                   : surf_zinv_scan((const cplx<double>*)h->D1, f, nxy, h->cfg.nz, t.twz, t.kz, trig, opts->arm, kcol,
-                                    kev, ns, val + (size_t)SV_GZ * ns * nxy, h->st);
-    if (e == hipSuccess) zfused = true;
-    else if (e != hipErrorNotSupported) return fail(SMX_ERR_HIP, std::string("surfTrack z pass: ") + hipGetErrorString(e));
+  // pass: from the split form itself (k_nsplit_scan, k_zsplit_scan), or from the y inverse of the standard one
+  // in D1 (k_dct_zinv_scan, k_zinv_scan)
+  double* dz = val + (size_t)(h->neumann ? SV_DZZ : SV_GZ) * ns * nxy;
+  hipError_t ze = hipErrorNotSupported;
+  if (h->split) {
+    const SplitScan sc{f, trig, opts->arm, kcol, kev, ns, dz};
+    if (h->neumann)
+      ze = h->fp32 ? nsplit_scan_surf<float>((const cplx<float>*)h->A, p, t.qtwz, sc, h->st)
+                   : nsplit_scan_surf<double>((const cplx<double>*)h->A, p, t.qtwz, sc, h->st);
+    else
+      ze = h->fp32 ? split_scan_surf<float>((const cplx<float>*)h->A, p, sc, h->st)
+                   : split_scan_surf<double>((const cplx<double>*)h->A, p, sc, h->st);
   }
+  if (ze == hipErrorNotSupported) {
+    if (f32in) {
+      const hipError_t e =
+          surf_dct_yinv_f32((const float*)x_stage, (double*)h->D1, h->cfg.ny, h->npencils, t.twy, t.qtwy, h->st);
+      if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("surfTrack transforms: ") + hipGetErrorString(e));
+    } else {
+      CHK(ypass<double>(h, x_stage, h->D1, +1));
+    }
+    ze = h->neumann ? surf_dct_zinv_scan((const double*)h->D1, f, nxy, h->cfg.nz, t.twz, t.qtwz, t.kz, trig, opts->arm,
+                                         kcol, kev, ns, dz, h->st)
+                    : surf_zinv_scan((const cplx<double>*)h->D1, f, nxy, h->cfg.nz, t.twz, t.kz, trig, opts->arm, kcol,
+                                     kev, ns, dz, h->st);
+  }
+  const bool zfused = ze == hipSuccess;
+  if (!zfused && ze != hipErrorNotSupported)
+    return fail(SMX_ERR_HIP, std::string("surfTrack z pass: ") + hipGetErrorString(ze));
   const unsigned blocks = (unsigned)((nxy + 255) / 256);
   if (!zfused) {
     CHK(zpass<double>(h, p, Z_IN_SPEC, Z_OUT_REAL, Z_OP_ID, h->D1, nullptr, nullptr, f));

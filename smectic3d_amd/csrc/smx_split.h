@@ -206,14 +206,14 @@ __device__ __forceinline__ uint32_t zs_leg(int k, uint32_t step, uint32_t cb) {
 // Inverse half: radix RA over k1 of the tile's rows and the C2R along z; v receives (psi_a, psi_b) of
 // the column pair q at z = pos_in<inv_last>.  TI: type of the stage array (float: widened).  kzm: k_z
 // table of the spectral d/dz (rows times i k_z, Nyquist +pi/dz, pf3d.cpp:184), or nullptr.  twg: the
-// z twiddles in memory, copied to twl behind the tile's loads, or nullptr if they are there.
+// z twiddles in memory, copied to twl behind the tile's loads, or nullptr if they are there.  w receives the
+// thread's items: the lines' half spectra along z.
 template <typename Z, typename TI, typename T = typename Z::T>
-__device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F,
-                                           const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v,
-                                           const T* kzm = nullptr, const cplx<T>* twg = nullptr) {
-  constexpr int L = Z::L, RA = Z::RA;
+__device__ __forceinline__ void zs_inverse_w(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F,
+                                             const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v,
+                                             cplx<T> (&w)[Z::IPT][Z::H], const T* kzm, const cplx<T>* twg) {
+  constexpr int L = Z::L;
   constexpr uint32_t CB = sizeof(cplx<TI>);
-  cplx<T> w[Z::IPT][Z::H];
 #pragma unroll
   for (int it = 0; it < Z::IPT; ++it) {  // every load is issued before the first is used
     const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, m = i / Z::P / Z::NY2;
@@ -257,12 +257,19 @@ __device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, i
     v[e] = F[Tile<T, L, Z::E, Z::HP>::template pos_in<inv_first<L, Z::V>()>(tc, e) * Z::HP + q];
   InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
 }
+template <typename Z, typename TI, typename T = typename Z::T>
+__device__ __forceinline__ void zs_inverse(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F,
+                                           const cplx<T>* twl, int tid, int q, int tc, cplx<T>* v,
+                                           const T* kzm = nullptr, const cplx<T>* twg = nullptr) {
+  cplx<T> w[Z::IPT][Z::H];
+  zs_inverse_w<Z, TI>(src, rowb, rb, F, twl, tid, q, tc, v, w, kzm, twg);
+}
 
 // Forward half: the R2C along z of the pairs in v and radix RA over y1 of the half spectra.
 template <typename Z, typename T = typename Z::T>
 __device__ __forceinline__ void zs_forward(cplx<T>* v, cplx<T>* dst, uint32_t rowb, int rb, cplx<T>* F,
                                            const cplx<T>* twl, int tid, int q, int tc) {
-  constexpr int L = Z::L, RA = Z::RA;
+  constexpr int L = Z::L;
   constexpr uint32_t CB = sizeof(cplx<T>);
   FwdFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
   __syncthreads();

@@ -345,10 +345,42 @@ hipError_t nsplit_x(const SplitNeuArgs<T>& s, hipStream_t st) {
 }
 #endif
 
-#ifdef SMX_SPLIT_NEU_REAL
+#if defined(SMX_SPLIT_NEU_REAL) || defined(SMX_SPLIT_SURF)
 // FP64 tiles also of the grids whose FP32 step fits: one y2 where two do not.
 template <int L, int RA>
 using NZReal = NZ<double, L, RA, NZ<double, L, RA>::fits ? nsplit_ny2<double>(L, RA) : 1>;
+#endif
+
+#ifdef SMX_SPLIT_SURF
+template <typename TI>
+hipError_t split_scan_surf(const cplx<TI>* a, const PParams<double>& p, const SplitScan& s, hipStream_t st) {
+  return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
+    using Z = ZS<double, decltype(l)::value, decltype(r)::value>;
+    if constexpr (!split_scan_fits<Z, 2>()) {
+      return hipErrorNotSupported;
+    } else {
+      SMX_LAUNCH((k_zsplit_scan<Z, TI>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, a, p, s);
+      return hipGetLastError();
+    }
+  });
+}
+template <typename TI>
+hipError_t nsplit_scan_surf(const cplx<TI>* a, const PParams<double>& p, const cplx<double>* qtz, const SplitScan& s,
+                            hipStream_t st) {
+  return split_z_dispatch(p.nz, nsplit_ra(p.ny, p.nx), [&](auto l, auto r) -> hipError_t {
+    using Z = NZReal<decltype(l)::value, decltype(r)::value>;
+    if constexpr (!split_scan_fits<Z, 4>()) {
+      return hipErrorNotSupported;
+    } else {
+      SMX_LAUNCH((k_nsplit_scan<Z, TI>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, a, p, qtz,
+                 s);
+      return hipGetLastError();
+    }
+  });
+}
+#endif
+
+#ifdef SMX_SPLIT_NEU_REAL
 bool nsplit_real_fits(int nx, int ny, int nz) {
   const int ra = nsplit_ra(ny, nx);
   return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {

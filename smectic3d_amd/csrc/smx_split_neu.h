@@ -114,14 +114,14 @@ __device__ __forceinline__ void nz_twiddles(const cplx<T>* __restrict__ qtz, int
 }
 
 // Inverse half: radix RA over k1 of the tile's rows and the DCT-III along z; v receives (psi_a, psi_b) of
-// column pair q at z = src(pos_in<inv_last>).  The z twiddles go to twl behind the tile's loads.
+// column pair q at z = src(pos_in<inv_last>).  The z twiddles go to twl behind the tile's loads.  w receives
+// the thread's items: the lines' cosine coefficients along z at a pair of kz.
 template <typename Z, typename TI, typename T = typename Z::T>
-__device__ __forceinline__ void nz_inverse(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F, cplx<T>* TW,
-                                           const cplx<T>* __restrict__ twg, const cplx<T> (*qw)[2], int tid, int q,
-                                           int tc, cplx<T>* v) {
+__device__ __forceinline__ void nz_inverse_w(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F, cplx<T>* TW,
+                                             const cplx<T>* __restrict__ twg, const cplx<T> (*qw)[2], int tid, int q,
+                                             int tc, cplx<T>* v, cplx<T> (&w)[Z::IPT][Z::H]) {
   constexpr int L = Z::L;
   constexpr uint32_t CB = sizeof(cplx<TI>);
-  cplx<T> w[Z::IPT][Z::H];
 #pragma unroll
   for (int it = 0; it < Z::IPT; ++it) {  // every load is issued before the first is used
     const int i = tid + it * Z::NT, lo = i % Z::P, c = i / Z::P % Z::NY2, j = i / Z::P / Z::NY2;
@@ -156,6 +156,13 @@ __device__ __forceinline__ void nz_inverse(const cplx<TI>* src, uint32_t rowb, i
 #pragma unroll
   for (int e = 0; e < Z::E; ++e) v[e] = F[Tile<T, L, Z::E, Z::HP>::template pos_in<inv_first<L, Z::V>()>(tc, e) * Z::HP + q];
   InvFFT<T, L, Z::FP, Z::V>::run(v, F, q, tc, twl);
+}
+template <typename Z, typename TI, typename T = typename Z::T>
+__device__ __forceinline__ void nz_inverse(const cplx<TI>* src, uint32_t rowb, int rb, cplx<T>* F, cplx<T>* TW,
+                                           const cplx<T>* __restrict__ twg, const cplx<T> (*qw)[2], int tid, int q,
+                                           int tc, cplx<T>* v) {
+  cplx<T> w[Z::IPT][Z::H];
+  nz_inverse_w<Z, TI>(src, rowb, rb, F, TW, twg, qw, tid, q, tc, v, w);
 }
 
 // Forward half: the DCT-II along z of the pairs in v and radix RA over y1.

@@ -3,6 +3,7 @@
 #pragma once
 #include "smx_split_adv.h"
 #include "smx_split_neu.h"
+#include "smx_split_surf.h"
 
 namespace smx {
 
@@ -29,6 +30,13 @@ template <typename T> hipError_t split_adv_stokes(const SplitAdvArgs<T>& s, hipS
 template <typename T> hipError_t split_adv_advnl(const SplitAdvArgs<T>& s, hipStream_t st);
 template <typename T> hipError_t split_adv_update(const SplitAdvArgs<T>& s, hipStream_t st);
 bool split_real_fits(int ny, int nz);
+// surfTrack's psi, scan and z derivative from a split-form stage array (smx_split_surf.h); hipErrorNotSupported
+// for a grid whose tile does not take it.
+template <typename TI>
+hipError_t split_scan_surf(const cplx<TI>* a, const PParams<double>& p, const SplitScan& s, hipStream_t st);
+template <typename TI>
+hipError_t nsplit_scan_surf(const cplx<TI>* a, const PParams<double>& p, const cplx<double>* qtz, const SplitScan& s,
+                            hipStream_t st);
 // The Neumann step's two launches, its real field and its change of form (smx_split_neu.h).
 template <typename T> bool nsplit_z_fits(int nx, int ny, int nz);
 template <typename T> bool nsplit_x_fits(int nx, int ny);
