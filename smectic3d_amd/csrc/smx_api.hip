@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -2343,10 +2344,15 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
     HIPCHK(hipGetLastError());
     return SMX_OK;
   };
-  auto ypoint = [&](const void* xs, int ykop, int slot) -> int {
-    hipError_t e = surf_ypoint(h->neumann, xs == x_stage && f32in, xs, kev, h->cfg.nx, h->cfg.ny, h->cfg.nz, ns, t.twy, t.qtwy,
-                               ykop >= 0 ? t.ky : nullptr, ykop, t.kz, -1, trig, val + (size_t)slot * ns * nxy,
-                               h->st);
+  // fields from x stages of one type in one launch: their blocks fill the chip together
+  auto field = [&](const void* xs, int ykop, int slot) {
+    return YPoint{xs, ykop >= 0 ? t.ky : nullptr, ykop, val + (size_t)slot * ns * nxy};
+  };
+  auto ypoint = [&](std::initializer_list<YPoint> fs) -> int {
+    YPoints ys = {};
+    std::copy(fs.begin(), fs.end(), ys.f);
+    const hipError_t e = surf_ypoint(h->neumann, f32in && fs.begin()->in == x_stage, ys, (int)fs.size(), kev, h->cfg.nx,
+                                     h->cfg.ny, h->cfg.nz, ns, t.twy, t.qtwy, t.kz, -1, trig, h->st);
     if (e != hipSuccess) return fail(SMX_ERR_HIP, std::string("surfTrack field values: ") + hipGetErrorString(e));
     return SMX_OK;
   };
@@ -2355,9 +2361,9 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
     pk.kop = mode;
     return xpass<double>(h, pk, X_INV, spec, h->D1, nullptr, nullptr);
   };
-  auto along_y = [&](int mode, int slot) -> int { return ypoint(x_stage, mode, slot); };
-  // two x multipliers from the x stage in one pass (X_MUL2) into D1 and D2, then their values
-  auto x_pair = [&](int op1, int slot1, int op2, int slot2) -> int {
+  // two x multipliers from the x stage in one pass (X_MUL2) into D1 and D2, then their values and those of
+  // one with a k_y multiplier
+  auto x_pair = [&](int op1, int slot1, int op2, int slot2, int yop, int yslot) -> int {
     PParams<double> pm = p;
     pm.scale = xscale;
     pm.kop = op1;
@@ -2369,12 +2375,14 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
     } else {
       CHK(xpass<double>(h, pm, X_MUL2, x_stage, h->D1, h->D2, nullptr));
     }
-    CHK(ypoint(h->D1, -1, slot1));
-    return ypoint(h->D2, -1, slot2);
+    const YPoint f1 = field(h->D1, -1, slot1), f2 = field(h->D2, -1, slot2), fy = field(x_stage, yop, yslot);
+    if (!f32in) return ypoint({f1, f2, fy});
+    CHK(ypoint({f1, f2}));
+    return ypoint({fy});
   };
   auto along_x = [&](int mode, int slot) -> int {
     CHK(x_inv(mode, h->D2));
-    return ypoint(h->D1, -1, slot);
+    return ypoint({field(h->D1, -1, slot)});
   };
   // psi_zz (Neumann, cosNoAdvMorphCurv.cpp:750) or psi_z (periodic, surfTrack.cpp:611-626) first:
   // the first x inverse overwrites psi's y inverse in D1
@@ -2387,27 +2395,22 @@ int smx_surftrack(smx_handle* h, const smx_surf_opts* opts, double* surfz, doubl
     CHK(advected_n_spectrum(h));
     CHK(kmul(h, KM_DTPSI, h->D2, h->D1));
     CHK(x_inv(-1, h->D1));
-    CHK(ypoint(h->D1, -1, SV_RATE));
-  } else {
-    CHK(x_pair(KM_ALIN, SV_RATE, KM_DXX, SV_DXX));
+    CHK(ypoint({field(h->D1, -1, SV_RATE)}));
   }
-  if (!h->neumann) {
-    // spectral gradient, psi_xx, psi_yy, psi_xy (surfTrack.cpp:611-626); psi_xx + psi_yy is the
-    // sum of the two at the crossing (k_surf_periodic)
-    if (xmul2) {
-      CHK(x_pair(KM_IKX, SV_GX, KM_DXY, SV_DXY));
-    } else {
-      CHK(along_x(KM_IKX, SV_GX));
-      CHK(along_x(KM_DXX, SV_DXX));
-      CHK(along_x(KM_DXY, SV_DXY));
-    }
-    CHK(along_y(KM_IKY, SV_GY));
-    CHK(along_y(KM_DYY, SV_DYY));
+  // The others: the spectral gradient, psi_xx, psi_yy and psi_xy in a periodic box (surfTrack.cpp:611-626; psi_xx
+  // + psi_yy is the sum of the two at the crossing, k_surf_periodic), psi_xx, psi_yy and psi_zz in a Neumann one
+  // (cosNoAdvMorphCurv.cpp:746-750)
+  if (xmul2) {
+    CHK(x_pair(KM_ALIN, SV_RATE, KM_DXX, SV_DXX, KM_DYY, SV_DYY));
+    if (!h->neumann) CHK(x_pair(KM_IKX, SV_GX, KM_DXY, SV_DXY, KM_IKY, SV_GY));
+  } else if (h->neumann) {
+    CHK(along_x(KM_DXX, SV_DXX));
+    CHK(ypoint({field(x_stage, KM_DYY, SV_DYY)}));
   } else {
-    // psi_xx, psi_yy, psi_zz (spectral, cosNoAdvMorphCurv.cpp:746-750; psi_xx with the rate above
-    // unless advected)
-    if (!xmul2) CHK(along_x(KM_DXX, SV_DXX));
-    CHK(along_y(KM_DYY, SV_DYY));
+    CHK(along_x(KM_IKX, SV_GX));
+    CHK(along_x(KM_DXX, SV_DXX));
+    CHK(along_x(KM_DXY, SV_DXY));
+    CHK(ypoint({field(x_stage, KM_IKY, SV_GY), field(x_stage, KM_DYY, SV_DYY)}));
   }
   HIPCHK(hipMemsetAsync(h->flag, 0, sizeof(unsigned int), h->st));
   SurfParams sp;

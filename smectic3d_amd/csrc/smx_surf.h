@@ -20,12 +20,12 @@ namespace smx {
 // kz splits of one evaluation: block (x, s) sums kz units [s U / ns, (s+1) U / ns) (U: pencil
 // pairs for the Neumann kernel, spectral planes for the periodic one) and writes its part of
 // every column of that x to out[s nxy + c]; the tail kernels add the ns parts in split order.
-// Enough splits for about 1024 blocks (more splits repeat each block's set-up for fewer rounds
+// Enough splits for about 512 blocks a field (more splits repeat each block's set-up for fewer rounds
 // of pencils), at most kSurfMaxSplit and at most U.
 constexpr int kSurfMaxSplit = 16;
 inline int surf_nsplit(bool neu, int nx, int nz) {
   const int units = neu ? (nz + 1) / 2 : nz / 2 + 1;
-  return std::max(1, std::min({kSurfMaxSplit, units, (1024 + nx - 1) / nx}));
+  return std::max(1, std::min({kSurfMaxSplit, units, (512 + nx - 1) / nx}));
 }
 
 // Trigonometric tables of the z evaluation, one per grid (4 nz doubles): Neumann
@@ -106,6 +106,21 @@ __global__ __launch_bounds__(256) void k_surf_point(const double* __restrict__ s
   }
 }
 
+// The fields of one launch of the evaluation kernels: x stages, k_y multipliers (kq: the k_y table, kop;
+// nullptr and -1 without one) and where their values go.  Three at once take half the splits that one at a
+// time needs to fill the chip: 222 -> 194 us for three at 256 x 256 x 384 Neumann, 118 -> 98 at 256^3 and 78 -> 54
+// at 192 x 96 x 384 periodic.
+constexpr int kYPointFields = 3;
+struct YPoint {
+  const void* in;
+  const double* kq;
+  int kop;
+  double* out;
+};
+struct YPoints {
+  YPoint f[kYPointFields];
+};
+
 // Plan variant of the evaluation kernels: E = 8 where the length has that variant (fewer
 // registers beside the per-entry accumulators), else the length's plan.
 template <int L> constexpr int ypoint_v() { return HasPlanV<L, 1>::value ? 1 : 0; }
@@ -124,12 +139,15 @@ template <int L> constexpr int ypoint_groups() {
 // to the same column's sum.  kq: -k_y^2 on the input (psi_yy) when set.  The cosines come from
 // an LDS copy of k_surf_tables' table, indexed by k(2n+1) mod 4nz.  Each round's rows are
 // loaded during the previous round's transform (the exchanges order LDS only, lds_barrier).
-// Columns with ke < 0 get an unused value.  Grid (nx, ns); dynamic LDS 5 nz doubles.
+// Columns with ke < 0 get an unused value.  Grid (nx, ns, fields); dynamic LDS 5 nz doubles.
 template <int L, int V, int NPR, typename TI>
 __global__ __launch_bounds__(NPR*(L / PlanV<L, V>::E)) void k_dct_ypoint(
-    const TI* __restrict__ in, const int* __restrict__ ke, int nx, int nz, const cplx<double>* __restrict__ tw,
-    const cplx<double>* __restrict__ qtw, const double* __restrict__ kq, const double* __restrict__ kzt, int zop,
-    const double* __restrict__ trig, double* __restrict__ out) {
+    YPoints ys, const int* __restrict__ ke, int nx, int nz, const cplx<double>* __restrict__ tw,
+    const cplx<double>* __restrict__ qtw, const double* __restrict__ kzt, int zop, const double* __restrict__ trig) {
+  const YPoint& y = ys.f[blockIdx.z];
+  const TI* __restrict__ in = (const TI*)y.in;
+  const double* __restrict__ kq = y.kq;
+  double* __restrict__ out = y.out;
   using T = double;
   constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NPR * TPC;
   using AD = ColAddr<L>;
@@ -233,10 +251,10 @@ __global__ __launch_bounds__(NPR*(L / PlanV<L, V>::E)) void k_dct_ypoint(
   for (int e = 0; e < E; ++e) R[q0 * L + mk_src(TL::template pos_in<RL>(tc0, e), L)] = acc[e];
   lds_barrier();
   double* o = out + (int64_t)s * nx * L + (int64_t)x * L;
-  for (int y = tid; y < L; y += NT) {
+  for (int i = tid; i < L; i += NT) {
     double sum = 0.0;
-    for (int g = 0; g < NPR; ++g) sum += R[g * L + y];
-    o[y] = sum;
+    for (int g = 0; g < NPR; ++g) sum += R[g * L + i];
+    o[i] = sum;
   }
 }
 
@@ -248,12 +266,16 @@ __global__ __launch_bounds__(NPR*(L / PlanV<L, V>::E)) void k_dct_ypoint(
 // m_k the k_z multiplier (zop KM_IKZ: i k_z, KM_DZZ: -k_z^2, else 1).  kq with kop: the k_y
 // multiplier on the input (KM_IKY: i k_y, KM_DYY: -k_y^2), as in k_ypass.  Cosines and sines
 // from an LDS copy of k_surf_tables' tables, indexed by kn mod nz; rows prefetched as in
-// k_dct_ypoint.  Grid (nx, ns); dynamic LDS 2 nz + 2 (nz/2 + 1) doubles.
+// k_dct_ypoint.  Grid (nx, ns, fields); dynamic LDS 2 nz + 2 (nz/2 + 1) doubles.
 template <int L, int V, int NPC>
 __global__ __launch_bounds__(NPC*(L / PlanV<L, V>::E)) void k_ypoint(
-    const cplx<double>* __restrict__ in, const int* __restrict__ ke, int nx, int nz,
-    const cplx<double>* __restrict__ tw, const double* __restrict__ kq, int kop, const double* __restrict__ kzt,
-    int zop, const double* __restrict__ trig, double* __restrict__ out) {
+    YPoints ys, const int* __restrict__ ke, int nx, int nz, const cplx<double>* __restrict__ tw,
+    const double* __restrict__ kzt, int zop, const double* __restrict__ trig) {
+  const YPoint& y = ys.f[blockIdx.z];
+  const cplx<double>* __restrict__ in = (const cplx<double>*)y.in;
+  const double* __restrict__ kq = y.kq;
+  const int kop = y.kop;
+  double* __restrict__ out = y.out;
   using T = double;
   constexpr int E = PlanV<L, V>::E, TPC = L / E, NT = NPC * TPC;
   using AD = ColAddr<L>;
@@ -340,51 +362,50 @@ __global__ __launch_bounds__(NPC*(L / PlanV<L, V>::E)) void k_ypoint(
   for (int e = 0; e < E; ++e) R[col0 * L + TL::template pos_in<RL>(tc0, e)] = acc[e];
   lds_barrier();
   double* o = out + (int64_t)s * nx * L + (int64_t)x * L;
-  for (int y = tid; y < L; y += NT) {
+  for (int i = tid; i < L; i += NT) {
     double sum = 0.0;
-    for (int g = 0; g < NPC; ++g) sum += R[g * L + y];
-    o[y] = sum;
+    for (int g = 0; g < NPC; ++g) sum += R[g * L + i];
+    o[i] = sum;
   }
 }
 
 template <int L>
-static hipError_t surf_ypoint_launch(bool neu, bool f32in, const void* in, const int* ke, int nx, int nz, int ns,
-                                     const cplx<double>* tw, const cplx<double>* qtw, const double* kq, int kop,
-                                     const double* kzt, int zop, const double* trig, double* out, hipStream_t st) {
+static hipError_t surf_ypoint_launch(bool neu, bool f32in, const YPoints& ys, int n, const int* ke, int nx, int nz, int ns,
+                                     const cplx<double>* tw, const cplx<double>* qtw, const double* kzt, int zop,
+                                     const double* trig, hipStream_t st) {
   constexpr int V = ypoint_v<L>(), G = ypoint_groups<L>(), NT = G * (L / PlanV<L, V>::E);
-  const dim3 grid((unsigned)nx, (unsigned)ns), block(NT);
+  const dim3 grid((unsigned)nx, (unsigned)ns, (unsigned)n), block(NT);
   if (neu) {
     const size_t dyn = sizeof(double) * 5 * (size_t)nz;
     if (f32in)
-      SMX_LAUNCH((k_dct_ypoint<L, V, G, float>), grid, block, dyn, st, (const float*)in, ke, nx, nz, tw, qtw, kq, kzt,
-                 zop, trig, out);
+      SMX_LAUNCH((k_dct_ypoint<L, V, G, float>), grid, block, dyn, st, ys, ke, nx, nz, tw, qtw, kzt, zop, trig);
     else
-      SMX_LAUNCH((k_dct_ypoint<L, V, G, double>), grid, block, dyn, st, (const double*)in, ke, nx, nz, tw, qtw, kq,
-                 kzt, zop, trig, out);
+      SMX_LAUNCH((k_dct_ypoint<L, V, G, double>), grid, block, dyn, st, ys, ke, nx, nz, tw, qtw, kzt, zop, trig);
   } else {
     if (f32in) return hipErrorInvalidValue;
     const size_t dyn = sizeof(double) * (2 * (size_t)nz + 2 * (size_t)(nz / 2 + 1));
-    SMX_LAUNCH((k_ypoint<L, V, G>), grid, block, dyn, st, (const cplx<double>*)in, ke, nx, nz, tw, kq, kop, kzt, zop,
-               trig, out);
+    SMX_LAUNCH((k_ypoint<L, V, G>), grid, block, dyn, st, ys, ke, nx, nz, tw, kzt, zop, trig);
   }
   return hipGetLastError();
 }
 
-// Field values at ke of every column into out[ns][nx*ny] (parts per kz split) from an x stage
-// `in` of an nx x ny x nz grid: FP64, or (Neumann, f32in) the FP32 stage.  kq/kop: k_y
-// multiplier (Neumann: KM_DYY only); zop: k_z multiplier (Neumann: KM_DZZ only); -1: none.
+// Values of n fields at ke of every column, each into its out[ns][nx*ny] (parts per kz split), from x stages
+// of an nx x ny x nz grid: FP64, or (Neumann, f32in) FP32 ones.  k_y multipliers: Neumann KM_DYY only; zop: k_z
+// multiplier (Neumann: KM_DZZ only); -1: none.
 // tw, qtw: the y-axis twiddles (qtw Neumann); trig: k_surf_tables' table of this nz.
-inline hipError_t surf_ypoint(bool neu, bool f32in, const void* in, const int* ke, int nx, int ny, int nz, int ns,
-                              const cplx<double>* tw, const cplx<double>* qtw, const double* kq, int kop,
-                              const double* kzt, int zop, const double* trig, double* out, hipStream_t st) {
-  if (ns < 1 || ns > kSurfMaxSplit) return hipErrorInvalidValue;
-  if ((kq == nullptr) != (kop < 0)) return hipErrorInvalidValue;
-  if (neu ? (kop >= 0 && kop != KM_DYY) || (zop >= 0 && zop != KM_DZZ)
-          : (kop >= 0 && kop != KM_IKY && kop != KM_DYY) || (zop >= 0 && zop != KM_IKZ && zop != KM_DZZ))
-    return hipErrorInvalidValue;
+inline hipError_t surf_ypoint(bool neu, bool f32in, const YPoints& ys, int n, const int* ke, int nx, int ny, int nz,
+                              int ns, const cplx<double>* tw, const cplx<double>* qtw, const double* kzt, int zop,
+                              const double* trig, hipStream_t st) {
+  if (ns < 1 || ns > kSurfMaxSplit || n < 1 || n > kYPointFields) return hipErrorInvalidValue;
+  for (int i = 0; i < n; ++i) {
+    const int kop = ys.f[i].kop;
+    if ((ys.f[i].kq == nullptr) != (kop < 0)) return hipErrorInvalidValue;
+    if (neu ? (kop >= 0 && kop != KM_DYY) || (zop >= 0 && zop != KM_DZZ)
+            : (kop >= 0 && kop != KM_IKY && kop != KM_DYY) || (zop >= 0 && zop != KM_IKZ && zop != KM_DZZ))
+      return hipErrorInvalidValue;
+  }
 #define SMX_CASE(L)                                                                                        \
-  if (ny == L)                                                                                             \
-    return surf_ypoint_launch<L>(neu, f32in, in, ke, nx, nz, ns, tw, qtw, kq, kop, kzt, zop, trig, out, st);
+  if (ny == L) return surf_ypoint_launch<L>(neu, f32in, ys, n, ke, nx, nz, ns, tw, qtw, kzt, zop, trig, st);
   SMX_FOR_EACH_LENGTH(SMX_CASE)
 #undef SMX_CASE
   return hipErrorInvalidValue;
