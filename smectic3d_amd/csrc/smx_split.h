@@ -590,7 +590,8 @@ enum FormDir { FORM_TO_STD = 0, FORM_FROM_STD = 1, FORM_PERM_TO_STD = 2, FORM_PE
 // To standard, which every diagnostic on the spectrum begins with.  A thread has the RB values of one k1 of a
 // row, loads them in pieces of YC and stores them 16 bytes a lane with the lanes along k1: every load of the
 // block is in flight at once and nothing goes through LDS but the twiddles, so that the copy runs at the rate
-// of its bytes (256^3: FP64 78 -> 52 us, 5.2 TB/s, from FP32 78 -> 40).  In place allowed (TI = T): whole rows per block, stored behind a barrier.
+// of its bytes (256^3: FP64 78 -> 52 us, 5.2 TB/s, from FP32 78 -> 40).  In place allowed (TI = T): whole rows per
+// block, stored behind a barrier.
 // TI: the input's type (float rows widened into an FP64 copy).
 template <typename T, int RA, int RB, typename TI = T>
 __global__ __launch_bounds__(256) void k_form_std(const cplx<TI>* in, cplx<T>* out, int64_t nrows,
@@ -621,61 +622,62 @@ __global__ __launch_bounds__(256) void k_form_std(const cplx<TI>* in, cplx<T>* o
   for (int c = 0; c < RB; ++c) dst[RA * c] = (T)(1.0 / RB) * w[c];
 }
 
-// From standard and the carry's orders: once after a state is set, loaded or left in the other form.
-template <typename T, int RB>
-__global__ __launch_bounds__(256) void k_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny,
-                                              const cplx<T>* __restrict__ twy, int dir, const T* __restrict__ kmul) {
-  constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
-  __shared__ cplx<T> S[CAP + CAP / 16];
-  auto at = [](int i) { return i + (i >> 4); };
-  const int ra = ny / RB, rows = CAP / ny, tid = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * rows;
-  const int nr = (int)(nrows - r0 < rows ? nrows - r0 : rows);
-  const int n = nr * ny;
-  const cplx<T>* src = in + r0 * ny;
-  cplx<T>* dst = out + r0 * ny;
-  for (int i = tid; i < n; i += 256) {
-    cplx<T> e = src[i];
+// From standard, once after a state is set or loaded: the mirror image, loads along k1 and stores in pieces (256^3
+// FP64 70 us through LDS on both sides, now 58; FP32 31 and 26).
+template <typename T, int RA, int RB>
+__global__ __launch_bounds__(256) void k_form_split(const cplx<T>* in, cplx<T>* out, int64_t nrows,
+                                                    const cplx<T>* __restrict__ twy, const T* __restrict__ kmul) {
+  constexpr int NY = RA * RB, ROWS = 256 / RA, YC = kSplitYC;
+  __shared__ cplx<T> TW[NY];
+  const int tid = threadIdx.x, row = tid / RA, k1 = tid - row * RA;
+  const int64_t r = (int64_t)blockIdx.x * ROWS + row;
+  const bool item = row < ROWS && r < nrows;
+  cplx<T> w[RB];
+  if (item) {
+    const cplx<T>* src = in + r * NY + k1;
+#pragma unroll
+    for (int c = 0; c < RB; ++c) w[c] = src[RA * c];
     if (kmul != nullptr) {  // i k_y of the spectral d/dy (pf3d.cpp:405)
-      const T k = kmul[i % ny];
-      e = mk(-k * e.y, k * e.x);
+#pragma unroll
+      for (int c = 0; c < RB; ++c) {
+        const T k = kmul[k1 + RA * c];
+        w[c] = mk(-k * w[c].y, k * w[c].x);
+      }
     }
-    S[at(i)] = e;
   }
+  tw_lds<NY, 256>(TW, twy, tid);
+  __syncthreads();  // the table; and in place, every read of the rows
+  if (!item) return;
+  dft<RB, +1>(w);
+#pragma unroll
+  for (int c = 1; c < RB; ++c) w[c] = cmul(w[c], conjg(TW[k1 * c]));
+  cplx<T>* dst = out + r * NY + split_pos(k1, 0, RB);
+#pragma unroll
+  for (int c = 0; c < RB; c += 2)
+    *reinterpret_cast<cplx2<T>*>(dst + c / YC * 2 * YC + c % YC) = cplx2<T>{w[c], w[c + 1]};
+}
+
+// The carry's orders.
+template <typename T, int RA, int RB, bool TO_STD>
+__global__ __launch_bounds__(256) void k_form_perm(const cplx<T>* in, cplx<T>* out, int64_t nrows) {
+  constexpr int NY = RA * RB, ROWS = 1024 / NY, N = ROWS * NY;
+  __shared__ cplx<T> S[N + N / 16];
+  auto at = [](int i) { return i + (i >> 4); };
+  const int tid = threadIdx.x;
+  const int64_t r0 = (int64_t)blockIdx.x * ROWS;
+  const int n = (int)(nrows - r0 < ROWS ? nrows - r0 : ROWS) * NY;
+  const cplx<T>* src = in + r0 * NY;
+  cplx<T>* dst = out + r0 * NY;
+#pragma unroll
+  for (int u = 0; u < (N + 255) / 256; ++u)
+    if (const int i = tid + u * 256; i < n) S[at(i)] = src[i];
   __syncthreads();
-  if (dir == FORM_PERM_TO_STD || dir == FORM_PERM_FROM_STD) {
-    for (int i = tid; i < n; i += 256) {
-      const int row = i / ny, c = i - row * ny;
-      dst[i] = S[at(row * ny + (dir == FORM_PERM_TO_STD ? (c % ra) * RB + c / ra : c / RB + ra * (c % RB)))];
+#pragma unroll
+  for (int u = 0; u < (N + 255) / 256; ++u)
+    if (const int i = tid + u * 256; i < n) {
+      const int c = i % NY;
+      dst[i] = S[at(i - c + (TO_STD ? c % RA * RB + c / RA : c / RB + RA * (c % RB)))];
     }
-    return;
-  }
-  // item: one row and k1; its k2 values at k1 + ra k2, its y2 values at split_pos
-  constexpr int IPT = (CAP / RB + 255) / 256;
-  cplx<T> w[IPT][RB];
-#pragma unroll
-  for (int it = 0; it < IPT; ++it) {
-    const int i = tid + it * 256, row = i / ra, k1 = i - row * ra;
-    if (i < nr * ra) {
-#pragma unroll
-      for (int c = 0; c < RB; ++c) w[it][c] = S[at(row * ny + k1 + ra * c)];
-      dft<RB, +1>(w[it]);
-#pragma unroll
-      for (int c = 0; c < RB; ++c) w[it][c] = cmul(w[it][c], conjg(twy[k1 * c]));
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < IPT; ++it) {
-    const int i = tid + it * 256, row = i / ra, k1 = i - row * ra;
-    if (i < nr * ra) {
-#pragma unroll
-      for (int c = 0; c < RB; ++c) S[at(row * ny + split_pos(k1, c, RB))] = w[it][c];
-    }
-  }
-  __syncthreads();
-  for (int i = tid; i < n; i += 256) dst[i] = S[at(i)];
 }
 
 }  // namespace smx
-

@@ -253,19 +253,23 @@ hipError_t split_form_std(const cplx<TI>* in, cplx<T>* out, int64_t nrows, int n
 template <typename T>
 hipError_t split_form(const cplx<T>* in, cplx<T>* out, int64_t nrows, int ny, const cplx<T>* twy, int dir,
                       const T* kmul, hipStream_t st) {
-  if (dir == FORM_TO_STD) return kmul == nullptr ? split_form_std<T, T>(in, out, nrows, ny, twy, st) : hipErrorInvalidValue;
-  const int ra = split_ra(ny);
-  if (ra == 0 || nrows < 1) return hipErrorInvalidValue;
-  const int rows = 1024 / ny;
-  const dim3 grid((unsigned)((nrows + rows - 1) / rows));
-#define SMX_CASE(RB)                                                                                            \
-  case RB: SMX_LAUNCH((k_form<T, RB>), grid, dim3(256), 0, st, in, out, nrows, ny, twy, dir, kmul); break;
-  switch (ny / ra) {
-    SMX_CASE(4) SMX_CASE(8) SMX_CASE(12) SMX_CASE(16)
-    default: return hipErrorInvalidValue;
+  if (nrows < 1 || (kmul != nullptr && dir != FORM_FROM_STD)) return hipErrorInvalidValue;
+  if (dir == FORM_TO_STD) return split_form_std<T, T>(in, out, nrows, ny, twy, st);
+  auto grid = [&](int rows) { return dim3((unsigned)((nrows + rows - 1) / rows)); };
+#define SMX_CASE(NY)                                                                                              \
+  if (ny == NY) {                                                                                                 \
+    constexpr int RA = split_ra(NY), RB = NY / RA;                                                                \
+    if (dir == FORM_FROM_STD)                                                                                     \
+      SMX_LAUNCH((k_form_split<T, RA, RB>), grid(256 / RA), dim3(256), 0, st, in, out, nrows, twy, kmul);         \
+    else if (dir == FORM_PERM_TO_STD)                                                                             \
+      SMX_LAUNCH((k_form_perm<T, RA, RB, true>), grid(1024 / NY), dim3(256), 0, st, in, out, nrows);              \
+    else                                                                                                          \
+      SMX_LAUNCH((k_form_perm<T, RA, RB, false>), grid(1024 / NY), dim3(256), 0, st, in, out, nrows);             \
+    return hipGetLastError();                                                                                     \
   }
+  SMX_FOR_EACH_SPLIT(SMX_CASE)
 #undef SMX_CASE
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 #endif
 
@@ -402,40 +406,38 @@ hipError_t nsplit_real(const cplx<TI>* a, double* out, const PParams<double>& p,
     }
   });
 }
-template <typename TI, typename TO, int NY, int RA>
-static hipError_t nsplit_form_std(const TI* in, TO* out, int nx, int nz, const cplx<double>* twy,
-                                  const cplx<double>* qty, hipStream_t st) {
+template <typename TI, typename TO, int RA, int RB>
+static hipError_t nsplit_form_dir(const TI* in, TO* out, int nx, int nz, const cplx<double>* twy,
+                                  const cplx<double>* qty, int dir, hipStream_t st) {
   constexpr int ROWS = 128 / RA;
-  SMX_LAUNCH((k_nform_std<TI, TO, RA, NY / RA>), dim3((unsigned)((nx * (nz / 2) + ROWS - 1) / ROWS)), dim3(128), 0, st,
-             in, out, nx, nz, twy, qty);
+  const dim3 grid((unsigned)((nx * (nz / 2) + ROWS - 1) / ROWS));
+  if (dir == FORM_TO_STD) {
+    SMX_LAUNCH((k_nform_std<TI, TO, RA, RB>), grid, dim3(128), 0, st, in, out, nx, nz, twy, qty);
+  } else if constexpr (std::is_same_v<TI, TO>) {
+    if (dir == FORM_FROM_STD)
+      SMX_LAUNCH((k_nform_split<TI, RA, RB>), grid, dim3(128), 0, st, in, out, nx, nz, twy, qty);
+    else if (dir == FORM_PERM_TO_STD)
+      SMX_LAUNCH((k_nform_perm<TI, RA, RB, true>), grid, dim3(128), 0, st, in, out, nx, nz);
+    else
+      SMX_LAUNCH((k_nform_perm<TI, RA, RB, false>), grid, dim3(128), 0, st, in, out, nx, nz);
+  } else {
+    return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 template <typename TI, typename TO>
 hipError_t nsplit_form(const TI* in, TO* out, int nx, int ny, int nz, const cplx<double>* twy, const cplx<double>* qty,
                        int dir, hipStream_t st) {
   const int ra = nsplit_ra(ny, nx);
-  if (ra == 0) return hipErrorInvalidValue;
-  if (dir == FORM_TO_STD) {
 #define SMX_CASE(NY)                                                                                              \
   if (ny == NY) {                                                                                                 \
     constexpr int R0 = nsplit_ra(NY, 1), R3 = nsplit_ra(NY, 3);                                                   \
-    return ra == R0 ? nsplit_form_std<TI, TO, NY, R0>(in, out, nx, nz, twy, qty, st)                              \
-                    : nsplit_form_std<TI, TO, NY, R3>(in, out, nx, nz, twy, qty, st);                             \
+    return ra == R0 ? nsplit_form_dir<TI, TO, R0, NY / R0>(in, out, nx, nz, twy, qty, dir, st)                    \
+                    : nsplit_form_dir<TI, TO, R3, NY / R3>(in, out, nx, nz, twy, qty, dir, st);                   \
   }
-    SMX_FOR_EACH_SPLIT(SMX_CASE)
+  SMX_FOR_EACH_SPLIT(SMX_CASE)
 #undef SMX_CASE
-    return hipErrorInvalidValue;
-  }
-  const int rows = 1024 / ny;
-  const dim3 grid((unsigned)((nx * (nz / 2) + rows - 1) / rows));
-#define SMX_CASE(RB)                                                                                           \
-  case RB: SMX_LAUNCH((k_nform<TI, TO, RB>), grid, dim3(256), 0, st, in, out, nx, ny, nz, twy, qty, dir); break;
-  switch (ny / ra) {
-    SMX_CASE(4) SMX_CASE(8) SMX_CASE(12) SMX_CASE(16)
-    default: return hipErrorInvalidValue;
-  }
-#undef SMX_CASE
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 #endif
 

@@ -413,6 +413,15 @@ __global__ __launch_bounds__(X::NT) void k_nsplit_x(SplitNeuArgs<typename X::T> 
 
 // ---------------------------------------------------------------------------
 // Between the two forms, out of place, in FP64.  Rows (j, x) of the split form, two planes of the standard one.
+// Rows r0 .. of the split form and their two planes' rows of the standard one, PL, by the first nr threads.
+__device__ __forceinline__ void nform_planes(int64_t (*PL)[2], int r0, int nr, int nx, int nz, int ny, int tid) {
+  if (tid < nr) {
+    const int j = (r0 + tid) / nx, x = r0 + tid - j * nx;
+    PL[tid][0] = ((int64_t)j * nx + x) * ny;
+    PL[tid][1] = ((int64_t)(j == 0 ? nz / 2 : nz - j) * nx + x) * ny;
+  }
+}
+
 // To standard as k_form_std, but with the lines' untangling from LDS (ky and ny - ky of a row are two threads')
 // and real rows stored 8 bytes a lane (256 x 256 x 384 from FP32: 151 -> 67 us).
 template <typename TI, typename TO, int RA, int RB>
@@ -439,11 +448,7 @@ __global__ __launch_bounds__(128) void k_nform_std(const TI* __restrict__ in, TO
     }
   }
   tw_lds<NY, NT>(TW, twy, tid);
-  if (tid < nr) {
-    const int j = (r0 + tid) / nx, x = r0 + tid - j * nx;
-    PL[tid][0] = ((int64_t)j * nx + x) * NY;
-    PL[tid][1] = ((int64_t)(j == 0 ? nz / 2 : nz - j) * nx + x) * NY;
-  }
+  nform_planes(PL, r0, nr, nx, nz, NY, tid);
   __syncthreads();
   if (item) {
 #pragma unroll
@@ -464,69 +469,99 @@ __global__ __launch_bounds__(128) void k_nform_std(const TI* __restrict__ in, TO
   }
 }
 
-// From standard and the carry's orders; whole rows per block of 256 threads, an item the RB values of one row
-// and k1 (as k_form).
-template <typename TI, typename TO, int RB>
-__global__ __launch_bounds__(256) void k_nform(const TI* __restrict__ in, TO* __restrict__ out, int nx, int ny, int nz,
-                                               const cplx<double>* __restrict__ twy,
-                                               const cplx<double>* __restrict__ qty, int dir) {
+// From standard, once after a state is set or loaded: the mirror image, with both sides of memory along the rows and
+// every index by constants (256 x 256 x 384 FP32 128 us with divisions at run time, now 78; the carry 80 and 46;
+// 256^3 FP64 87 and 54).
+template <typename T, int RA, int RB>
+__global__ __launch_bounds__(128) void k_nform_split(const T* __restrict__ in, T* __restrict__ out, int nx, int nz,
+                                                     const cplx<double>* __restrict__ twy,
+                                                     const cplx<double>* __restrict__ qty) {
   using C = cplx<double>;
-  constexpr int CAP = 1024;  // >= 2 rows of the longest length with a split
-  static_assert(CAP / RB <= 256, "one item per thread");
-  __shared__ C S[CAP + CAP / 16];
+  constexpr int NT = 128, NY = RA * RB, ROWS = NT / RA, N = ROWS * NY, U = (N + NT - 1) / NT;
+  __shared__ C S[N + N / 16];
+  __shared__ C TW[NY];
+  __shared__ int64_t PL[ROWS][2];
   auto at = [](int i) { return i + (i >> 4); };
-  const int ra = ny / RB, rows = CAP / ny, tid = threadIdx.x, nrows = nx * (nz / 2);
-  const int r0 = blockIdx.x * rows, nr = nrows - r0 < rows ? nrows - r0 : rows, n = nr * ny;
-  // words of row r: its two planes in the standard form, and the split form's row
-  auto plane = [&](int r, int b) {
-    const int j = r / nx, kz = b == 0 ? j : (j == 0 ? nz / 2 : nz - j);
-    return ((int64_t)kz * nx + (r - j * nx)) * ny;
-  };
-  if (dir == FORM_PERM_TO_STD || dir == FORM_PERM_FROM_STD) {
-    for (int i = tid; i < n; i += 256) {
-      const int r = r0 + i / ny, c = i % ny;
-      const int t = c / (2 * RB), b = c / RB % 2, u = c % RB;
-      const int ka = nsplit_ky(t, u, ra, RB), k = b == 0 ? ka : (ka == 0 ? ny / 2 : ny - ka);
-      const int64_t o = 2 * ((int64_t)r * ny + c);
-      if (dir == FORM_PERM_TO_STD) {
-        out[plane(r, 0) + k] = (TO)in[o];
-        out[plane(r, 1) + k] = (TO)in[o + 1];
-      } else {
-        out[o] = (TO)in[plane(r, 0) + k];
-        out[o + 1] = (TO)in[plane(r, 1) + k];
-      }
-    }
-    return;
+  const int tid = threadIdx.x, row = tid / RA, k1 = tid - row * RA;
+  const int nrows = nx * (nz / 2), r0 = blockIdx.x * ROWS, nr = nrows - r0 < ROWS ? nrows - r0 : ROWS;
+  const bool item = row < nr;
+  nform_planes(PL, r0, nr, nx, nz, NY, tid);
+  __syncthreads();
+  cplx<T> g[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {  // every load is issued before the first is used
+    const int i = tid + u * NT, rr = i / NY, c = i - rr * NY;
+    if (rr < nr) g[u] = mk(in[PL[rr][0] + c], in[PL[rr][1] + c]);
   }
-  for (int i = tid; i < n; i += 256) {
-    const int r = r0 + i / ny, c = i % ny;
-    S[at(i)] = mk((double)in[plane(r, 0) + c], (double)in[plane(r, 1) + c]);
+  tw_lds<NY, NT>(TW, twy, tid);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = tid + u * NT;
+    if (i < nr * NY) S[at(i)] = mk((double)g[u].x, (double)g[u].y);
   }
   __syncthreads();
-  const int row = tid / ra, k1 = tid - row * ra;
-  const bool item = tid < nr * ra;
   C w[RB];
   if (item) {
 #pragma unroll
     for (int c = 0; c < RB; ++c) {
-      const int k = k1 + ra * c;
-      w[c] = dct3_in(S[at(row * ny + k)], k == 0 ? mk<double>(0, 0) : S[at(row * ny + ny - k)], qty[k]);
+      const int k = k1 + RA * c;
+      w[c] = dct3_in(S[at(row * NY + k)], k == 0 ? mk<double>(0, 0) : S[at(row * NY + NY - k)], qty[k]);
     }
     dft<RB, +1>(w);
 #pragma unroll
-    for (int c = 0; c < RB; ++c) w[c] = cmul(w[c], conjg(twy[k1 * c]));
+    for (int c = 1; c < RB; ++c) w[c] = cmul(w[c], conjg(TW[k1 * c]));
   }
   __syncthreads();
   if (item) {
 #pragma unroll
-    for (int c = 0; c < RB; ++c) S[at(row * ny + nsplit_pos(k1, c, ra, RB))] = w[c];
+    for (int c = 0; c < RB; ++c) S[at(row * NY + nsplit_pos(k1, c, RA, RB))] = w[c];
   }
   __syncthreads();
-  for (int i = tid; i < n; i += 256) {
-    const int rr = i / ny, r = r0 + rr, c = i - rr * ny;
-    const int64_t o = 2 * ((int64_t)r * ny + c);
-    out[o] = (TO)S[at(i)].x;
-    out[o + 1] = (TO)S[at(i)].y;
+  cplx<T>* dst = reinterpret_cast<cplx<T>*>(out) + (int64_t)r0 * NY;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = tid + u * NT;
+    if (i < nr * NY) dst[i] = mk((T)S[at(i)].x, (T)S[at(i)].y);
+  }
+}
+
+// The carry's orders: the pair of planes at ky of the standard form, at (t, ky or ny - ky, u) of the other.
+template <typename T, int RA, int RB, bool TO_STD>
+__global__ __launch_bounds__(128) void k_nform_perm(const T* __restrict__ in, T* __restrict__ out, int nx, int nz) {
+  constexpr int NT = 128, NY = RA * RB, ROWS = NT / RA, N = ROWS * NY, U = (N + NT - 1) / NT;
+  __shared__ cplx<T> S[N + N / 16];
+  __shared__ int64_t PL[ROWS][2];
+  auto at = [](int i) { return i + (i >> 4); };
+  auto ky = [](int c) {
+    const int k = nsplit_ky(c / (2 * RB), c % RB, RA, RB);
+    return c / RB % 2 == 0 ? k : (k == 0 ? NY / 2 : NY - k);
+  };
+  const int tid = threadIdx.x;
+  const int nrows = nx * (nz / 2), r0 = blockIdx.x * ROWS, nr = nrows - r0 < ROWS ? nrows - r0 : ROWS;
+  nform_planes(PL, r0, nr, nx, nz, NY, tid);
+  __syncthreads();
+  const cplx<T>* src = reinterpret_cast<const cplx<T>*>(in) + (int64_t)r0 * NY;
+  cplx<T>* dst = reinterpret_cast<cplx<T>*>(out) + (int64_t)r0 * NY;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = tid + u * NT, rr = i / NY, c = i - rr * NY;
+    if (rr < nr) {
+      if constexpr (TO_STD) S[at(rr * NY + ky(c))] = src[i];
+      else S[at(i)] = mk(in[PL[rr][0] + c], in[PL[rr][1] + c]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = tid + u * NT, rr = i / NY, c = i - rr * NY;
+    if (rr < nr) {
+      if constexpr (TO_STD) {
+        out[PL[rr][0] + c] = S[at(i)].x;
+        out[PL[rr][1] + c] = S[at(i)].y;
+      } else {
+        dst[i] = S[at(rr * NY + ky(c))];
+      }
+    }
   }
 }
 
