@@ -596,6 +596,13 @@ static int step_once(smx_handle* h, const PParams<T>& p, hipEvent_t* ev) {
   return SMX_OK;  // the x pass projects the self-conjugate planes of R itself
 }
 
+// Whether the two-launch periodic step is the faster one where it fits: not in FP64 boxes of long x lines with so
+// few blocks in the x kernel that it takes as long as the chain through one of them.  The four-pass x kernel has
+// tiles of half the columns: 512 x 16 x 16 (9 blocks) 27.3 us and 22.4 in four passes, 384 x 16 x 16 23.7 and 22.3;
+// 384 x 16 x 24 (13 blocks) 23.2 and 23.8, 256 x 16 x 16 (9) 16.1 and 18.0.
+static bool split_pays(bool fp32, int nx, int ny, int nz) {
+  return fp32 || 40 * split_x_blocks<double>(nx, ny, nz) >= nx;
+}
 // Whether the two-launch Neumann step is the faster one where it fits.  In FP64, 21 grids have tiles that leave
 // one block a CU in both kernels, 0.74 to 1.03 of the four passes' time.  Those behind are x lines of 256 (16
 // values and 190 registers a thread, 8.9 ns per thousand points where lines of 192 and 384 take 7.2 and 8.2):
@@ -1887,6 +1894,7 @@ int smx_create(const smx_config* cfg, smx_handle** out) {
   if (h->split_ok && !h->neumann) h->split_ok = split_real_fits(c.ny, c.nz);
   h->split_form = h->split_ok;
   if (h->split_ok && h->neumann) h->split_ok = nsplit_pays(h->fp32, c.nx, c.ny, c.nz);
+  if (h->split_ok && !h->neumann && !c.advect) h->split_ok = split_pays(h->fp32, c.nx, c.ny, c.nz);
   for (int k = 0; k < NSLOTS; ++k) h->sched[k] = default_sched(h, k);
   auto bail = [&](int code) {
     smx_destroy(h);

@@ -209,6 +209,17 @@ bool split_x_fits(int nx, int ny) {
          }) == hipSuccess;
 }
 template <typename T>
+int split_x_blocks(int nx, int ny, int nz) {
+  const int ra = split_ra(ny);
+  int n = 0;
+  if (ra != 0)
+    (void)split_x_dispatch(nx, ny / ra, [&](auto l, auto r) -> hipError_t {
+      n = ny / XS<T, decltype(l)::value, decltype(r)::value>::NC * (nz / 2 + 1);
+      return hipSuccess;
+    });
+  return n;
+}
+template <typename T>
 hipError_t split_x(const SplitArgs<T>& s, hipStream_t st) {
   return split_x_dispatch(s.p.nx, s.p.ny / split_ra(s.p.ny), [&](auto l, auto r) -> hipError_t {
     constexpr int L = decltype(l)::value, RB = decltype(r)::value;

@@ -10,6 +10,7 @@ namespace smx {
 // Whether the two kernels exist for this grid: ny has a split and both tiles fit a workgroup.
 template <typename T> bool split_z_fits(int ny, int nz);
 template <typename T> bool split_x_fits(int nx, int ny);
+template <typename T> int split_x_blocks(int nx, int ny, int nz);  // of one step (0: none)
 
 // Blocks of the z kernel that take a tile each (one FP64 partial per block).
 template <typename T> int split_z_blocks(const PParams<T>& p);
