@@ -58,6 +58,29 @@ constexpr int split_ny2(int l, int ra) {
              ? 4
              : 2;
 }
+// FP32 halves are 16 bytes: whole pieces also of a large tile, 12 or 24 values of a y line and a long z line, where
+// they leave blocks for most of the chip (us with halves and whole: 256 x 192 x 384 66 and 57, 256 x 384 x 192 55 and
+// 51, the advected kernels of 256 x 192 x 512 359 + 480 and 321 + 322; but 16 x 192 x 512, 64 whole blocks, a step 29.4 and
+// 31.8), not with 16 values (256 x 256 x 384 80 and 93).
+template <typename T>
+constexpr bool split_whole(int l, int ra) {
+  return sizeof(T) == 4 && ((ra == 12 && l >= 384) || (ra == 24 && l >= 192 && l <= 256));
+}
+constexpr int kSplitWholeBlocks = 192;
+// Padding of a z tile's rows of npr values for the items, whose lanes write runs of ny2 columns of successive
+// rows: ny2 columns, which lets those runs fall in other banks, or less where a CU has three blocks or fewer and the
+// room makes another one fit.
+// Rows of 8 more than a multiple of 16 then have one column (none, if that alone leaves one block), rows of 4 more
+// none, and fall apart as well.  FP64 z kernels: 256 x 192 x 256 78 us with two blocks a CU, 58 with three; 384 x 384 x
+// 128 130 and 86; 384 x 96 x 512 113 with one, 79 with two; FP32 256 x 192 x 256 43 and 32.
+template <typename T>
+constexpr int split_pad(int l, int npr, int ny2) {
+  const auto per_cu = [&](int pad) { return 160 * 1024 / (l * (npr + pad + 1) * 2 * (int)sizeof(T) + 128); };
+  const int full = per_cu(ny2);
+  if (npr % 16 == 0 || full > 3) return ny2;
+  if (npr % 16 == 8) return per_cu(1) > full ? 1 : (full < 2 && per_cu(0) >= 2 ? 0 : ny2);
+  return per_cu(0) > full ? 0 : ny2;
+}
 // Lanes that share one y line in the z kernel (pair_dft): two from radix 16 on, where one lane's 16
 // values make its loads the longest part (256^3 FP32: 40.6 -> 34.0 us; 192^3 FP32: 22.3 with one, 27.7).
 constexpr int split_lanes(int ra) { return ra >= 16 ? 2 : 1; }
@@ -103,12 +126,12 @@ struct ZS {
   static constexpr int E = PlanV<L, V>::E, TPC = L / E;
   static constexpr int NPR = RA * NY2 / 2, NT = NPR * TPC, NZH = L / 2 + 1;
   static constexpr int H = RA / P, HC = H / 2;
-  // Tile pitch of the transform, and of the items, whose lanes write runs of NY2 columns of successive rows:
-  // those fall in other banks.  Column q: the lines y1 = 2 (q / NY2) and the next, y2 = q % NY2.
-  static constexpr int FP = NPR, HP = NPR + NY2;
+  // Tile pitch of the transform, of the items, and of a tile whose columns are read along z (lanes on successive
+  // rows, an odd pitch or the items').  Column q: the lines y1 = 2 (q / NY2) and the next, y2 = q % NY2.
+  static constexpr int FP = NPR, HP = NPR + split_pad<T>(L, NPR, NY2), SP = NPR + 1;
   // Items of the y part, H values each: one kz, one y2 and (P = 2) one parity of k1, half of the y1.
   static constexpr int ITEMS = NZH * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
-  static constexpr int LDS = L * HP;
+  static constexpr int LDS = L * HP, SLDS = L * (HP > SP ? HP : SP);
   static constexpr int RED = (NT % 64 == 0) ? NT / 64 : NT;
   static constexpr bool fits = NT <= 1024 && (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8 <= 160 * 1024;
 };
@@ -380,7 +403,7 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_grp(const SplitArgs<typename Z
 template <typename Z, typename TI>
 __global__ __launch_bounds__(Z::NT) void k_zsplit_real(const cplx<TI>* a, double* __restrict__ out, PParams<double> p) {
   constexpr int L = Z::L, RA = Z::RA;
-  __shared__ cplx<double> F[Z::LDS];
+  __shared__ cplx<double> F[Z::SLDS];
   __shared__ cplx<double> TW[L];
   const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
   const int rb = p.ny / RA;
@@ -391,13 +414,13 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_real(const cplx<TI>* a, double
                     (uint32_t)p.nxy * (uint32_t)sizeof(cplx<TI>), rb, F, TW, tid, q, tc, v,
                     (const double*)nullptr, p.twz);
   __syncthreads();
-  Tile<double, L, Z::E, Z::HP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
+  Tile<double, L, Z::E, Z::SP>::template store<inv_last<L, Z::V>()>(v, F, q, tc);
   __syncthreads();
   // lanes run along z of one column pair: two coalesced rows
   for (int i = tid; i < Z::NPR * L; i += Z::NT) {
     const int qq = i / L, n = i - qq * L;
     const int y = 2 * (qq / Z::NY2) * rb + yg * Z::NY2 + qq % Z::NY2;
-    const cplx<double> w = F[n * Z::HP + qq];
+    const cplx<double> w = F[n * Z::SP + qq];
     double* row = out + ((int64_t)x * p.ny + y) * L;
     row[n] = w.x;
     row[(int64_t)rb * L + n] = w.y;

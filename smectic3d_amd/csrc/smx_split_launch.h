@@ -43,6 +43,18 @@ hipError_t split_x_dispatch(int nx, int rb, F&& f) {
 // The y lengths with a division (split_ra, nsplit_ra).
 #define SMX_FOR_EACH_SPLIT(X) X(16) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384)
 
+// f(ZS of the grid): the tile with whole pieces where split_whole asks for it and there are blocks enough.  One
+// choice for a box, alone or in a group, so that its partial sums are counted alike.
+template <typename T, int L, int RA, typename F>
+hipError_t split_z_tile(int nx, int ny, F&& f) {
+  if constexpr (split_whole<T>(L, RA)) {
+    using Z = ZS<T, L, RA, kSplitYC>;
+    static_assert(Z::fits, "both tiles fit");
+    if (nx * (ny / RA / kSplitYC) >= kSplitWholeBlocks) return f(Z{});
+  }
+  return f(ZS<T, L, RA>{});
+}
+
 // Blocks that project the carry: 8 pairs' entries per thread.
 template <typename Z, typename T>
 static int split_nproj(const PParams<T>& p) {
@@ -63,39 +75,43 @@ int split_z_blocks(const PParams<T>& p) {
   int n = 0;
   const int ra = split_ra(p.ny);
   (void)split_z_dispatch(p.nz, ra, [&](auto l, auto r) -> hipError_t {
-    n = p.nx * (p.ny / ra / ZS<T, decltype(l)::value, decltype(r)::value>::NY2);
-    return hipSuccess;
+    return split_z_tile<T, decltype(l)::value, decltype(r)::value>(p.nx, p.ny, [&](auto z) -> hipError_t {
+      n = p.nx * (p.ny / ra / decltype(z)::NY2);
+      return hipSuccess;
+    });
   });
   return n;
 }
 template <typename T>
 hipError_t split_z(const SplitArgs<T>& s, int op, hipStream_t st) {
   return split_z_dispatch(s.p.nz, split_ra(s.p.ny), [&](auto l, auto r) -> hipError_t {
-    constexpr int L = decltype(l)::value, RA = decltype(r)::value;
-    using Z = ZS<T, L, RA>;
-    if constexpr (!Z::fits) {
-      return hipErrorInvalidValue;
-    } else {
-      const int np = split_nproj<Z>(s.p);
-      SMX_LAUNCH((k_zsplit<Z>), dim3((unsigned)(np + split_z_blocks(s.p))), dim3(Z::NT), 0, st, s, op, np);
-      return hipGetLastError();
-    }
+    return split_z_tile<T, decltype(l)::value, decltype(r)::value>(s.p.nx, s.p.ny, [&](auto z) -> hipError_t {
+      using Z = decltype(z);
+      if constexpr (!Z::fits) {
+        return hipErrorInvalidValue;
+      } else {
+        const int np = split_nproj<Z>(s.p);
+        SMX_LAUNCH((k_zsplit<Z>), dim3((unsigned)(np + split_z_blocks(s.p))), dim3(Z::NT), 0, st, s, op, np);
+        return hipGetLastError();
+      }
+    });
   });
 }
 template <typename T>
 hipError_t split_z_grp(const SplitArgs<T>* g, int nbox, const PParams<T>& p, int op, hipStream_t st) {
   if (nbox < 1 || nbox > 65535) return hipErrorInvalidValue;
   return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
-    constexpr int L = decltype(l)::value, RA = decltype(r)::value;
-    using Z = ZS<T, L, RA>;
-    if constexpr (!Z::fits) {
-      return hipErrorInvalidValue;
-    } else {
-      const int np = split_nproj<Z>(p);
-      SMX_LAUNCH((k_zsplit_grp<Z>), dim3((unsigned)(np + split_z_blocks(p)), (unsigned)nbox), dim3(Z::NT), 0, st,
-                 g, op, np);
-      return hipGetLastError();
-    }
+    return split_z_tile<T, decltype(l)::value, decltype(r)::value>(p.nx, p.ny, [&](auto z) -> hipError_t {
+      using Z = decltype(z);
+      if constexpr (!Z::fits) {
+        return hipErrorInvalidValue;
+      } else {
+        const int np = split_nproj<Z>(p);
+        SMX_LAUNCH((k_zsplit_grp<Z>), dim3((unsigned)(np + split_z_blocks(p)), (unsigned)nbox), dim3(Z::NT), 0, st,
+                   g, op, np);
+        return hipGetLastError();
+      }
+    });
   });
 }
 #endif
@@ -113,27 +129,31 @@ template <typename T>
 hipError_t split_adv_force(const SplitAdvArgs<T>& s, hipStream_t st) {
   const PParams<T>& p = s.ap.p;
   return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
-    using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
-    if constexpr (!zsa_fits<Z>()) {
-      return hipErrorInvalidValue;
-    } else {
-      const int np = split_nproj<Z>(p), nb = p.nx * (p.ny / Z::RA / Z::NY2);
-      SMX_LAUNCH((k_zsplit_force<Z>), dim3((unsigned)(np + nb)), dim3(Z::NT), 0, st, s, np);
-      return hipGetLastError();
-    }
+    return split_z_tile<T, decltype(l)::value, decltype(r)::value>(p.nx, p.ny, [&](auto z) -> hipError_t {
+      using Z = decltype(z);
+      if constexpr (!zsa_fits<Z>()) {
+        return hipErrorInvalidValue;
+      } else {
+        const int np = split_nproj<Z>(p), nb = p.nx * (p.ny / Z::RA / Z::NY2);
+        SMX_LAUNCH((k_zsplit_force<Z>), dim3((unsigned)(np + nb)), dim3(Z::NT), 0, st, s, np);
+        return hipGetLastError();
+      }
+    });
   });
 }
 template <typename T>
 hipError_t split_adv_advnl(const SplitAdvArgs<T>& s, hipStream_t st) {
   const PParams<T>& p = s.ap.p;
   return split_z_dispatch(p.nz, split_ra(p.ny), [&](auto l, auto r) -> hipError_t {
-    using Z = ZS<T, decltype(l)::value, decltype(r)::value>;
-    if constexpr (!zsa_fits<Z>()) {
-      return hipErrorInvalidValue;
-    } else {
-      SMX_LAUNCH((k_zsplit_advnl<Z>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, s);
-      return hipGetLastError();
-    }
+    return split_z_tile<T, decltype(l)::value, decltype(r)::value>(p.nx, p.ny, [&](auto z) -> hipError_t {
+      using Z = decltype(z);
+      if constexpr (!zsa_fits<Z>()) {
+        return hipErrorInvalidValue;
+      } else {
+        SMX_LAUNCH((k_zsplit_advnl<Z>), dim3((unsigned)(p.nx * (p.ny / Z::RA / Z::NY2))), dim3(Z::NT), 0, st, s);
+        return hipGetLastError();
+      }
+    });
   });
 }
 #endif
@@ -180,7 +200,9 @@ bool split_real_fits(int ny, int nz) {
   const int ra = split_ra(ny);
   return ra != 0 && split_z_dispatch(nz, ra, [&](auto l, auto r) -> hipError_t {
            using Z = ZS<double, decltype(l)::value, decltype(r)::value>;
-           return Z::fits && (ny / ra) % Z::NY2 == 0 ? hipSuccess : hipErrorInvalidValue;
+           return Z::fits && (size_t)(Z::SLDS + Z::L) * sizeof(cplx<double>) <= 160 * 1024 && (ny / ra) % Z::NY2 == 0
+                      ? hipSuccess
+                      : hipErrorInvalidValue;
          }) == hipSuccess;
 }
 template <typename TI>

@@ -88,7 +88,8 @@ struct NZ {
   // that let a second block of 1024 threads on the CU (256^3: 40 -> 53 us).
   static constexpr int HP = NPR + NY2, FP = sizeof(T) == 8 ? NPR : HP;
   static constexpr int ITEMS = L / 2 * NY2 * P, IPT = (ITEMS + NT - 1) / NT;
-  static constexpr int LDS = L * HP, RED = (NT % 64 == 0) ? NT / 64 : NT;
+  static constexpr int SP = NPR + 1, LDS = L * HP, SLDS = LDS;  // (SP < HP)
+  static constexpr int RED = (NT % 64 == 0) ? NT / 64 : NT;
   static constexpr size_t BYTES = (size_t)(LDS + L) * sizeof(cplx<T>) + RED * 8;
   static constexpr bool fits = NT <= 1024 && BYTES <= 160 * 1024;
 };

@@ -85,8 +85,8 @@ __device__ __forceinline__ void split_line_sums(const double* acc, double* R, in
 template <typename Z, int TRIG>
 constexpr bool split_scan_fits() {
   return Z::fits && Z::NT % 64 == 0 && Z::NT % (Z::RA * Z::NY2) == 0 &&
-         2 * Z::LDS >= TRIG * Z::L + (Z::H + 1) * Z::NT &&
-         (size_t)(Z::LDS + Z::L) * sizeof(cplx<double>) + 2 * Z::NPR * sizeof(int) <= 160 * 1024;
+         2 * Z::SLDS >= TRIG * Z::L + (Z::H + 1) * Z::NT &&
+         (size_t)(Z::SLDS + Z::L) * sizeof(cplx<double>) + 2 * Z::NPR * sizeof(int) <= 160 * 1024;
 }
 
 // trig: k_surf_tables' table (periodic: 2 nz values, Neumann: 4 nz).  dz: ns parts of nxy, the sum in part 0
@@ -104,8 +104,8 @@ struct SplitScan {
 // real parts of X_0 and X_{nz/2} enter, as in psi itself.
 template <typename Z, typename TI>
 __global__ __launch_bounds__(Z::NT) void k_zsplit_scan(const cplx<TI>* a, PParams<double> p, SplitScan s) {
-  constexpr int L = Z::L, RA = Z::RA, NC = 2 * Z::NPR, G = Z::P * Z::NY2, SP = Z::NPR + 1;
-  __shared__ cplx<double> F[Z::LDS];
+  constexpr int L = Z::L, RA = Z::RA, NC = 2 * Z::NPR, G = Z::P * Z::NY2, SP = Z::SP;
+  __shared__ cplx<double> F[Z::SLDS];
   __shared__ cplx<double> TW[L];
   __shared__ int KE[NC];
   const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
@@ -169,8 +169,8 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_scan(const cplx<TI>* a, PParam
 template <typename Z, typename TI>
 __global__ __launch_bounds__(Z::NT) void k_nsplit_scan(const cplx<TI>* a, PParams<double> p,
                                                        const cplx<double>* __restrict__ qtz, SplitScan s) {
-  constexpr int L = Z::L, NC = 2 * Z::NPR, G = Z::P * Z::NY2, SP = Z::NPR + 1;
-  __shared__ cplx<double> F[Z::LDS];
+  constexpr int L = Z::L, NC = 2 * Z::NPR, G = Z::P * Z::NY2, SP = Z::SP;
+  __shared__ cplx<double> F[Z::SLDS];
   __shared__ cplx<double> TW[L];
   __shared__ int KE[NC];
   const int tid = threadIdx.x, q = tid % Z::NPR, tc = tid / Z::NPR;
