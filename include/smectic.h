@@ -278,7 +278,8 @@ int smx_batch_adjoint_nodes(smx_batch *b, int64_t *nodes);
  * in place a handle steps in two launches instead of four (a periodic advected one in four instead of
  * fifteen) where its grid allows it (the y transforms divided between the z and the x kernels: grids with
  * ny <= 384 whose tiles fit a workgroup's LDS, but FP64 Neumann boxes of nx = 256 and nz < 512 only where two
- * blocks of one kernel fit a CU); any other schedule selects the kernels it names.  On such a
+ * blocks of one kernel fit a CU, and FP64 periodic boxes only with nx / 40 blocks or more in the x kernel); any
+ * other schedule selects the kernels it names.  On such a
  * grid smx_get_schedule reports the default while it is in place, and installing the default also leaves
  * the tiles of the adjoint's four passes to the library: those that smx_autotune picked for the grid in
  * this process, else the default ones.
