@@ -140,7 +140,11 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_advnl(SplitAdvArgs<typename Z:
 }
 #undef SMX_ZSA_SETUP
 
-#define SMX_XSA_SETUP(ARGS)                                                                        \
+// AGAIN: lane indices made again for each transform, as in k_zsplit_force, for the kernels that spill otherwise, or
+// whose registers keep a second block off the CU (it costs the others 3 to 5%).  Stokes in FP64 on lines of 384, and
+// of 256 with 16 y2: 384 x 192 x 256 595 -> 505 us, 384 x 96 x 64 126 -> 109, 256^3 298 -> 274; the update in FP32 on
+// lines of 384 (k_xsplit_adv): 384 x 192 x 256 216 -> 164 us, 384 x 96 x 512 251 -> 204.
+#define SMX_XSA_SETUP(ARGS, AGAIN)                                                                 \
   using T = typename X::T;                                                                        \
   constexpr int L = X::L, RB = X::RB, NC = X::NC, V = X::V;                                       \
   constexpr int E = X::E, NT = X::NT, NCP = X::NCP, NK = X::NK;                                   \
@@ -163,20 +167,24 @@ __global__ __launch_bounds__(Z::NT) void k_zsplit_advnl(SplitAdvArgs<typename Z:
   const uint32_t aofs = (uint32_t)split_pos(bx * NK + col / RB, col % RB, RB) * CB;                \
   const T kyv = p.ky[ky], kzv = p.kz[kz];                                                         \
   auto forward = [&](cplx<T>* w) {                                                                \
+    int ti = tid, ci = col, cc = tc;                                                              \
+    if constexpr (AGAIN) asm volatile("" : "+v"(ti), "+v"(ci), "+v"(cc));                         \
     _Pragma("unroll") for (int e = 0; e < E; ++e) w[e] = cmul(w[e], tw);                          \
-    RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(w, S, col, tc, twl,             \
-                                                                  [&]() { XRow<X, -1>::run(S, tid); }); \
+    RowFFT<true, T, L, E, AD, -1, typename PlanV<L, V>::Fwd>::run(w, S, ci, cc, twl,              \
+                                                                  [&]() { XRow<X, -1>::run(S, ti); }); \
   };                                                                                              \
   auto inverse = [&](cplx<T>* w) {                                                                \
-    RowFFT<true, T, L, E, AD, +1, typename PlanV<L, V>::Inv>::run(w, S, col, tc, twl,             \
-                                                                  [&]() { XRow<X, +1>::run(S, tid); }); \
+    int ti = tid, ci = col, cc = tc;                                                              \
+    if constexpr (AGAIN) asm volatile("" : "+v"(ti), "+v"(ci), "+v"(cc));                         \
+    RowFFT<true, T, L, E, AD, +1, typename PlanV<L, V>::Inv>::run(w, S, ci, cc, twl,              \
+                                                                  [&]() { XRow<X, +1>::run(S, ti); }); \
     _Pragma("unroll") for (int e = 0; e < E; ++e) w[e] = cmul(w[e], conjg(tw));                   \
   };
 
 // Stokes projection in full k-space (pf3d.cpp:433-447), U(k = 0) = 0.
 template <typename X>
 __global__ __launch_bounds__(X::NT) void k_xsplit_stokes(SplitAdvArgs<typename X::T> s) {
-  SMX_XSA_SETUP(s)
+  SMX_XSA_SETUP(s, (sizeof(typename X::T) == 8 && (X::L > 256 || (X::L == 256 && X::RB == 16))))
   cplx<T>* arr[3] = {s.as + plane, s.s1 + plane, s.s2 + plane};
   cplx<T> v[3][E];
 #pragma unroll
@@ -218,10 +226,11 @@ __global__ __launch_bounds__(X::NT) void k_xsplit_stokes(SplitAdvArgs<typename X
   }
 }
 
-// CNAB2 update (as k_xsplit) with four inverse outputs.
-template <typename X>
+// CNAB2 update (as k_xsplit) with four inverse outputs.  AGAIN in FP32 on lines of 384 with more blocks than CUs
+// (132 blocks, 384 x 64 x 64: a step 92.4 us without, 95.1).
+template <typename X, bool AGAIN>
 __global__ __launch_bounds__(X::NT) void k_xsplit_adv(SplitAdvArgs<typename X::T> s) {
-  SMX_XSA_SETUP(s)
+  SMX_XSA_SETUP(s, AGAIN)
   const uint32_t cofs = (uint32_t)(bx * NC + col) * CB;
   cplx<T>* rb = s.r + plane;
   cplx<T> v[E], ps[E];

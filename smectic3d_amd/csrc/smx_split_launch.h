@@ -188,7 +188,14 @@ hipError_t split_adv_update(const SplitAdvArgs<T>& s, hipStream_t st) {
     if constexpr (!xsa_fits<X>()) {
       return hipErrorInvalidValue;
     } else {
-      SMX_LAUNCH((k_xsplit_adv<X>), dim3((unsigned)(p.ny / X::NC * p.nzh)), dim3(X::NT), 0, st, s);
+      const unsigned nb = (unsigned)(p.ny / X::NC * p.nzh);
+      if constexpr (sizeof(T) == 4 && X::L >= 384) {
+        if (nb > 256) {
+          SMX_LAUNCH((k_xsplit_adv<X, true>), dim3(nb), dim3(X::NT), 0, st, s);
+          return hipGetLastError();
+        }
+      }
+      SMX_LAUNCH((k_xsplit_adv<X, false>), dim3(nb), dim3(X::NT), 0, st, s);
       return hipGetLastError();
     }
   });

@@ -54,6 +54,15 @@ def test_padding_of_a_tiles_rows(shape, kw, prec):
     run(shape, prec, **kw)
 
 
+@pytest.mark.parametrize("shape,prec", [((256, 256, 16), A.SMX_FP64), ((384, 32, 16), A.SMX_FP64),
+                                        ((384, 96, 24), A.SMX_FP64), ((384, 64, 16), A.SMX_FP32_MIXED),
+                                        ((384, 64, 128), A.SMX_FP32_MIXED)])
+def test_advected_x_kernels_of_long_lines(shape, prec):
+    """FP64 Stokes on lines of 256 with 16 y2 and of 384; the FP32 update on lines of 384 with 36 and 260 blocks."""
+    print(shape, prec, flush=True)
+    run(shape, prec, dt=2e-3, advect=1)
+
+
 def test_a_group_takes_the_tile_of_its_boxes():
     shape = (48, 192, 384)
     cfgs = [cfg_reference(*shape, eps=0.5 + 0.1 * i, beta=0.3, dt=0.05, nl_model=A.SMX_NL_CUBIC,
