@@ -7,7 +7,7 @@
 // S0, U0 and N take As's array, as in the fifteen launches.  27 moves of a stage array instead of 48: the
 // eleven y passes go, and d_y psi is formed in the x kernel, which has k_y at hand, so it is a fifth
 // carried array.
-// 256^3 FP32: 148 + 170 + 198 + 122 us against 680 in fifteen launches; FP64 1230 against 1410; 96 x 64 x
+// 256^3 FP32: 148 + 170 + 198 + 122 us against 680 in fifteen launches; FP64 1210 against 1410; 96 x 64 x
 // 128 FP64, where the launches and their gaps are the larger part, 97 against 138 us a step.  Moves alone
 // would take 262 us of the 638: the z kernels are bound by their transforms (seven inverse and one forward
 // in k_zsplit_advnl, each with two or three trips through LDS between barriers, and two blocks a CU to
